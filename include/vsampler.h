@@ -132,6 +132,11 @@ size_t vsamp_workspace_bytes(int32_t batch, int32_t vocab, int64_t hist_total);
  * need no clearing: each launch tags them. No counterpart in the engine. */
 size_t vsamp_split_workspace_bytes(int32_t batch, int32_t vocab, int64_t hist_total);
 
+/* Workspace bytes of a vsamp_probs call that writes its rows over the whole chip (the rows' states
+ * after the penalty part); a call with less (vsamp_workspace_bytes()) writes each row from one
+ * workgroup, with the same results. No counterpart in the engine. */
+size_t vsamp_probs_workspace_bytes(int32_t batch, int32_t vocab, int64_t hist_total);
+
 /* Sample one token per row: penalties, temperature, top-k, softmax, min-p, top-p, then the
  * inverse-CDF draw with u over the kept tokens taken in descending probability (equal
  * probabilities: ascending id). Replaces `sample(logits, params, seed, position)`

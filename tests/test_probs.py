@@ -1,0 +1,65 @@
+"""The probabilities' two launches (the rows' states, then the rows written over the whole chip) against
+the one-launch form, which a C caller with the smaller workspace gets: the same bits."""
+
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+import torch
+
+from vinfer_amd import _lib
+from vinfer_amd.registry import BackendContext
+from vinfer_amd.sampler import SAMPLER
+from vinfer_amd.sampling import PackedParams
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda", 0)
+
+
+def one_launch(s, logits, params, hist_ids, hist_offsets):
+    a, keep = s._args(logits, params, hist_ids, hist_offsets)  # (a workspace of vsamp_workspace_bytes())
+    B, V = logits.shape
+    need = int(s._lib.vsamp_workspace_bytes(B, V, a.hist_total))
+    ws = torch.zeros(need + 512, dtype=torch.uint8, device=DEV)
+    a.workspace, a.workspace_bytes = (ws.data_ptr() + 255) & ~255, need
+    out = torch.full((B, V), -1.0, device=DEV)
+    _lib.check(s._lib.vsamp_probs(ctypes.byref(a), out.data_ptr(), V, s._stream(DEV)))
+    torch.cuda.synchronize()
+    return out
+
+
+# (2048 ids a workgroup of the second launch: one short of a tile, one tile, one past it, a large and an odd
+# vocabulary; `offset` moves the rows off 16-byte alignment)
+@pytest.mark.parametrize("pen", [False, True], ids=["plain", "penalties"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=str)
+@pytest.mark.parametrize("V,offset", [(1, 0), (2047, 0), (2048, 0), (2049, 1), (50257, 0), (151936, 0), (151936, 3)])
+def test_two_launches_equal_one(V, offset, dtype, pen):
+    s = SAMPLER.resolve("hip", BackendContext(DEV, dtype))
+    g = torch.Generator(device=DEV).manual_seed(V + offset)
+    B = 9
+    x = torch.randn(B * V + offset, generator=g, device=DEV) * 3.0
+    logits = x.to(dtype)[offset:].view(B, V)
+    logits[1] = 0.25  # every token tied: the cutoff group splits
+    logits[2, 0] = float("inf")
+    logits[3, V // 2] = float("nan")
+    logits[4] = float("-inf")
+    f = lambda v: torch.tensor(v, dtype=torch.float32, device=DEV)  # noqa: E731
+    params = PackedParams(
+        temperature=f([0.8, 0.7, 0.9, 1.0, 1.0, 0.0, 1.2, 0.5, 1.0]),
+        top_k=torch.tensor([0, 0, 0, 0, 0, 0, 50, 700, 0], dtype=torch.int32, device=DEV),
+        top_p=f([0.95, 0.6, 0.9, 0.9, 0.9, 1.0, 0.9, 0.99, 1.0]), min_p=f([0, 0, 0, 0, 0, 0, 0, 0, 0.02]),
+        repetition_penalty=f([1.1 if pen else 1.0] * B), presence_penalty=f([0.5 if pen else 0.0] * B),
+        frequency_penalty=f([0.2 if pen else 0.0] * B))
+    ids = off = None
+    if pen:  # (one empty history, one past what the histogram path counts)
+        lengths = torch.tensor([100, 40, 7, 9, 11, 500, 0, 9000, 3000])
+        off = torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)]).to(torch.int32).to(DEV)
+        ids = torch.randint(0, V, (int(lengths.sum()),), generator=g, device=DEV).to(torch.int32)
+    print(f"probs V={V} offset={offset} {dtype} pen={pen}", flush=True)
+    got = s.probs(logits, params, ids, off)
+    torch.cuda.synchronize()
+    want = one_launch(s, logits, params, ids, off)
+    rows = [(r, int((got[r] != want[r]).sum()), got[r][got[r] != want[r]][:3].tolist(), want[r][got[r] != want[r]][:3].tolist())
+            for r in range(B) if not torch.equal(got[r], want[r])]
+    assert not rows, rows

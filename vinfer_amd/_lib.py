@@ -28,6 +28,7 @@ EXPORTS = (
     "vsamp_query",
     "vsamp_workspace_bytes",
     "vsamp_split_workspace_bytes",
+    "vsamp_probs_workspace_bytes",
     "vsamp_sample",
     "vsamp_sample_noalloc",
     "vsamp_probs",
@@ -150,6 +151,8 @@ def load() -> ctypes.CDLL:
         lib.vsamp_workspace_bytes.restype = ctypes.c_size_t
         lib.vsamp_split_workspace_bytes.argtypes = [ctypes.c_int32, ctypes.c_int32, ctypes.c_int64]
         lib.vsamp_split_workspace_bytes.restype = ctypes.c_size_t
+        lib.vsamp_probs_workspace_bytes.argtypes = [ctypes.c_int32, ctypes.c_int32, ctypes.c_int64]
+        lib.vsamp_probs_workspace_bytes.restype = ctypes.c_size_t
         lib.vsamp_sample.argtypes = [ctypes.POINTER(VsampArgs), ctypes.c_void_p]
         lib.vsamp_sample.restype = ctypes.c_int
         lib.vsamp_sample_noalloc.argtypes = [ctypes.POINTER(VsampArgs), ctypes.c_void_p]

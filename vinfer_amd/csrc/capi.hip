@@ -17,6 +17,7 @@
 #include "verify.cuh"
 #include "logprobs.cuh"
 #include "lmhead.cuh"
+#include "probs.cuh"
 
 namespace {
 
@@ -265,7 +266,7 @@ int run_sample(const vsamp_args* a, float* probs, int64_t probs_stride, hipStrea
                vs::RowState* state = nullptr, int param_div = 1, const float* tile_max = nullptr,
                uint32_t* tile_arrive = nullptr, int tile_G = 1) {
   const bool pen = wants_penalties(a);
-  if (state && pen) return fail(VSAMP_E_ARG, "row states are written without penalties only");
+  if (state && pen && !probs) return fail(VSAMP_E_ARG, "row states are written without penalties only");
   if ((a->flags & VSAMP_HIST_APPEND) && (state || probs))
     return fail(VSAMP_E_ARG, "VSAMP_HIST_APPEND goes with a call that draws from penalised rows");
   vs::SampleArgs s;
@@ -328,7 +329,9 @@ int run_sample(const vsamp_args* a, float* probs, int64_t probs_stride, hipStrea
     return e == hipSuccess ? VSAMP_OK : hip_fail(e, "launch k_sample (split rows)");
   }
   // One launch per step: the penalty phase runs at the start of the same kernel.
-  if (state)  // (the verify's launches, which apply no penalties)
+  if (state && pen)  // (probabilities)
+    hipLaunchKernelGGL((vs::k_sample<Tin, true, true>), dim3(a->batch), dim3(vs::kThreads), 0, st, s);
+  else if (state)
     hipLaunchKernelGGL((vs::k_sample<Tin, false, true>), dim3(a->batch), dim3(vs::kThreads), 0, st, s);
   else if (pen)
     hipLaunchKernelGGL((vs::k_sample<Tin, true>), dim3(a->batch), dim3(vs::kThreads), 0, st, s);
@@ -353,6 +356,37 @@ int run_tile_pass(const vsamp_args* a, float* tile_max, uint32_t* arrive, hipStr
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e, "launch k_tile_max");
   return run_sample<Tin>(a, nullptr, 0, st, nullptr, 1, tile_max);
+}
+
+// The probabilities' two launches keep the rows' states after the penalty part of the workspace.
+size_t probs_states(int64_t B, int64_t V, int64_t H) { return align_up(layout(B, V, H).total); }
+size_t probs_total(int64_t B, int64_t V, int64_t H) {
+  return probs_states(B, V, H) + sizeof(vs::RowState) * static_cast<size_t>(B);
+}
+
+// Probabilities: with a workspace that holds the row states, the states' launch and a launch that
+// writes the rows over the whole chip (32 bf16 rows of 151936: 104.8 -> 32.3 us); otherwise one
+// launch, each row written by its own workgroup.
+template <class Tin>
+int run_probs(const vsamp_args* a, float* out, int64_t out_stride, hipStream_t st) {
+  if (!a->workspace || (reinterpret_cast<uintptr_t>(a->workspace) & 255u) ||
+      a->workspace_bytes < probs_total(a->batch, a->vocab, a->hist_total) || a->batch > 65535)
+    return run_sample<Tin>(a, out, out_stride, st);
+  char* w = static_cast<char*>(a->workspace);
+  vs::RowState* states = reinterpret_cast<vs::RowState*>(w + probs_states(a->batch, a->vocab, a->hist_total));
+  if (int rc = run_sample<Tin>(a, out, out_stride, st, states)) return rc;
+  const Tin* logits = static_cast<const Tin*>(a->logits);
+  const vs::Workspace ws = workspace_of(a, layout(a->batch, a->vocab, a->hist_total));
+  const int hstep = (a->flags & VSAMP_HIST_RANGES) ? 2 : 1;
+  const dim3 grid((a->vocab + vs::kPwTile - 1) / vs::kPwTile, a->batch), block(vs::kPwThreads);
+  if (wants_penalties(a))
+    hipLaunchKernelGGL((vs::k_probs_write<Tin, true>), grid, block, 0, st, logits, a->row_stride, a->vocab, states, out,
+                       out_stride, ws, a->hist_offsets, hstep);
+  else
+    hipLaunchKernelGGL((vs::k_probs_write<Tin, false>), grid, block, 0, st, logits, a->row_stride, a->vocab, states,
+                       out, out_stride, ws, a->hist_offsets, hstep);
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? VSAMP_OK : hip_fail(e, "launch k_probs_write");
 }
 
 struct VerifyLayout {
@@ -404,6 +438,11 @@ size_t vsamp_workspace_bytes(int32_t batch, int32_t vocab, int64_t hist_total) {
 size_t vsamp_split_workspace_bytes(int32_t batch, int32_t vocab, int64_t hist_total) {
   if (batch < 0 || vocab < 1 || hist_total < 0) return 0;
   return split_total(batch, vocab, hist_total);
+}
+
+size_t vsamp_probs_workspace_bytes(int32_t batch, int32_t vocab, int64_t hist_total) {
+  if (batch < 0 || vocab < 1 || hist_total < 0) return 0;
+  return probs_total(batch, vocab, hist_total);
 }
 
 int vsamp_sample(const vsamp_args* a, void* stream) {
@@ -467,8 +506,8 @@ int vsamp_probs(const vsamp_args* a, float* out, int64_t out_stride, void* strea
   if (out_stride < a->vocab) return fail(VSAMP_E_ARG, "out_stride must be >= vocab");
   if (int rc = check_current_device()) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  return a->dtype == VSAMP_BF16 ? run_sample<uint16_t>(a, out, out_stride, st)
-                                : run_sample<float>(a, out, out_stride, st);
+  return a->dtype == VSAMP_BF16 ? run_probs<uint16_t>(a, out, out_stride, st)
+                                : run_probs<float>(a, out, out_stride, st);
 }
 
 int vsamp_penalized_logits(const vsamp_args* a, float* out, int32_t* counts, int64_t out_stride,

@@ -56,7 +56,7 @@ struct SampleArgs {
   int32_t* out_ids;
   int32_t* hist_out;  // when non-null, each row's drawn id also goes to hist_out[its history's end]
   float* out_dprob;
-  float* out_probs;  // probs mode when non-null
+  float* out_probs;  // probs mode when non-null (with STATE: the states alone, nothing drawn)
   int64_t probs_stride;
   RowState* out_state;  // optional: each row's RowState
   int param_div;        // (row-state launches) rows per parameter entry: row r reads entry r / param_div
@@ -959,6 +959,7 @@ __device__ __forceinline__ void finish(const SampleArgs& a, const Row<Tin>& row,
     st.S = k.S;
     a.out_state[r] = st;
   }
+  if (STATE && a.out_probs) return;  // (the states alone: k_probs_write writes the rows)
   if (a.out_probs) {
     float* o = a.out_probs + static_cast<int64_t>(r) * a.probs_stride;
     if (k.point >= 0) {
@@ -2641,6 +2642,16 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, Row<uint16_t> row,
   auto need_bitmap = [&]() {  // (uniform)
     if (ne > 0 && !row.bm) build_bitmap(row, hist + kBitmapOffset);
   };
+  auto finish_row = [&](int draw) {
+    if constexpr (PEN && STATE) {  // (probabilities: the row's penalised values for k_probs_write)
+      for (int e = tid; e < ne; e += kThreads) {
+        a.ws.exc_id[p.h0 + e] = f.eid[e];
+        a.ws.exc_val[p.h0 + e] = f.eval[e];
+      }
+      if (tid == 0) a.ws.n_exc[r] = static_cast<uint32_t>(ne);
+    }
+    finish<STATE>(a, row, p, mz, k, draw, &srch.vslot, r);
+  };
   if (status == kPlanPoint) {
     const float xmax = val_of(mkey);
     // point rows: the first NaN, the first max (greedy), the first +inf z, or index 0 (all -inf)
@@ -2652,7 +2663,7 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, Row<uint16_t> row,
       if constexpr (SPLIT) {
         need_bitmap();
         pt = split_find(a, row, f, ne, xmax, 0ull, srch, hist + kMatchOffset, recs);
-      } else if (!a.out_probs && cells_per(row) * kThreads <= 4 * kMatchWords) {  // (uniform)
+      } else if ((STATE || !a.out_probs) && cells_per(row) * kThreads <= 4 * kMatchWords) {  // (uniform)
         // the first id holding the max, by the member search from the kept low bytes (as the
         // draw's member) instead of a pass over the row
         uint8_t* cells = reinterpret_cast<uint8_t*>(hist + kMatchOffset);
@@ -2671,7 +2682,7 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, Row<uint16_t> row,
       need_bitmap();
       if (!degenerate(row, p, mkey, 0, mz, srch, k)) k.point = 0;
     }
-    finish<STATE>(a, row, p, mz, k, 0, &srch.vslot, r);
+    finish_row(0);
     return true;
   }
   // ---- 5. [all] per-chunk masses of elements >= x0 ---------------------------------------
@@ -2849,7 +2860,7 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, Row<uint16_t> row,
   const u64 j = f.plan.j;
   // One pass zeroes the member search's cells and, when a pass over the row will need it, the
   // position bitmap of the penalised ids.
-  const bool cells_fit = !SPLIT && !a.out_probs && cells_per(row) * kThreads <= 4 * kMatchWords;
+  const bool cells_fit = !SPLIT && (STATE || !a.out_probs) && cells_per(row) * kThreads <= 4 * kMatchWords;
   const bool bitmap_now = ne > 0 && !cells_fit;  // (uniform)
   {
     uint32_t* bmw = hist + kBitmapOffset;
@@ -2907,7 +2918,7 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, Row<uint16_t> row,
       draw = find_first(row, [&](float x, int) -> u64 { return x == vd; }, j, srch);
     }
   }
-  finish<STATE>(a, row, p, mz, k, draw, &srch.vslot, r);
+  finish_row(draw);
   return true;
 }
 
@@ -3343,7 +3354,8 @@ __device__ __forceinline__ SampleArgs globalized(SampleArgs a) {
   return a;
 }
 
-// STATE: also write each row's RowState (the speculative verify's launches; never with PEN).
+// STATE: also write each row's RowState (the speculative verify's launches, without PEN, and the
+// probabilities' first launch, marked by a.out_probs, which draws nothing).
 // SPLIT: a bf16 split-row launch (grid B * G).
 // TILES: rows (bf16 or fp32) with their tile maxima (a.tile_max): the rows tile_row can decide
 // are decided from a few tiles, the others take the row passes below.
