@@ -455,8 +455,8 @@ __global__ __launch_bounds__(kTsThreads) void k_tile_stats(const uint16_t* logit
   float x[8];
   int nv = 0;  // this lane's logits inside the row
   if (t < nT) {
-    if ((reinterpret_cast<uintptr_t>(row + i0) & 15u) == 0 && i0 + 8 <= V) {
-      const uint4 q = ld_global_u4(reinterpret_cast<const uint4*>(row + i0));
+    if (i0 + 8 <= V) {
+      const uint4 q = ld_row16(row + i0);
       const uint32_t w[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
       for (int i = 0; i < 4; ++i) {

@@ -46,7 +46,7 @@ struct LogprobArgs {
 // in fp64: the terms the per-element sum adds) and the n-th largest key; each thread keeps the
 // three largest elements it read (packed key and position, by a min/max insertion), and those
 // >= the n-th key are the candidate list, complete unless some thread's third is >= that key.
-// Returns false, with no output written, for a row it does not serve -- unaligned, a NaN, an
+// Returns false, with no output written, for a row it does not serve -- a NaN, an
 // infinite or no finite max, a key count past 2^16, an n-th largest value <= 0 (where -0.0 and
 // +0.0 would need their ties by id), an incomplete list -- and the caller runs its two passes.
 // On success `kn32` is the n-th largest key as an ordered 32-bit key.
@@ -56,15 +56,14 @@ __device__ __forceinline__ bool lp_one_pass(const LogprobArgs& a, const Row<uint
   const int tid = threadIdx.x;
   const int V = row.V;
   const int n = a.n_top;
-  if (!row.vec) return false;  // (uniform)
   const int nfull = V / kBlk;
   // (a row without a whole block loads a constant block instead, unused)
-  const uint4* blocks = reinterpret_cast<const uint4*>(nfull > 0 ? row.p : g_unused_block);
+  const uint16_t* blocks = nfull > 0 ? row.p : g_unused_block;
   // blocks tid + 1024 m; kAhead of them in flight while the previous kAhead are counted
   constexpr int kAhead = 4;
   uint4 d[kAhead];
 #pragma unroll
-  for (int k = 0; k < kAhead; ++k) d[k] = ld_global_u4(blocks + min(k * kThreads + tid, max(nfull - 1, 0)));
+  for (int k = 0; k < kAhead; ++k) d[k] = ld_block(blocks, min(k * kThreads + tid, max(nfull - 1, 0)));
   for (int i = tid; i < 32768 / 4; i += kThreads) reinterpret_cast<uint4*>(hist)[i] = make_uint4(0, 0, 0, 0);
   if (tid < 8) sh[tid] = 0;
   __syncthreads();
@@ -92,7 +91,7 @@ __device__ __forceinline__ bool lp_one_pass(const LogprobArgs& a, const Row<uint
     for (int k = 0; k < kAhead; ++k) {
       const int m = it * kAhead + k;
       const uint4 q = d[k];
-      d[k] = ld_global_u4(blocks + min((m + kAhead) * kThreads + tid, max(nfull - 1, 0)));
+      d[k] = ld_block(blocks, min((m + kAhead) * kThreads + tid, max(nfull - 1, 0)));
       if (m * kThreads + tid < nfull) {
         const uint32_t w[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
@@ -207,7 +206,6 @@ __global__ __launch_bounds__(kThreads) void k_logprobs(LogprobArgs a) {
   row.V = a.V;
   row.nblk = (a.V + kBlk - 1) / kBlk;
   row.nstripes = (row.nblk + kThreads - 1) / kThreads;
-  row.vec = (reinterpret_cast<uintptr_t>(row.p) & 15u) == 0;
   row.bm = nullptr;
   row.eid = nullptr;
   row.eval = nullptr;

@@ -13,12 +13,13 @@
 namespace vs {
 
 constexpr int kPwThreads = 256;
+typedef float f32x4_any_t __attribute__((ext_vector_type(4), aligned(4)));  // (16-byte stores at any fp32 address)
 constexpr int kPwTile = kPwThreads * kBlk;  // ids per workgroup
 
 // Grid (ceil(V / kPwTile), B): workgroup (t, r) writes ids kPwTile t .. of row r, a token's
 // probability as the one-launch form computes it (the same expressions, so the same bits). Thread
-// i takes eight consecutive ids where the row and the output are 16-byte aligned, else ids
-// i + 256 k (coalesced element by element, eight loads in flight). With PEN the tile's penalised
+// i takes eight consecutive ids (16-byte loads and stores); in the row's last, partial tile, ids
+// i + 256 k (element by element, eight loads in flight). With PEN the tile's penalised
 // ids are written again from the row's list, after the workgroup's own bulk stores.
 template <class Tin, bool PEN>
 __global__ __launch_bounds__(kPwThreads) void k_probs_write(const Tin* logits, int64_t stride, int V, const RowState* state,
@@ -42,10 +43,9 @@ __global__ __launch_bounds__(kPwThreads) void k_probs_write(const Tin* logits, i
     if (st.point >= 0) return id == st.point ? 1.0f : 0.0f;
     return kept.keep(x, id) ? static_cast<float>(ptilde(x, st.T, st.mz) * inv) : 0.0f;
   };
-  const bool vec = ((reinterpret_cast<uintptr_t>(row) | reinterpret_cast<uintptr_t>(o)) & 15u) == 0;  // (uniform)
   const int b0 = i0 + kBlk * tid;
   float v[kBlk];
-  const bool whole = vec && i0 + kPwTile <= V;  // (uniform)
+  const bool whole = i0 + kPwTile <= V;  // (uniform)
   if (whole) {
     WholeBlock<Tin> q;
     q.load(row, b0 / kBlk);
@@ -59,7 +59,7 @@ __global__ __launch_bounds__(kPwThreads) void k_probs_write(const Tin* logits, i
   }
   __syncthreads();  // (the exp table)
   if (whole) {
-    float4 a, b;
+    f32x4_any_t a, b;
     a.x = prob(v[0], b0);
     a.y = prob(v[1], b0 + 1);
     a.z = prob(v[2], b0 + 2);
@@ -68,8 +68,8 @@ __global__ __launch_bounds__(kPwThreads) void k_probs_write(const Tin* logits, i
     b.y = prob(v[5], b0 + 5);
     b.z = prob(v[6], b0 + 6);
     b.w = prob(v[7], b0 + 7);
-    *reinterpret_cast<float4*>(o + b0) = a;
-    *reinterpret_cast<float4*>(o + b0 + 4) = b;
+    *reinterpret_cast<f32x4_any_t*>(o + b0) = a;
+    *reinterpret_cast<f32x4_any_t*>(o + b0 + 4) = b;
   } else {
 #pragma unroll
     for (int e = 0; e < kBlk; ++e) {

@@ -184,8 +184,7 @@ struct __align__(16) FastSmem {
 __device__ __align__(16) uint16_t g_unused_block[kBlk];  // (read, never written)
 
 __device__ __forceinline__ uint4 ld_block(const uint16_t* base, int b) {
-  const u32x4_t v = ld_global(reinterpret_cast<const u32x4_t*>(base + b * kBlk));
-  return make_uint4(v.x, v.y, v.z, v.w);
+  return ld_row16(base + b * kBlk);
 }
 
 // defaults of the parameter words (RowParams order): T 1, top-p 1, min-p 0, u 0, top-k 0,
@@ -275,7 +274,7 @@ static_assert(offsetof(FastSmem, eid) == offsetof(FastSmem, eval) + sizeof(float
               "ccnt .. eid must be contiguous");
 static_assert(kExcCap <= 2 * kThreads, "two ranks per thread");
 
-// Block b of a 16-byte-aligned row whose block is wholly inside it, as loaded (one
+// Block b of a row, wholly inside it, as loaded (one
 // unconditional vector load, so that several in flight are waited for together: Row::load's
 // per-lane range test puts each load behind a branch), and its values.
 template <class Tin>
@@ -283,7 +282,7 @@ struct WholeBlock;
 template <>
 struct WholeBlock<uint16_t> {
   uint4 d;
-  __device__ __forceinline__ void load(const uint16_t* p, int b) { d = *reinterpret_cast<const uint4*>(p + b * kBlk); }
+  __device__ __forceinline__ void load(const uint16_t* p, int b) { d = ld_row16(p + b * kBlk); }
   __device__ __forceinline__ void values(float v[kBlk]) const {
     const uint32_t w[4] = {d.x, d.y, d.z, d.w};
 #pragma unroll
@@ -295,14 +294,15 @@ struct WholeBlock<uint16_t> {
 };
 template <>
 struct WholeBlock<float> {
-  float4 d0, d1;
+  uint4 d0, d1;
   __device__ __forceinline__ void load(const float* p, int b) {
-    d0 = *reinterpret_cast<const float4*>(p + b * kBlk);
-    d1 = *reinterpret_cast<const float4*>(p + b * kBlk + 4);
+    d0 = ld_row16(p + b * kBlk);
+    d1 = ld_row16(p + b * kBlk + 4);
   }
   __device__ __forceinline__ void values(float v[kBlk]) const {
-    v[0] = d0.x; v[1] = d0.y; v[2] = d0.z; v[3] = d0.w;
-    v[4] = d1.x; v[5] = d1.y; v[6] = d1.z; v[7] = d1.w;
+    const uint32_t w[kBlk] = {d0.x, d0.y, d0.z, d0.w, d1.x, d1.y, d1.z, d1.w};
+#pragma unroll
+    for (int i = 0; i < kBlk; ++i) v[i] = __uint_as_float(w[i]);
   }
 };
 
@@ -312,7 +312,6 @@ struct Row {
   int V;
   int nblk;
   int nstripes;
-  bool vec;
   const uint8_t* bm;   // per-block lane masks of exceptions, or null
   const int32_t* eid;  // exceptions of this row (in no particular order)
   const float* eval;
@@ -326,14 +325,10 @@ template <>
 __device__ __forceinline__ uint32_t Row<uint16_t>::load(int b, float v[kBlk]) const {
   const int base = b * kBlk;
   uint32_t valid;
-  if (vec && base + kBlk <= V) {
-    const uint4 d = *reinterpret_cast<const uint4*>(p + base);
-    const uint32_t w[4] = {d.x, d.y, d.z, d.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v[2 * i] = __uint_as_float(w[i] << 16);
-      v[2 * i + 1] = __uint_as_float(w[i] & 0xFFFF0000u);
-    }
+  if (base + kBlk <= V) {
+    WholeBlock<uint16_t> q;
+    q.load(p, b);
+    q.values(v);
     valid = 0xFFu;
   } else {
     valid = 0;
@@ -352,11 +347,10 @@ template <>
 __device__ __forceinline__ uint32_t Row<float>::load(int b, float v[kBlk]) const {
   const int base = b * kBlk;
   uint32_t valid;
-  if (vec && base + kBlk <= V) {
-    const float4 d0 = *reinterpret_cast<const float4*>(p + base);
-    const float4 d1 = *reinterpret_cast<const float4*>(p + base + 4);
-    v[0] = d0.x; v[1] = d0.y; v[2] = d0.z; v[3] = d0.w;
-    v[4] = d1.x; v[5] = d1.y; v[6] = d1.z; v[7] = d1.w;
+  if (base + kBlk <= V) {
+    WholeBlock<float> q;
+    q.load(p, b);
+    q.values(v);
     valid = 0xFFu;
   } else {
     valid = 0;
@@ -386,12 +380,12 @@ __device__ __forceinline__ float max_of8(const float (&x)[kBlk]) {
 
 // Every block of the row once, as fb(v, out, b) in the calling thread: v its eight values and
 // `out` the lanes that hold no bulk value (penalised, or past the row's end). The groups of kDepth
-// stripes wholly inside an aligned row have their loads (and lane masks) issued together, ahead
+// stripes wholly inside the row have their loads (and lane masks) issued together, ahead
 // of the work on them. Exceptions are the caller's.
 template <class Tin, class FB>
 __device__ __forceinline__ void for_each_block_ahead(const Row<Tin>& row, FB fb, int j0 = 0) {
   constexpr int kDepth = 2;  // (measured on logprobs and fp32 rows: 2 beats 4 and 8)
-  const int whole = row.vec ? row.V / kBlk / kThreads : 0;  // (uniform) such stripes
+  const int whole = row.V / kBlk / kThreads;  // (uniform) such stripes
   int j = j0;  // (the stripes below j0, a multiple of kDepth, were visited by the caller)
   if constexpr (kRollDepth > 0) {
     // a rolling window: as stripe j's values are taken out of slot k, the slot's next load
@@ -1340,7 +1334,7 @@ __device__ __forceinline__ void generic_row(const SampleArgs& a, Row<Tin> row, c
   // largest; its own histogram then gives the K-th largest's bin)
   constexpr int kStreamDepth = 2;
   Cand* stage = reinterpret_cast<Cand*>(reinterpret_cast<uint32_t*>(&g) + kMatchOffset + 2 * kCandCap);
-  const bool stream = sizeof(Tin) == 4 && topk && p.K <= kStreamK && row.vec &&
+  const bool stream = sizeof(Tin) == 4 && topk && p.K <= kStreamK &&
                       row.V / kBlk / kThreads >= kStreamDepth;  // (uniform)
   uint32_t tau_bin = 0;
   auto first_pass = [&](auto greedy_c) {
@@ -2015,7 +2009,7 @@ __device__ __forceinline__ int select_member(const Row<uint16_t>& row, FastSmem&
   if (bf) {
     const uint32_t pat = t16 * 0x10001u, patb = t16b * 0x10001u;
     auto match8 = [&](uint4 w) -> uint32_t { return match1(w, pat) | (t16b != t16 ? match1(w, patb) : 0u); };
-    const int nfull = row.vec ? V / kBlk : 0;
+    const int nfull = V / kBlk;
     const uint32_t ka = ok16(t16), kb = ok16(t16b);
     const bool cand = mxk >= (ka < kb ? ka : kb);
     // this thread's blocks tid + m * kThreads, m < nm
@@ -2069,7 +2063,7 @@ __device__ __forceinline__ int select_member(const Row<uint16_t>& row, FastSmem&
       }
     }
     lds_barrier();  // (the byte stores above land before the word atomics below)
-    // the rest: a ragged tail, or every element of an unaligned row
+    // the rest: a ragged tail
     if (cand) {
       for (int i = nfull * kBlk + tid; i < V; i += kThreads) {
         const uint32_t raw = base[i];
@@ -2264,7 +2258,7 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, Row<uint16_t> row,
   // ---- 1. histogram of every key, then the penalised tokens' original keys taken out ----------
   // (u16 halves of a word wrap and borrow exactly: only the final counts must stay below 2^16)
   const uint16_t* base = row.p;
-  const int nfull = row.vec ? V / kBlk : 0;  // blocks read as one 16-byte load
+  const int nfull = V / kBlk;  // blocks read as one 16-byte load
   // A rolling prefetch: slot k of d holds block tid + (D * round + k) * kThreads and is reloaded
   // for the next round as soon as it is consumed (into the same registers: loading before the
   // old value is consumed would need a copy at the loop's end, which waits for every load).
@@ -2457,7 +2451,7 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, Row<uint16_t> row,
   // original values just requested, as a wait at a loop's head would)
   if (rounds > 4) round(4);
   for (int it = 5; it < rounds; ++it) round(it);
-  // the rest: a ragged tail, or every element of an unaligned row
+  // the rest: a ragged tail
   uint32_t mxk = mx2.x > mx2.y ? mx2.x : mx2.y;
   for (int i = nfull * kBlk + tid; !SPLIT && i < V; i += kThreads) {  // (split rows: the last slice's)
     const uint32_t ko = ok16(base[i]);
@@ -3026,8 +3020,7 @@ __device__ __forceinline__ uint32_t lane_tile_key(const uint4 (&v)[kTileLoads<Ti
   }
   return mk;
 }
-// The same for a lane whose eight logits are not one aligned run inside the row: element by
-// element (fewer past the end).
+// The same for a lane whose eight logits reach past the row's end: element by element.
 template <class Tin>
 __device__ __forceinline__ uint32_t lane_tile_key_each(const Tin* row, int i0, int V) {
   uint32_t mk = 0;
@@ -3045,10 +3038,10 @@ __global__ __launch_bounds__(kTileMaxThreads) void k_tile_max(const Tin* logits,
   const int i0 = t * kStatTile + 8 * l16;  // this lane's first logit
   uint32_t mk = 0;                         // (below every key)
   if (t < nT) {
-    if ((reinterpret_cast<uintptr_t>(row + i0) & 15u) == 0 && i0 + 8 <= V) {
+    if (i0 + 8 <= V) {
       uint4 q[kTileLoads<Tin>];
 #pragma unroll
-      for (int j = 0; j < kTileLoads<Tin>; ++j) q[j] = ld_global_u4(reinterpret_cast<const uint4*>(row + i0) + j);
+      for (int j = 0; j < kTileLoads<Tin>; ++j) q[j] = ld_row16(reinterpret_cast<const char*>(row + i0) + 16 * j);
       mk = lane_tile_key<Tin>(q);
     } else {
       mk = lane_tile_key_each<Tin>(row, i0, V);
@@ -3081,7 +3074,7 @@ __device__ __forceinline__ bool tile_share(const SampleArgs& a, int r, int g, in
   const Tin* row = as_global(static_cast<const Tin*>(a.logits)) + static_cast<int64_t>(r) * a.stride;
   const int V = a.V;
   float* out = const_cast<float*>(a.tile_max) + static_cast<int64_t>(r) * nT;
-  // pass q: tile g * per + threadIdx.x / 16 + 64 q (the same in a 16-lane row); whole aligned
+  // pass q: tile g * per + threadIdx.x / 16 + 64 q (the same in a 16-lane row); whole
   // 16-byte chunks are loaded first (every lane issues its loads: one that has none reads a
   // constant aligned block, unused), the rest element by element
   uint4 v[kTileSharePasses][kTileLoads<Tin>];
@@ -3090,11 +3083,11 @@ __device__ __forceinline__ bool tile_share(const SampleArgs& a, int r, int g, in
   for (int q = 0; q < kTileSharePasses; ++q) {
     const int t = g * per + static_cast<int>(threadIdx.x >> 4) + kWave * q;
     const int i0 = t * kStatTile + 8 * l16;
-    whole[q] = t < end && (reinterpret_cast<uintptr_t>(row + i0) & 15u) == 0 && i0 + 8 <= V;
+    whole[q] = t < end && i0 + 8 <= V;
 #pragma unroll
     for (int j = 0; j < kTileLoads<Tin>; ++j)
-      v[q][j] = ld_global_u4(whole[q] ? reinterpret_cast<const uint4*>(row + i0) + j
-                                      : reinterpret_cast<const uint4*>(g_unused_block));
+      v[q][j] = ld_row16(whole[q] ? reinterpret_cast<const char*>(row + i0) + 16 * j
+                                  : reinterpret_cast<const char*>(g_unused_block));
   }
   auto umax = [](uint32_t x, uint32_t y) { return x > y ? x : y; };
 #pragma unroll
@@ -3382,7 +3375,6 @@ __global__ __launch_bounds__(kThreads) void k_sample(SampleArgs a_) {
   row.V = a.V;
   row.nblk = (a.V + kBlk - 1) / kBlk;
   row.nstripes = (row.nblk + kThreads - 1) / kThreads;
-  row.vec = (reinterpret_cast<uintptr_t>(row.p) & 15u) == 0;
   row.nexc = 0;
   row.bm = nullptr;  // built in LDS by the path that masks penalised positions
   row.eid = f.eid;   // the fast path keeps the penalised ids and values in LDS

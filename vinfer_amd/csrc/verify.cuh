@@ -198,8 +198,6 @@ __device__ __forceinline__ void residual_item(const VerifyArgs& a, int b, int sl
   rt.V = rd.V = a.V;
   rt.nblk = rd.nblk = (a.V + kBlk - 1) / kBlk;
   rt.nstripes = rd.nstripes = (rt.nblk + kThreads - 1) / kThreads;
-  rt.vec = (reinterpret_cast<uintptr_t>(rt.p) & 15u) == 0;
-  rd.vec = (reinterpret_cast<uintptr_t>(rd.p) & 15u) == 0;
   rt.bm = rd.bm = nullptr;
   rt.eid = rd.eid = nullptr;
   rt.eval = rd.eval = nullptr;
@@ -306,7 +304,7 @@ __device__ __forceinline__ void residual_item(const VerifyArgs& a, int b, int sl
       if (lane_id() == 0) cell[wv][j - j_begin] = s;
     };
     for (int j0 = j_begin; j0 < j_end; j0 += 4) {
-      if (rt.vec && rd.vec && j0 + 4 <= j_end && (j0 + 4) * kThreads * kBlk <= a.V) {
+      if (j0 + 4 <= j_end && (j0 + 4) * kThreads * kBlk <= a.V) {
         // (uniform) four stripes wholly inside both rows
         WholeBlock<Tin> qt[4], qd[4];
 #pragma unroll
@@ -385,7 +383,7 @@ __device__ __forceinline__ void residual_item(const VerifyArgs& a, int b, int sl
     // 3. per-thread sums inside stripe js; the thread whose block holds the target
     u64 w[kBlk] = {};
     const int blk = js * kThreads + tid;
-    if (rt.vec && rd.vec && (js + 1) * kThreads * kBlk <= a.V) {  // (uniform) a whole stripe
+    if ((js + 1) * kThreads * kBlk <= a.V) {  // (uniform) a whole stripe
       WholeBlock<Tin> qt, qd;
       qt.load(rt.p, blk);
       qd.load(rd.p, blk);
