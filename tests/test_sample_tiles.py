@@ -401,3 +401,33 @@ def test_gpu_prepared_launches_equal_the_calls():
         for ids, dp in ((a, ap), (b, bp), (c, cp)):
             assert torch.equal(ids, want), rep
             assert torch.equal(dp.view(torch.int32), wantp.view(torch.int32)), rep
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=str)
+def test_gpu_tile_pass_top_k_up_to_the_list(dtype):
+    # top-k around the tiles read at a time (64) and up to the sorted list's 256, on rows whose tile
+    # maxima fall into one coarse key bin ([8, 16) and [-16, -8)), spread out, all tied, or hold -inf
+    s = hip()
+    V = 151936
+    ks = [1, 2, 20, 63, 64, 65, 127, 128, 129, 200, 255, 256]
+    g = torch.Generator(device=DEV).manual_seed(5)
+    for label in ("normal", "one bin", "negative", "tied", "masked"):
+        x = torch.randn(len(ks), V, generator=g, device=DEV) * 3.0
+        if label == "one bin":
+            x = 10.0 + x * 1e-3
+        elif label == "negative":
+            x = -10.0 + x * 1e-3
+        elif label == "tied":
+            x = (x * 0.25).round()
+        elif label == "masked":
+            x[:, 3000:] = -math.inf
+        logits = x.to(dtype)
+        pp = pack_params([SamplingParams(temperature=0.7, top_k=k, top_p=0.8) for k in ks]).to(DEV)
+        u = torch.rand(len(ks), generator=g, device=DEV)
+        draft = logits.float().argmax(dim=1).to(torch.int32)
+        print(f"tile pass top-k {label} {dtype}", flush=True)
+        a, ap = s.sample_tile_pass(logits, pp, u, None, None, draft)
+        b, bp = row_passes(s, logits, pp, u, None, None, draft)
+        torch.cuda.synchronize()
+        assert torch.equal(a, b) and torch.equal(ap, bp), label

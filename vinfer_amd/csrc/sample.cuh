@@ -2925,17 +2925,18 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, Row<uint16_t> row,
 //     row max (as values: -0 equals +0), and only that tile is read;
 //   * rows sampled at T > 0 with top-k (K <= kSortCap) or min-p: every kept token has
 //     x >= xlo, where for top-k xlo is the least x with fl(x / T) >= fl(theta / T), theta the
-//     K-th largest tile max (the K largest tile maxima are K logits, so theta is at most the
-//     K-th largest logit, whose z every kept token reaches), and for min-p the least x whose
-//     p~ = exp(fl(x / T) - max z) reaches min_p; a kept token then lies in a tile whose max is
-//     >= xlo. The elements >= xlo of those tiles (at most kTileRowTiles tiles, at most
-//     kSortCap elements) are sorted as the generic path sorts its short lists, the exact top-k
+//     K-th largest tile max to 20 bits of its key, exactly it for bf16 (the K largest tile maxima
+//     are K logits, so theta is at most the K-th largest logit, whose z every kept token
+//     reaches), and for min-p the least x whose p~ = exp(fl(x / T) - max z) reaches min_p; a
+//     kept token then lies in a tile whose max is >= xlo. The elements >= xlo of those tiles (at
+//     most kTileRowTiles tiles, at most kSortCap elements) are sorted as the generic path sorts its short lists, the exact top-k
 //     and min-p thresholds taken from them, and sorted_tail finishes the row: the same
 //     cutoff, masses and draw as a pass over the row.
 // Rows with penalties, NaN maxima, infinite scaled logits, top-p alone, or more candidates than
 // that take the row passes (the caller's path) as if no tile maxima were given.
 constexpr int kStatTile = 128;      // logits per statistics tile (k_lm_head's column tile)
-constexpr int kTileRowTiles = 64;   // candidate tiles a row decided from its tiles reads at most
+constexpr int kTileRowTiles = 256;  // candidate tiles a row decided from its tiles reads at most
+constexpr int kTileRead = 64;       // of them read at a time
 
 // The key of the k-th largest (1-based, with multiplicity) of the 16-bit keys keys[0 .. nk) of
 // every thread (nk <= 4; k <= the number of keys): two rounds over the high and the low byte,
@@ -3186,14 +3187,19 @@ __device__ __forceinline__ bool tile_row(const SampleArgs& a, const Row<Tin>& ro
     finish<false>(a, row, p, 0.0f, k, 0, &g.srch.vslot, r);
     return true;
   }
-  // Top-k rows count their tiles' maxima by the top 12 bits of their keys (4096 bins in LDS; of
-  // a bf16 value, the top 12 bits of its 16-bit key): the lowest value of the bin holding the
-  // K-th largest is at most the K-th largest tile max, so at most the K-th largest logit. The row
-  // max rides the same barrier (one LDS atomicMax per wave).
+  // Top-k rows count their tiles' maxima by the top 12 bits of their keys (4096 bins in LDS), then
+  // those of the K-th largest's bin by the next 8 (of a bf16 value's 16-bit key all the rest): the
+  // lowest value of that bin is at most the K-th largest tile max, so at most the K-th largest
+  // logit. (The 12 bits alone leave a bin as wide as [8, 9) or [10, 11): at K = 20 of 151936 N(0, 3)
+  // logits half of the rows had more tiles at its floor than could be read and were handed on: 36.5 us
+  // a per-token call against 22.7 now, whichever the row; 36.5 against 25.5 at K = 100.) The row max rides the first barrier (one LDS
+  // atomicMax per wave).
   uint32_t* h12 = reinterpret_cast<uint32_t*>(&g) + kBitmapOffset;
+  uint32_t* h8 = h12 + 4096;  // 256 bins
   uint32_t* smax = &g.rdx.ncand;
   uint32_t* tcount = reinterpret_cast<uint32_t*>(g.rdx.bq);  // (the candidate tiles' count)
   if (topk) reinterpret_cast<uint4*>(h12)[tid] = make_uint4(0, 0, 0, 0);
+  if (topk && tid < 256) h8[tid] = 0;
   if (tid == 0) *smax = 0;
   lds_barrier();
 #pragma unroll
@@ -3214,9 +3220,8 @@ __device__ __forceinline__ bool tile_row(const SampleArgs& a, const Row<Tin>& ro
   if (!(mz > -INFINITY && mz < INFINITY)) return false;  // point rows: the row passes
   // xlo: no kept token lies below it (wave 0 decides; the others wait at the barrier)
   const uint32_t lo_key = key_of(-INFINITY);
-  if (tid < kWave) {
-    float xlo = -INFINITY, xm = -INFINITY;
-    if (topk) {
+  if (topk) {  // (uniform)
+    if (tid < kWave) {
       // the bin of the K-th largest: lane l sums bins 4095 - 64 l - 63 .. 4095 - 64 l (lane 0
       // the top ones), then lane i of the crossing lane's 64 bins takes bin 4095 - 64 L - i
       const uint32_t K = static_cast<uint32_t>(p.K);
@@ -3233,17 +3238,36 @@ __device__ __forceinline__ bool tile_row(const SampleArgs& a, const Row<Tin>& ro
       const uint32_t c = h12[4095 - 64 * L - l];
       const uint32_t incl2 = above + wave_incl_scan<uint32_t>(c);
       const int i = __ffsll(static_cast<long long>(__ballot(incl2 >= K))) - 1;
-      const uint32_t bin = static_cast<uint32_t>(4095 - 64 * L - i);
-      // the least value of the bin (not below -inf): of bf16 rows, the bf16 value of its least
-      // 16-bit key; of fp32 rows, the value of its least 32-bit key
-      float theta;
-      if constexpr (sizeof(Tin) == 2) {
-        const uint32_t k16 = (bin << 4) > 0x007Fu ? (bin << 4) : 0x007Fu;
-        theta = val16(k16);
-      } else {
-        const uint32_t k32 = (bin << 20) > key_of(-INFINITY) ? (bin << 20) : key_of(-INFINITY);
-        theta = val_of(k32);
+      if (l == i) {
+        sh[2] = static_cast<uint32_t>(4095 - 64 * L - i);
+        sh[3] = incl2 - c;  // tile maxima above the bin
       }
+    }
+    lds_barrier();
+    const uint32_t bin = sh[2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (tid + i * kThreads < nT && (kt[i] >> 20) == bin) atomicAdd(&h8[(kt[i] >> 12) & 255u], 1u);
+    lds_barrier();
+  }
+  if (tid < kWave) {
+    float xlo = -INFINITY, xm = -INFINITY;
+    if (topk) {
+      // lane l: the bin's sub-bins 255 - 4 l .. 252 - 4 l, descending
+      const uint32_t K = static_cast<uint32_t>(p.K);
+      const uint4 v = reinterpret_cast<const uint4*>(h8)[63 - tid];
+      const uint32_t c4[4] = {v.w, v.z, v.y, v.x};
+      const uint32_t s4 = v.x + v.y + v.z + v.w;
+      uint32_t run = sh[3] + wave_incl_scan<uint32_t>(s4) - s4;
+      uint32_t sub = 0xFFFFFFFFu;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (run < K && K <= run + c4[i]) sub = static_cast<uint32_t>(255 - 4 * tid - i);
+        run += c4[i];
+      }
+      const int L = __ffsll(static_cast<long long>(__ballot(sub != 0xFFFFFFFFu))) - 1;  // (one lane holds it)
+      const uint32_t k32 = (sh[2] << 20) | (__builtin_amdgcn_readlane(sub, L) << 12);
+      const float theta = val_of(k32 > lo_key ? k32 : lo_key);
       const float zt = theta / T;
       xlo = val_of(wave_bisect(lo_key, key_of(theta), key_of(zt * T), [&](float x) { return x / T >= zt; }));
     }
@@ -3281,27 +3305,30 @@ __device__ __forceinline__ bool tile_row(const SampleArgs& a, const Row<Tin>& ro
   lds_barrier();
   const uint32_t ntile = *tcount;
   if (ntile > static_cast<uint32_t>(kTileRowTiles)) return false;  // (uniform)
-  // their elements >= xlo, into the candidate list (every element's load first)
+  // their elements >= xlo, into the candidate list, kTileRead tiles at a time (every element's load
+  // first)
   Cand* c = reinterpret_cast<Cand*>(reinterpret_cast<uint32_t*>(&g) + kMatchOffset);
-  constexpr int kPer = kTileRowTiles * kStatTile / kThreads;
-  float xs[kPer];
-  int ids[kPer];
+  constexpr int kPer = kTileRead * kStatTile / kThreads;
+  for (int e0 = tid; e0 - tid < static_cast<int>(ntile) * kStatTile; e0 += kTileRead * kStatTile) {  // (uniform)
+    float xs[kPer];
+    int ids[kPer];
 #pragma unroll
-  for (int q = 0; q < kPer; ++q) {
-    const int e = tid + q * kThreads;
-    ids[q] = e < static_cast<int>(ntile) * kStatTile ? ctile[e / kStatTile] * kStatTile + e % kStatTile : V;
-    xs[q] = load_one<Tin>(row.p, ids[q] < V ? ids[q] : 0);
-  }
+    for (int q = 0; q < kPer; ++q) {
+      const int e = e0 + q * kThreads;
+      ids[q] = e < static_cast<int>(ntile) * kStatTile ? ctile[e / kStatTile] * kStatTile + e % kStatTile : V;
+      xs[q] = load_one<Tin>(row.p, ids[q] < V ? ids[q] : 0);
+    }
 #pragma unroll
-  for (int q = 0; q < kPer; ++q) {
-    const bool in = ids[q] < V && xs[q] >= xlo;
-    const u64 bal = __ballot(in);  // (one counter update per wave)
-    if (bal) {
-      const int leader = __ffsll(static_cast<long long>(bal)) - 1;
-      uint32_t pos = 0;
-      if (lane_id() == leader) pos = atomicAdd(&sh[2], static_cast<uint32_t>(__popcll(bal)));
-      pos = __builtin_amdgcn_readlane(pos, leader) + static_cast<uint32_t>(__popcll(bal & ((1ull << lane_id()) - 1ull)));
-      if (in && pos < static_cast<uint32_t>(kSortCap)) c[pos] = Cand{xs[q], ids[q]};
+    for (int q = 0; q < kPer; ++q) {
+      const bool in = ids[q] < V && xs[q] >= xlo;
+      const u64 bal = __ballot(in);  // (one counter update per wave)
+      if (bal) {
+        const int leader = __ffsll(static_cast<long long>(bal)) - 1;
+        uint32_t pos = 0;
+        if (lane_id() == leader) pos = atomicAdd(&sh[2], static_cast<uint32_t>(__popcll(bal)));
+        pos = __builtin_amdgcn_readlane(pos, leader) + static_cast<uint32_t>(__popcll(bal & ((1ull << lane_id()) - 1ull)));
+        if (in && pos < static_cast<uint32_t>(kSortCap)) c[pos] = Cand{xs[q], ids[q]};
+      }
     }
   }
   lds_barrier();
