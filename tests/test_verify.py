@@ -300,3 +300,31 @@ def test_gpu_verify_residual_over_signed_zeros(dtype):
         assert int(counts[b]) == 1 and tokens[b, 0].item() == w.tokens[0], (b, tokens[b].tolist(), w.tokens)
         on_neg += w.tokens[0] in neg[b]
     assert 10 <= on_neg <= 38  # about half the draws land on a -0.0 token
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=str)
+@pytest.mark.parametrize("B,K,V", [(1, 1, 7), (3, 2, 4099), (40, 3, 8195), (300, 1, 2048)])
+def test_gpu_rows_without_residual_mass_take_the_targets_draw(dtype, B, K, V):
+    # the draft's logits are the target's: a rejected draft (outside the vocabulary, at a position of its
+    # own for every sequence) leaves no residual, so the target's own draw at that position is emitted, and
+    # sequences without one get the bonus draw; both are those of a batched draw from the same row (300
+    # sequences: more rows than CUs)
+    dev = torch.device("cuda", 0)
+    s = SAMPLER.resolve("hip", BackendContext(dev, dtype))
+    g = torch.Generator(device=dev).manual_seed(B * K + V)
+    target = (torch.randn(B, K + 1, V, generator=g, device=dev) * 2).to(dtype)
+    params = pack_params([SamplingParams(temperature=(0.0, 0.7, 1.2)[b % 3], top_p=0.9) for b in range(B)]).to(dev)
+    first = torch.arange(B, device=dev) % (K + 1)  # the rejected position (K: none)
+    draws, u = [], torch.rand(B, generator=g, device=dev)
+    for j in range(K + 1):
+        draws.append(s.sample_batch(target[:, j].contiguous(), params, u)[0])
+    draws = torch.stack(draws, 1)
+    drafts = torch.where(torch.arange(K, device=dev)[None, :] == first[:, None], -1, draws[:, :K])
+    print(f"verify without residual mass B={B} K={K} V={V} {dtype}", flush=True)
+    tokens, counts = s.verify(target, target[:, :K].contiguous(), drafts, params, torch.zeros(B, K, device=dev),
+                              torch.rand(B, K, generator=g, device=dev), u)
+    torch.cuda.synchronize()
+    assert torch.equal(counts.long(), first + 1)
+    keep = torch.arange(K + 1, device=dev)[None, :] <= first[:, None]
+    assert torch.equal(tokens, torch.where(keep, draws, -1).to(torch.int32))

@@ -261,26 +261,10 @@ int launch_penalties(const vs::PenaltyArgs& p, int B, hipStream_t st) {
   return e == hipSuccess ? VSAMP_OK : hip_fail(e, "launch k_penalty_prep");
 }
 
-template <class Tin>
-int run_sample(const vsamp_args* a, float* probs, int64_t probs_stride, hipStream_t st,
-               vs::RowState* state = nullptr, int param_div = 1, const float* tile_max = nullptr,
-               uint32_t* tile_arrive = nullptr, int tile_G = 1) {
-  const bool pen = wants_penalties(a);
-  if (state && pen && !probs) return fail(VSAMP_E_ARG, "row states are written without penalties only");
-  if ((a->flags & VSAMP_HIST_APPEND) && (state || probs))
-    return fail(VSAMP_E_ARG, "VSAMP_HIST_APPEND goes with a call that draws from penalised rows");
+// The rows, parameters and outputs of a call; everything else off.
+vs::SampleArgs sample_args(const vsamp_args* a) {
   vs::SampleArgs s;
   std::memset(&s, 0, sizeof s);
-  if (pen) {
-    const Layout L = layout(a->batch, a->vocab, a->hist_total);
-    if (int rc = check_workspace(a, L)) return rc;
-    s.ws = workspace_of(a, L);
-    s.pen = penalty_args(a, s.ws);
-    s.has_exc = 1;
-    s.off = a->hist_offsets;
-    // (the drawn id goes behind each row's range: the caller's history buffer is writable)
-    if (a->flags & VSAMP_HIST_APPEND) s.hist_out = const_cast<int32_t*>(a->hist_ids);
-  }
   s.logits = a->logits;
   s.stride = a->row_stride;
   s.V = a->vocab;
@@ -292,11 +276,37 @@ int run_sample(const vsamp_args* a, float* probs, int64_t probs_stride, hipStrea
   s.draft = a->draft_ids;
   s.out_ids = a->out_ids;
   s.out_dprob = a->out_draft_prob;
+  s.nrows = a->batch;
+  s.param_div = 1;
+  return s;
+}
+
+// state: the rows' states are written too; with probs also set, they alone, and nothing is drawn.
+// skip_every (with state): of every skip_every + 1 rows the last is left out.
+template <class Tin>
+int run_sample(const vsamp_args* a, float* probs, int64_t probs_stride, hipStream_t st,
+               vs::RowState* state = nullptr, int param_div = 1, const float* tile_max = nullptr,
+               uint32_t* tile_arrive = nullptr, int tile_G = 1, int skip_every = 0) {
+  const bool pen = wants_penalties(a);
+  if (state && pen && !probs) return fail(VSAMP_E_ARG, "row states are written without penalties only");
+  if ((a->flags & VSAMP_HIST_APPEND) && (state || probs))
+    return fail(VSAMP_E_ARG, "VSAMP_HIST_APPEND goes with a call that draws from penalised rows");
+  vs::SampleArgs s = sample_args(a);
+  if (pen) {
+    const Layout L = layout(a->batch, a->vocab, a->hist_total);
+    if (int rc = check_workspace(a, L)) return rc;
+    s.ws = workspace_of(a, L);
+    s.pen = penalty_args(a, s.ws);
+    s.has_exc = 1;
+    s.off = a->hist_offsets;
+    // (the drawn id goes behind each row's range: the caller's history buffer is writable)
+    if (a->flags & VSAMP_HIST_APPEND) s.hist_out = const_cast<int32_t*>(a->hist_ids);
+  }
   s.out_probs = probs;
   s.probs_stride = probs_stride;
   s.out_state = state;
   s.param_div = param_div;
-  s.nrows = a->batch;
+  s.skip_every = skip_every;
   if (tile_max) {  // (bf16 rows with the LM head's tile maxima: no split rows, no states)
     s.tile_max = tile_max;
     s.nT = (a->vocab + VSAMP_LM_TILE - 1) / VSAMP_LM_TILE;
@@ -332,7 +342,8 @@ int run_sample(const vsamp_args* a, float* probs, int64_t probs_stride, hipStrea
   if (state && pen)  // (probabilities)
     hipLaunchKernelGGL((vs::k_sample<Tin, true, true>), dim3(a->batch), dim3(vs::kThreads), 0, st, s);
   else if (state)
-    hipLaunchKernelGGL((vs::k_sample<Tin, false, true>), dim3(a->batch), dim3(vs::kThreads), 0, st, s);
+    hipLaunchKernelGGL((vs::k_sample<Tin, false, true>),
+                       dim3(skip_every ? a->batch / (skip_every + 1) * skip_every : a->batch), dim3(vs::kThreads), 0, st, s);
   else if (pen)
     hipLaunchKernelGGL((vs::k_sample<Tin, true>), dim3(a->batch), dim3(vs::kThreads), 0, st, s);
   else
@@ -390,17 +401,13 @@ int run_probs(const vsamp_args* a, float* out, int64_t out_stride, hipStream_t s
 }
 
 struct VerifyLayout {
-  size_t tids, dids, ts, ds, jr, done, sums, rej, nrej, total;
+  size_t ts, ds, jr, done, sums, rej, acc, nrej, total;
 };
 
 VerifyLayout verify_layout(int64_t B, int64_t K) {
   VerifyLayout L;
   const size_t nt = static_cast<size_t>(B * (K + 1)), nd = static_cast<size_t>(B * K);
   size_t o = 0;
-  L.tids = o;
-  o = align_up(o + 4 * nt);
-  L.dids = o;
-  o = align_up(o + 4 * nd);
   L.ts = o;
   o = align_up(o + sizeof(vs::RowState) * nt);
   L.ds = o;
@@ -412,6 +419,8 @@ VerifyLayout verify_layout(int64_t B, int64_t K) {
   L.sums = o;
   o = align_up(o + 8 * static_cast<size_t>(B) * vs::kMaxStripes);
   L.rej = o;
+  o = align_up(o + 4 * static_cast<size_t>(B));
+  L.acc = o;
   o = align_up(o + 4 * static_cast<size_t>(B));
   L.nrej = o;
   o = align_up(o + 4);
@@ -568,32 +577,35 @@ int vsamp_verify(const vsamp_verify_args* v, void* stream) {
     return fail(VSAMP_E_ARG, "verify does not apply penalties (histories must be NULL)");
   if (B > 0 && (!v->draft_tokens || !v->u_accept || !v->u_residual || !v->out_tokens || !v->out_count))
     return fail(VSAMP_E_ARG, "draft_tokens, u_accept, u_residual, out_tokens and out_count must be set");
-  if (!d.uniforms) d.uniforms = v->u_residual;  // (the draft rows' own draws are not used)
+  if (!d.uniforms) d.uniforms = v->u_residual;  // (nothing is drawn from the draft rows)
   const VerifyLayout L = verify_layout(B, K);
   if (v->workspace_bytes < L.total || (L.total && !v->workspace))
     return fail(VSAMP_E_WORKSPACE, "workspace of %zu bytes given, %zu needed", v->workspace_bytes, L.total);
   if (reinterpret_cast<uintptr_t>(v->workspace) & 255u)
     return fail(VSAMP_E_WORKSPACE, "workspace must be 256-byte aligned");
   char* w = static_cast<char*>(v->workspace);
-  int32_t* tids = reinterpret_cast<int32_t*>(w + L.tids);
-  int32_t* dids = reinterpret_cast<int32_t*>(w + L.dids);
   vs::RowState* ts = reinterpret_cast<vs::RowState*>(w + L.ts);
   vs::RowState* ds = reinterpret_cast<vs::RowState*>(w + L.ds);
-  t.out_ids = tids;
-  d.out_ids = dids;  // (the draft rows' own draws are not used)
+  t.out_ids = d.out_ids = v->out_tokens;  // (the draft rows write none)
   if (int rc = validate(&t, true)) return rc;
   if (int rc = validate(&d, true)) return rc;
   if (B == 0) return VSAMP_OK;
   if (int rc = check_current_device()) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool bf = t.dtype == VSAMP_BF16;
-  // parameters and uniforms: one entry per sequence for all of its rows
-  if (int rc = bf ? run_sample<uint16_t>(&t, nullptr, 0, st, ts, K + 1) : run_sample<float>(&t, nullptr, 0, st, ts, K + 1))
-    return rc;
+  // parameters and uniforms: one entry per sequence for all of its rows. The states of the target
+  // rows at the drafted positions and of the draft rows; nothing is drawn yet (`probs` only marks
+  // that).
+  auto states_of = [&](const vsamp_args& q, vs::RowState* out, int rows, int skip) {
+    float* mark = reinterpret_cast<float*>(out);
+    return bf ? run_sample<uint16_t>(&q, mark, 0, st, out, rows, nullptr, nullptr, 1, skip)
+              : run_sample<float>(&q, mark, 0, st, out, rows, nullptr, nullptr, 1, skip);
+  };
+  if (int rc = states_of(t, ts, K + 1, K)) return rc;
   if (v->draft_states) {
     if (reinterpret_cast<uintptr_t>(v->draft_states) & 7u) return fail(VSAMP_E_ARG, "draft_states must be 8-byte aligned");
     ds = static_cast<vs::RowState*>(const_cast<void*>(v->draft_states));
-  } else if (int rc = bf ? run_sample<uint16_t>(&d, nullptr, 0, st, ds, K) : run_sample<float>(&d, nullptr, 0, st, ds, K)) {
+  } else if (int rc = states_of(d, ds, K, 0)) {
     return rc;
   }
   vs::VerifyArgs a;
@@ -606,7 +618,6 @@ int vsamp_verify(const vsamp_verify_args* v, void* stream) {
   a.drafts = v->draft_tokens;
   a.u_acc = v->u_accept;
   a.u_res = v->u_residual;
-  a.tids = tids;
   a.ts = ts;
   a.ds = ds;
   a.out_tokens = v->out_tokens;
@@ -615,19 +626,24 @@ int vsamp_verify(const vsamp_verify_args* v, void* stream) {
   a.done = reinterpret_cast<uint32_t*>(w + L.done);
   a.sums = reinterpret_cast<vs::u64*>(w + L.sums);
   a.rej = reinterpret_cast<int32_t*>(w + L.rej);
+  a.acc = reinterpret_cast<int32_t*>(w + L.acc);
   a.nrej = reinterpret_cast<int32_t*>(w + L.nrej);
+  a.B = B;
   const int nstripes = ((t.vocab + vs::kBlk - 1) / vs::kBlk + vs::kThreads - 1) / vs::kThreads;
   a.max_slices = 1;
   while (2 * a.max_slices <= nstripes && 2 * a.max_slices <= kMaxResidualSlices) a.max_slices *= 2;
-  // at most one workgroup per CU: items beyond the rejected rows' exit without holding a CU
-  const int64_t items = B * a.max_slices;
-  const dim3 gr(static_cast<unsigned>(items < current_cus() ? items : current_cus()));
+  // (the bonus rows and the rejected rows' slices: never more than this)
+  const int64_t items = static_cast<int64_t>(B) * a.max_slices;
+  const int64_t on_cus = items < current_cus() ? items : current_cus();
+  const dim3 gr(static_cast<unsigned>(on_cus > B ? on_cus : B));
+  vs::SampleArgs s = sample_args(&t);
+  s.param_div = K + 1;
   if (bf) {
-    hipLaunchKernelGGL(vs::k_verify_accept<uint16_t>, dim3(1), dim3(vs::kThreads), 0, st, a, B);
-    hipLaunchKernelGGL(vs::k_verify_residual<uint16_t>, gr, dim3(vs::kThreads), 0, st, a);
+    hipLaunchKernelGGL(vs::k_verify_accept<uint16_t>, dim3(1), dim3(vs::kThreads), 0, st, a);
+    hipLaunchKernelGGL(vs::k_verify_finish<uint16_t>, gr, dim3(vs::kThreads), 0, st, a, s);
   } else {
-    hipLaunchKernelGGL(vs::k_verify_accept<float>, dim3(1), dim3(vs::kThreads), 0, st, a, B);
-    hipLaunchKernelGGL(vs::k_verify_residual<float>, gr, dim3(vs::kThreads), 0, st, a);
+    hipLaunchKernelGGL(vs::k_verify_accept<float>, dim3(1), dim3(vs::kThreads), 0, st, a);
+    hipLaunchKernelGGL(vs::k_verify_finish<float>, gr, dim3(vs::kThreads), 0, st, a, s);
   }
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? VSAMP_OK : hip_fail(e, "launch k_verify");

@@ -59,7 +59,8 @@ struct SampleArgs {
   float* out_probs;  // probs mode when non-null (with STATE: the states alone, nothing drawn)
   int64_t probs_stride;
   RowState* out_state;  // optional: each row's RowState
-  int param_div;        // (row-state launches) rows per parameter entry: row r reads entry r / param_div
+  int param_div;        // (verify's launches) rows per parameter entry: row r reads entry r / param_div
+  int skip_every;       // (row-state launches) of every skip_every + 1 rows the last is left out (0: none)
   Workspace ws;
   int has_exc;  // the workspace holds this batch's exceptions
   const int32_t* off;
@@ -79,9 +80,13 @@ struct SampleArgs {
   int tile_G;
 };
 
-// The row of this workgroup.
+// The row of this workgroup in a split-row launch, and in a row-state launch.
 __device__ __forceinline__ int row_index(const SampleArgs& a) {
   return a.G > 1 ? static_cast<int>(blockIdx.x % static_cast<unsigned>(a.nrows)) : static_cast<int>(blockIdx.x);
+}
+__device__ __forceinline__ int state_row_index(const SampleArgs& a) {
+  const int b = static_cast<int>(blockIdx.x);
+  return a.skip_every > 0 ? b + b / a.skip_every : b;
 }
 
 // Scratch of the id-order search.
@@ -197,9 +202,9 @@ __device__ const uint32_t kParamDefaults[16] = {0x3F800000u, 0x3F800000u, 0u, 0u
 // instead would index the argument struct, which then has to live in scratch memory.
 // Word w of row r's parameters, one load per lane: the lane picks its column's address (or the
 // default's) first, so nothing waits for the load until the word is used.
-template <bool PEN, bool STATE = false>
+template <bool PEN, bool DIV = false>
 __device__ __forceinline__ uint32_t param_word(const SampleArgs& a, int r0, int w) {
-  const int r = STATE ? r0 / a.param_div : r0;
+  const int r = DIV ? r0 / a.param_div : r0;
   const void* cols[kParamWords] = {a.temp, a.topp, a.minp, a.u, a.topk, a.draft,
                                    PEN ? a.pen.rep : nullptr, PEN ? a.pen.pres : nullptr,
                                    PEN ? a.pen.freq : nullptr, PEN ? a.off : nullptr, PEN ? a.off : nullptr};
@@ -2646,7 +2651,7 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, Row<uint16_t> row,
     }
     finish<STATE>(a, row, p, mz, k, draw, &srch.vslot, r);
   };
-  if (status == kPlanPoint) {
+  if (__builtin_expect(status == kPlanPoint, 0)) {
     const float xmax = val_of(mkey);
     // point rows: the first NaN, the first max (greedy), the first +inf z, or index 0 (all -inf)
     if (f.plan.nnan) {
@@ -2907,7 +2912,7 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, Row<uint16_t> row,
       draw = cells_fit ? select_member(row, f, ne, vd, j, reinterpret_cast<uint8_t*>(hist + kMatchOffset), mxk, low,
                                        sl, og, e0, estep)
                        : -1;
-    if (draw < 0) {  // (uniform)
+    if (__builtin_expect(draw < 0, 0)) {  // (uniform)
       need_bitmap();
       draw = find_first(row, [&](float x, int) -> u64 { return x == vd; }, j, srch);
     }
@@ -3374,29 +3379,15 @@ __device__ __forceinline__ SampleArgs globalized(SampleArgs a) {
   return a;
 }
 
-// STATE: also write each row's RowState (the speculative verify's launches, without PEN, and the
-// probabilities' first launch, marked by a.out_probs, which draws nothing).
-// SPLIT: a bf16 split-row launch (grid B * G).
-// TILES: rows (bf16 or fp32) with their tile maxima (a.tile_max): the rows tile_row can decide
-// are decided from a few tiles, the others take the row passes below.
-template <class Tin, bool PEN, bool STATE = false, bool SPLIT = false, bool TILES = false>
-__global__ __launch_bounds__(kThreads) void k_sample(SampleArgs a_) {
-  const SampleArgs a = globalized(a_);
-  // 128 KB: the key histogram (or the generic path's penalty counts), then the id-search /
-  // radix scratch
-  __shared__ __align__(16) uint32_t big[kChunk];
-  __shared__ FastSmem f;
+// Row r by the calling workgroup, its parameter words loaded (pw). `big` is 128 KB: the key
+// histogram (or the generic path's penalty counts), then the id-search / radix scratch. The
+// template parameters are k_sample's.
+template <class Tin, bool PEN, bool STATE, bool SPLIT, bool TILES>
+__device__ __forceinline__ void sample_row(const SampleArgs& a, int r, uint32_t pw, bool fused, uint32_t* big,
+                                           FastSmem& f) {
   static_assert(sizeof(GenericSmem) <= sizeof(uint32_t) * kBitmapOffset, "scratch must fit below the bitmap");
   static_assert(kMatchOffset + kMatchWords <= kChunk, "count cells must fit");
-  const bool fused = TILES && a.tile_arrive != nullptr;  // (uniform)
-  const int r = SPLIT ? row_index(a) : fused ? static_cast<int>(blockIdx.x) / a.tile_G : static_cast<int>(blockIdx.x);
   const int tid = threadIdx.x;
-  exp_table_init();  // (published by the first barrier of either path)
-  // the row's parameters: thread w < kParamWords loads word w, the others word 0 (every thread
-  // loads: a load on one branch only would make later waits wait for every load in flight)
-  const uint32_t pw = param_word<PEN, STATE>(a, r, tid < kParamWords ? tid : 0);
-  __builtin_amdgcn_sched_barrier(0);  // (issued before the row's first loads)
-
   Row<Tin> row;
   row.p = static_cast<const Tin*>(a.logits) + static_cast<int64_t>(r) * a.stride;
   row.V = a.V;
@@ -3427,7 +3418,7 @@ __global__ __launch_bounds__(kThreads) void k_sample(SampleArgs a_) {
     }
   }
   if constexpr (sizeof(Tin) == 2) {
-    if (fast_row<PEN, STATE, SPLIT>(a, row, f.prm, big, f, g.srch, pw, r)) return;
+    if (__builtin_expect(fast_row<PEN, STATE, SPLIT>(a, row, f.prm, big, f, g.srch, pw, r), 1)) return;
     lds_barrier();  // (every thread is done with the fast path's LDS; f.prm is set)
   } else {
     if (tid < kParamWords) reinterpret_cast<uint32_t*>(&f.prm)[tid] = pw;
@@ -3446,6 +3437,30 @@ __global__ __launch_bounds__(kThreads) void k_sample(SampleArgs a_) {
     row.eval = a.ws.exc_val + p.h0;
   }
   generic_row<STATE>(a, row, p, g, f, r, have_bitmap);
+}
+
+// STATE: write each row's RowState (the speculative verify's launches, without PEN, and the
+// probabilities' first launch; with a.out_probs set nothing is drawn).
+// SPLIT: a bf16 split-row launch (grid B * G).
+// TILES: rows (bf16 or fp32) with their tile maxima (a.tile_max): the rows tile_row can decide
+// are decided from a few tiles, the others take the row passes.
+template <class Tin, bool PEN, bool STATE = false, bool SPLIT = false, bool TILES = false>
+__global__ __launch_bounds__(kThreads) void k_sample(SampleArgs a_) {
+  const SampleArgs a = globalized(a_);
+  __shared__ __align__(16) uint32_t big[kChunk];
+  __shared__ FastSmem f;
+  const bool fused = TILES && a.tile_arrive != nullptr;  // (uniform)
+  const int r = SPLIT ? row_index(a)
+                : fused ? static_cast<int>(blockIdx.x) / a.tile_G
+                : STATE ? state_row_index(a)
+                        : static_cast<int>(blockIdx.x);
+  const int tid = threadIdx.x;
+  exp_table_init();  // (published by the first barrier of either path)
+  // the row's parameters: thread w < kParamWords loads word w, the others word 0 (every thread
+  // loads: a load on one branch only would make later waits wait for every load in flight)
+  const uint32_t pw = param_word<PEN, STATE>(a, r, tid < kParamWords ? tid : 0);
+  __builtin_amdgcn_sched_barrier(0);  // (issued before the row's first loads)
+  sample_row<Tin, PEN, STATE, SPLIT, TILES>(a, r, pw, fused, big, f);
 }
 
 }  // namespace vs

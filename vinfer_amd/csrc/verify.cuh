@@ -15,10 +15,16 @@
 // whose inclusive prefix of w exceeds floor(m * R / 2^24), R the sum. A point-mass row (greedy,
 // degenerate) has mass 2^42 at its token and S = 2^42.
 //
-// The sampling kernel has already run over every target and draft row (its RowState output
-// gives each row's kept set, max and S), so this kernel reads logits only where it decides:
-// the drafted tokens' two values per position, and for a rejected position the target and
-// draft rows, once to sum the residual and once more inside the stripe that holds the token.
+// The sampling kernel has already run over the target rows at the drafted positions and the draft
+// rows (its RowState output gives each row's kept set, max and S), so these kernels read logits
+// only where they decide: the drafted tokens' two values per position, for a rejected position
+// the target and draft rows, once to sum the residual and once more inside the stripe that holds
+// the token, and for a sequence whose drafts were all accepted the bonus position's row, which is
+// sampled then. So the rows at the bonus position cost nothing where a draft is rejected, the
+// drafted positions' rows are not drawn from (but in the rare row without residual mass), and the
+// bonus rows and the residuals share one launch: 192 sequences of one draft, V = 262144, 137.4 us
+// a call when every target row was sampled first (384 rows, one and a half rounds on 256 CUs) and
+// the residuals took a launch of their own, 91 us now.
 // A bf16 row holds at most 65536 distinct values, and its kept ones sit in a short run of keys
 // below the row's max: the two terms of w are tabulated per key in LDS for the top kTab keys
 // of each row (a kept token below that run is computed directly), so the residual pass costs
@@ -41,8 +47,7 @@ struct VerifyArgs {
   const int32_t* drafts;  // [B * K] drafted tokens
   const float* u_acc;     // [B * K] acceptance uniforms
   const float* u_res;     // [B * K] residual-draw uniforms
-  const int32_t* tids;    // [B * (K + 1)] the target's draws
-  const RowState* ts;     // [B * (K + 1)]
+  const RowState* ts;     // [B * (K + 1)] (the drafted positions' entries)
   const RowState* ds;     // [B * K]
   int32_t* out_tokens;    // [B * (K + 1)]: the emitted tokens, then -1
   int32_t* out_count;     // [B]
@@ -50,7 +55,9 @@ struct VerifyArgs {
   uint32_t* done;         // [B] slices of the row's residual finished
   u64* sums;              // [B * kMaxStripes] per-stripe residual sums
   int32_t* rej;           // [B] the rejected sequences, ascending
-  int32_t* nrej;          // [1] how many
+  int32_t* acc;           // [B] the others, ascending
+  int32_t* nrej;          // [1] how many are rejected
+  int B;
   int max_slices;         // most workgroups per rejected row (a power of two)
 };
 
@@ -119,15 +126,15 @@ struct ResidualSide {
   }
 };
 
-// One workgroup, a thread per sequence: the acceptance chain. Writes the accepted drafts and,
-// when all are accepted, the bonus token; leaves the first rejected position in jr, clears the
-// row's slice counter and lists the rejected sequences (ascending) for k_verify_residual.
+// One workgroup, a thread per sequence: the acceptance chain. Writes the accepted drafts and, when
+// all are accepted, the count; leaves the first rejected position in jr, clears the row's slice
+// counter and lists the rejected and the accepted sequences (ascending) for k_verify_finish.
 template <class Tin>
-__global__ __launch_bounds__(kThreads) void k_verify_accept(VerifyArgs a, int B) {
+__global__ __launch_bounds__(kThreads) void k_verify_accept(VerifyArgs a) {
   __shared__ uint32_t red[kWaves];
   exp_table_init();
   __syncthreads();
-  const int K = a.K;
+  const int K = a.K, B = a.B;
   const Tin* tgt = static_cast<const Tin*>(a.tgt);
   const Tin* drf = static_cast<const Tin*>(a.drf);
   uint32_t listed = 0;
@@ -149,10 +156,7 @@ __global__ __launch_bounds__(kThreads) void k_verify_accept(VerifyArgs a, int B)
       }
       int32_t* out = a.out_tokens + static_cast<int64_t>(b) * (K + 1);
       for (int i = 0; i <= K; ++i) out[i] = i < j ? a.drafts[b * K + i] : -1;
-      if (j == K) {
-        out[K] = a.tids[b * (K + 1) + K];
-        a.out_count[b] = K + 1;
-      }
+      if (j == K) a.out_count[b] = K + 1;  // (k_verify_finish draws the bonus token)
       a.jr[b] = j;
       a.done[b] = 0;
     }
@@ -160,30 +164,44 @@ __global__ __launch_bounds__(kThreads) void k_verify_accept(VerifyArgs a, int B)
     uint32_t tot;
     const uint32_t at = listed + block_excl_scan<uint32_t>(r, red, &tot);
     if (r) a.rej[at] = b;
+    else if (b < B) a.acc[b - static_cast<int>(at)] = b;
     listed += tot;
   }
   if (threadIdx.x == 0) *a.nrej = static_cast<int32_t>(listed);
 }
 
 // Workgroups per rejected row: the largest power of two with every (row, slice) item on its own
-// workgroup of the grid, at most max_slices.
-__device__ __forceinline__ int residual_slices(int nrej, int grid, int max_slices) {
+// of the `room` workgroups that the bonus rows leave, at most max_slices.
+__device__ __forceinline__ int residual_slices(int nrej, int room, int max_slices) {
   int s = 1;
-  while (2 * s <= max_slices && static_cast<int64_t>(2 * s) * nrej <= grid) s *= 2;
+  while (2 * s <= max_slices && static_cast<int64_t>(2 * s) * nrej <= room) s *= 2;
   return s;
 }
 
+// The residual's LDS: the tabulated terms lie over the sampling kernel's histogram, the rest over its
+// FastSmem.
+struct ResidualSmem {
+  u64 cell[kWaves][kMaxStripes];
+  u64 red[kWaves];
+  u64 sq[4];
+  int si[4];
+};
+static_assert(sizeof(ResidualSmem) <= sizeof(FastSmem), "the residual's scratch lies over FastSmem");
+static_assert(2 * kTab * sizeof(u64) <= kChunk * sizeof(uint32_t), "the tables lie over the histogram");
+
 // One (row, slice) item of the residual draw of rejected sequence b: the slice sums the residual
 // over its share of the row's stripes; the last slice of the row to finish finds the stripe that
-// holds floor(m * R / 2^24) and the token inside it.
+// holds floor(m * R / 2^24) and the token inside it. Returns true (in every thread of the last
+// slice's workgroup) when the row has no residual mass: the caller draws from the target row.
 template <class Tin>
-__device__ __forceinline__ void residual_item(const VerifyArgs& a, int b, int slice, int slices) {
+__device__ __forceinline__ bool residual_item(const VerifyArgs& a, int b, int slice, int slices, uint32_t* big,
+                                              ResidualSmem& m) {
   constexpr bool kBf16 = sizeof(Tin) == 2;
-  __shared__ u64 cell[kWaves][kMaxStripes];
-  __shared__ u64 red[kWaves];
-  __shared__ u64 tab[2][kBf16 ? kTab : 1];
-  __shared__ u64 sq[4];
-  __shared__ int si[4];
+  auto& cell = m.cell;
+  auto& red = m.red;
+  auto& sq = m.sq;
+  auto& si = m.si;
+  u64* const tab[2] = {reinterpret_cast<u64*>(big), reinterpret_cast<u64*>(big) + kTab};
   const int tid = threadIdx.x;
   const int wv = tid / kWave;
   const int K = a.K;
@@ -269,27 +287,27 @@ __device__ __forceinline__ void residual_item(const VerifyArgs& a, int b, int sl
     }
     return kept;
   };
+  auto weight = [&](float xt, float xd, int id, auto tab_mode) -> u64 {
+    u64 pt, qd;
+    if constexpr (decltype(tab_mode)::value) {
+      pt = side[0].term(xt, bf16_key_z(__float_as_uint(xt) >> 16), id);
+      qd = side[1].term(xd, bf16_key_z(__float_as_uint(xd) >> 16), id);
+    } else {
+      pt = side[0].direct(xt, id);
+      qd = side[1].direct(xd, id);
+    }
+    return pt > qd ? pt - qd : 0;
+  };
   auto weights = [&](const float (&vt)[kBlk], const float (&vd)[kBlk], uint32_t kept, int blk, u64 w[kBlk],
                      auto tab_mode) {
 #pragma unroll
     for (int i = 0; i < kBlk; ++i) {
       w[i] = 0;
-      if (kept & (1u << i)) {
-        const int id = blk * kBlk + i;
-        u64 pt, qd;
-        if constexpr (decltype(tab_mode)::value) {
-          pt = side[0].term(vt[i], bf16_key_z(__float_as_uint(vt[i]) >> 16), id);
-          qd = side[1].term(vd[i], bf16_key_z(__float_as_uint(vd[i]) >> 16), id);
-        } else {
-          pt = side[0].direct(vt[i], id);
-          qd = side[1].direct(vd[i], id);
-        }
-        w[i] = pt > qd ? pt - qd : 0;
-      }
+      if (kept & (1u << i)) w[i] = weight(vt[i], vd[i], blk * kBlk + i, tab_mode);
     }
   };
   // Both phases that read the rows, for one mode (tabulated terms or direct ones).
-  auto residual = [&](auto tab_mode) {
+  auto residual = [&](auto tab_mode) -> bool {
     // 1. this slice's per-stripe sums; four stripes' loads of both rows in flight (the draft
     // block is read whether or not a target value in it is kept: a load behind a branch would
     // be waited for alone)
@@ -303,6 +321,109 @@ __device__ __forceinline__ void residual_item(const VerifyArgs& a, int b, int sl
       s = wave_sum<u64>(s);
       if (lane_id() == 0) cell[wv][j - j_begin] = s;
     };
+    if constexpr (decltype(tab_mode)::value) {
+      // Tabulated rows: both values of a word at once. idx2 gives their table entries (the key less
+      // the lowest kept one, saturating: 0 for a dropped token, whose term is 0), in a handful of
+      // packed instructions; a split group's values past its id take entry 0 too. Two stripes of
+      // both rows stay in flight. (As whole blocks of values with a term's own key, range and group
+      // tests a token, four stripes loaded and then worked on, the launch of 149 bonus rows
+      // and 43 rejected ones of 262144 took 58-60 us, two slices a row; 44 now, the bonus rows' own
+      // time. 192 rejected ones, one workgroup each: 143 us a call, now 111.)
+      const int nfull = a.V / kBlk;
+      const uint16_t* pt = nfull > 0 ? reinterpret_cast<const uint16_t*>(rt.p) : g_unused_block;
+      const uint16_t* pd = nfull > 0 ? reinterpret_cast<const uint16_t*>(rd.p) : g_unused_block;
+      uint32_t below[2], split[2];  // (key below the lowest kept, the split group's entry) twice
+      bool fold[2];                 // a zero may be kept: -0.0 takes +0.0's key
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        below[h] = (side[h].tlo - 1u) * 0x10001u;
+        fold[h] = side[h].tlo <= 0x8000u;
+        split[h] = side[h].vcx == side[h].vcx
+                       ? bf16_key_z(__float_as_uint(side[h].vcx) >> 16) - (side[h].tlo - 1u)
+                       : 0u;  // (0: no split group, or one that holds no bf16 value)
+        if (split[h] && (__float_as_uint(side[h].vcx) & 0xFFFFu)) split[h] = 0u;
+      }
+      auto idx2 = [&](uint32_t w, int h) -> ushort2_t {
+        if (fold[h]) {  // (uniform) the halves that are 0x8000 become 0
+          const ushort2_t nz = __builtin_elementwise_min(__builtin_bit_cast(ushort2_t, w ^ 0x80008000u), ones2());
+          w &= ~(__builtin_bit_cast(uint32_t, ones2() - nz) << 15);
+        }
+        return __builtin_elementwise_sub_sat(__builtin_bit_cast(ushort2_t, ok16x2(w)),
+                                             __builtin_bit_cast(ushort2_t, below[h]));
+      };
+      auto load = [&](int j, uint4& t, uint4& d) {
+        const int blk = min(j * kThreads + tid, max(nfull - 1, 0));
+        t = ld_block(pt, blk);
+        d = ld_block(pd, blk);
+      };
+      auto one_stripe = [&](int j, uint4 t, uint4 d) {
+        const int blk = j * kThreads + tid;
+        if (blk >= nfull) {  // the ragged last block; past it nothing (a NaN's bits: entry 0)
+          uint32_t wt[4], wd[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            wt[i] = wd[i] = 0xFFFFFFFFu;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const int id = blk * kBlk + 2 * i + h;
+              if (blk == nfull && id < a.V) {
+                wt[i] = (wt[i] & ~(0xFFFFu << (16 * h))) | static_cast<uint32_t>(ld_global(reinterpret_cast<const uint16_t*>(rt.p) + id)) << (16 * h);
+                wd[i] = (wd[i] & ~(0xFFFFu << (16 * h))) | static_cast<uint32_t>(ld_global(reinterpret_cast<const uint16_t*>(rd.p) + id)) << (16 * h);
+              }
+            }
+          }
+          t = make_uint4(wt[0], wt[1], wt[2], wt[3]);
+          d = make_uint4(wd[0], wd[1], wd[2], wd[3]);
+        }
+        const uint32_t wt[4] = {t.x, t.y, t.z, t.w}, wd[4] = {d.x, d.y, d.z, d.w};
+        u64 s = 0;
+        auto add = [&](uint32_t it, uint32_t id_) {
+          const u64 p = tab[0][it], q = tab[1][id_];
+          s += p > q ? p - q : 0ull;
+        };
+        // (uniform over the wave) its ids, and whether a split group ends at or before their last
+        const int id0 = (j * kThreads + wv * kWave) * kBlk;
+        const bool ends = (split[0] && id0 + kWave * kBlk - 1 > side[0].st.idr) ||
+                          (split[1] && id0 + kWave * kBlk - 1 > side[1].st.idr);
+        if (ends) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const ushort2_t a2 = idx2(wt[i], 0), b2 = idx2(wd[i], 1);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const int id = blk * kBlk + 2 * i + h;
+              const uint32_t it = h ? a2.y : a2.x, jd = h ? b2.y : b2.x;
+              add(split[0] && it == split[0] && id > side[0].st.idr ? 0u : it,
+                  split[1] && jd == split[1] && id > side[1].st.idr ? 0u : jd);
+            }
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const ushort2_t a2 = idx2(wt[i], 0), b2 = idx2(wd[i], 1);
+            add(a2.x, b2.x);
+            add(a2.y, b2.y);
+          }
+        }
+        s = wave_sum<u64>(s);
+        if (lane_id() == 0) cell[wv][j - j_begin] = s;
+      };
+      if (j_begin < j_end) {  // (uniform; a slice past the row's stripes has none)
+        uint4 t0, d0, t1, d1;
+        load(j_begin, t0, d0);
+        load(min(j_begin + 1, j_end - 1), t1, d1);
+        for (int j = j_begin; j < j_end; j += 2) {
+          const uint4 t = t0, d = d0;
+          load(min(j + 2, j_end - 1), t0, d0);
+          one_stripe(j, t, d);
+          if (j + 1 < j_end) {
+            const uint4 u = t1, v = d1;
+            load(min(j + 3, j_end - 1), t1, d1);
+            one_stripe(j + 1, u, v);
+          }
+        }
+      }
+    } else
     for (int j0 = j_begin; j0 < j_end; j0 += 4) {
       if (j0 + 4 <= j_end && (j0 + 4) * kThreads * kBlk <= a.V) {
         // (uniform) four stripes wholly inside both rows
@@ -348,7 +469,7 @@ __device__ __forceinline__ void residual_item(const VerifyArgs& a, int b, int sl
     __syncthreads();
     if (tid == 0) si[2] = static_cast<int>(atomicAdd(&a.done[b], 1u));
     __syncthreads();
-    if (si[2] != slices - 1) return;  // (uniform) another slice finishes the row
+    if (si[2] != slices - 1) return false;  // (uniform) another slice finishes the row
     // 2. (last slice) stripe totals; the stripe where the running sum passes floor(m * R / 2^24)
     if (wv == 0) {
       const int j = lane_id();
@@ -370,12 +491,9 @@ __device__ __forceinline__ void residual_item(const VerifyArgs& a, int b, int sl
       if (hit) sq[2] = inc - t;
     }
     __syncthreads();
-    if (sq[0] == 0) {  // no residual mass: the target's own draw at this position
-      if (tid == 0) {
-        out[jr] = a.tids[b * (K + 1) + jr];
-        a.out_count[b] = jr + 1;
-      }
-      return;
+    if (sq[0] == 0) {  // (uniform) no residual mass: the target's own draw at this position
+      if (tid == 0) a.out_count[b] = jr + 1;
+      return true;
     }
     const u64 tg = sq[1];
     const int js = si[1];
@@ -413,24 +531,44 @@ __device__ __forceinline__ void residual_item(const VerifyArgs& a, int b, int sl
       out[jr] = tok;
       a.out_count[b] = jr + 1;
     }
+    return false;
   };
-  if (kBf16 && tabled)
-    residual(std::integral_constant<bool, kBf16>{});
-  else
-    residual(std::false_type{});
+  if (kBf16 && tabled) return residual(std::integral_constant<bool, kBf16>{});
+  return residual(std::false_type{});
 }
 
-// The residual draws of the rejected rows: a grid of at most one workgroup per CU walks the
-// (row, slice) items, row-major over the list of rejected sequences.
+// The bonus rows of the accepted sequences (k_sample's row code, one workgroup a row) and the
+// residual draws of the rejected ones, (row, slice) items row-major over their list, one item a
+// workgroup: the grid is the larger of B and the CUs the items can use (the LDS holds one
+// workgroup a CU), and the slices are chosen to fit it. (No loop over the items: with one the
+// compiler kept both kinds' values live across it and spilled, 640 bytes a lane, 72-78 us.)
+// `s_` describes the target rows, its out_ids the emitted tokens: row (b, j)'s draw is token (b, j).
 template <class Tin>
-__global__ __launch_bounds__(kThreads) void k_verify_residual(VerifyArgs a) {
+__global__ __launch_bounds__(kThreads) void k_verify_finish(VerifyArgs a, SampleArgs s_) {
+  __shared__ __align__(16) uint32_t big[kChunk];
+  __shared__ FastSmem f;
   exp_table_init();
   const int nrej = *a.nrej;
-  const int slices = residual_slices(nrej, static_cast<int>(gridDim.x), a.max_slices);
-  for (int item = blockIdx.x; item < nrej * slices; item += gridDim.x) {
-    __syncthreads();  // (publishes the exp table; the previous item's LDS is free)
-    residual_item<Tin>(a, a.rej[item / slices], item % slices, slices);
+  const int nacc = a.B - nrej;
+  const int item = blockIdx.x;
+  int r;  // (uniform) the target row to draw from
+  if (item < nacc) {
+    r = a.acc[item] * (a.K + 1) + a.K;
+  } else {
+    const int slices = residual_slices(nrej, static_cast<int>(gridDim.x) - nacc, a.max_slices);
+    const int q = item - nacc;
+    if (q >= nrej * slices) return;
+    const int b = a.rej[q / slices];
+    __syncthreads();  // (publishes the exp table)
+    if (!residual_item<Tin>(a, b, q % slices, slices, big, *reinterpret_cast<ResidualSmem*>(&f))) return;  // (uniform)
+    r = b * (a.K + 1) + a.jr[b];
+    __syncthreads();  // (the residual's LDS is free)
   }
+  const SampleArgs s = globalized(s_);
+  const int tid = threadIdx.x;
+  const uint32_t pw = param_word<false, true>(s, r, tid < kParamWords ? tid : 0);
+  __builtin_amdgcn_sched_barrier(0);  // (issued before the row's first loads)
+  sample_row<Tin, false, false, false, false>(s, r, pw, false, big, f);
 }
 
 }  // namespace vs
