@@ -1,0 +1,79 @@
+"""Top-k rows with penalties that only lower values (repetition >= 1, presence and frequency >= 0): decided
+from the elements above a sampled bound and their counts alone, or handed to the penalty pass. Against the
+oracle, at the sizes and parameters where the route changes."""
+
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from tests.parity import compare_ids, oracle
+from vinfer_amd.registry import BackendContext
+from vinfer_amd.sampler import SAMPLER
+from vinfer_amd.sampling import SamplingParams, pack_history, pack_params
+from vinfer_amd.workloads import Workload
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda", 0)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("V", [16383, 16384, 16385, 24583])  # two whole stripes of 8192 are sampled
+def test_lowered_top_k_rows_match_the_oracle(V, dtype):
+    s = SAMPLER.resolve("hip", BackendContext(DEV, dtype))
+    rng = np.random.default_rng(V)
+    x = torch.randn(24, V, generator=torch.Generator().manual_seed(V)) * 2.5
+    order = x.argsort(dim=1, descending=True)
+    rows, hist, draft = [], [], []
+
+    def row(k, ids, d=0, **kw):
+        rows.append(SamplingParams(**{"temperature": 0.8, "top_k": k, "top_p": 0.95, "repetition_penalty": 1.1,
+                                      "presence_penalty": 0.4, "frequency_penalty": 0.2, **kw}))
+        hist.append([int(i) for i in ids])
+        draft.append(int(d))
+
+    def some(n):
+        return rng.integers(0, V, n)
+
+    for k in (1, 2, 50, 191, 192, 193):  # the largest top-k served, one past it
+        row(k, some(300), order[len(rows), 0])
+    row(50, order[6, :10].repeat(3), order[6, 3])  # the best tokens penalised, the draft among them
+    row(50, order[7, :4000], order[7, 0])  # every candidate penalised: too few stay
+    row(50, order[8, ::2].repeat(2)[:9000], order[8, 1])  # every other one, a long history
+    row(50, some(100), order[9, 5], repetition_penalty=0.9)  # raises values: the penalty pass
+    row(50, some(100), order[10, 5], presence_penalty=-0.5)
+    row(50, some(100), order[11, 5], frequency_penalty=-0.1)
+    row(50, some(100), order[12, 5], repetition_penalty=1.0, presence_penalty=0.0, frequency_penalty=0.0)  # off
+    row(20, [-1, -7, V, V + 5, *some(40)], order[13, 0])  # ids outside the vocabulary
+    row(50, [], order[14, 0])
+    row(50, some(100), order[15, 0])
+    x[15, :] = (x[15] * 0.5).round()  # ties
+    row(50, some(100), order[16, 0])
+    x[16, 40:] = -math.inf  # fewer than k finite
+    row(5, [3, 3, 4], 4)
+    x[17, 100] = math.inf
+    row(5, [3, 3, 4], 4)
+    x[18, 100] = math.nan
+    row(30, some(3000), order[19, 2], min_p=0.2)
+    row(30, some(3000), order[20, 2], temperature=0.0)
+    row(30, order[21, :1].repeat(5000), order[21, 0], frequency_penalty=0.01)  # one id's count
+    row(30, some(20), order[22, 9], repetition_penalty=3e38)  # products overflow to -inf
+    row(30, some(20), 7)
+    x[23, :] = 1.5  # all tied
+    pp = pack_params(rows)
+    ids, off = pack_history(hist)
+    logits = x.to(dtype)
+    u = torch.from_numpy(rng.random(24, dtype=np.float32))
+    w = Workload("lowered", logits, pp, u, ids, off, torch.tensor(draft, dtype=torch.int32))
+    print(f"lowered top-k V={V} {dtype}", flush=True)
+    d = w.to(DEV)
+    for tiles in (False, True):  # (24 rows of this vocabulary: the row launch, then the tile pass's)
+        s.tile_pass = tiles
+        got, dp = s.sample_batch(d.logits, d.params, d.uniforms, d.hist_ids, d.hist_offsets, d.draft_ids)
+        torch.cuda.synchronize()
+        _, bad = compare_ids(got, oracle(w), dp)
+        assert not bad, (tiles, bad[:8])
+    s.tile_pass = True

@@ -571,6 +571,41 @@ __device__ __forceinline__ uint32_t bisect_key_wave(uint32_t lo, uint32_t hi, P 
   return hi;
 }
 
+// Smallest key K in [lo, hi] with pred(val_of(K)) (pred(val_of(hi)) must hold; pred is false
+// below the answer and true from it on), by the 64 lanes of one wave: 64 probes per round.
+// `guess` is an estimate of the answer: the first round probes the 64 keys around it.
+template <class P>
+__device__ __forceinline__ uint32_t wave_bisect(uint32_t lo, uint32_t hi, uint32_t guess, P pred) {
+  const uint32_t l = lane_id();
+  if (lo < hi) {
+    const uint32_t g = guess < lo ? lo : (guess > hi ? hi : guess);
+    const uint32_t g0 = g - lo >= 32u ? g - 32u : lo;  // probes g0 .. g0 + 63, clamped to hi
+    const u64 p64 = static_cast<u64>(g0) + l;
+    const uint32_t probe = p64 < hi ? static_cast<uint32_t>(p64) : hi;
+    const u64 hm = __ballot(pred(val_of(probe)));
+    const int first = hm ? __ffsll(static_cast<long long>(hm)) - 1 : 64;
+    // (first comes from a ballot: the same in every lane, so the lanes are read directly)
+    if (first < 64) hi = __builtin_amdgcn_readlane(probe, first);
+    if (first > 0) lo = __builtin_amdgcn_readlane(probe, first - 1) + 1;
+    if (first == 0) lo = lo < hi ? lo : hi;
+  }
+  while (lo < hi) {
+    // probes lo + step*(l+1) - 1 for l = 0..63 split [lo, hi] into 64 pieces
+    const u64 span = static_cast<u64>(hi) - lo;
+    const u64 step = (span + 63) / 64;
+    const u64 probe64 = static_cast<u64>(lo) + step * (l + 1) - 1;
+    const uint32_t probe = probe64 < hi ? static_cast<uint32_t>(probe64) : hi;
+    const u64 hm = __ballot(pred(val_of(probe)));
+    // the first probe that holds bounds the answer from above; the one before it from below
+    const int first = hm ? __ffsll(static_cast<long long>(hm)) - 1 : 64;
+    const uint32_t nhi = first < 64 ? __builtin_amdgcn_readlane(probe, first) : hi;
+    const uint32_t nlo = first > 0 ? __builtin_amdgcn_readlane(probe, first - 1) + 1 : lo;
+    lo = nlo;
+    hi = nhi;
+  }
+  return hi;
+}
+
 // First element index (ascending id) where the running count of w(x, id) (0 or 1) exceeds
 // `target` (clamped to total - 1). Returns -1 when no element has w = 1.
 template <class Tin, class W>
@@ -1278,6 +1313,233 @@ __device__ __forceinline__ bool sorted_tail(const SampleArgs& a, const Row<Tin>&
   return true;
 }
 
+// ---- top-k rows whose penalties only lower values ----------------------------------------------
+// With rep >= 1, pres >= 0 and freq >= 0 no penalised value is above its original (each step of
+// apply_penalty rounds a value no larger). So every token whose penalised value reaches a bound
+// tau has an original value that does, and a top-k row needs the counts of those few tokens alone:
+// one pass over the row stages the elements >= tau, their ids go into an LDS hash table, one pass
+// over the history counts the ids it holds, and the candidates' penalised values >= tau, when at
+// least K of them, hold the top K (and the row's max). In place of the penalty pass -- the whole
+// history's presence bitmap, ranks, counts, (id, count) pairs and a gather of every distinct id's
+// value, ~30 us of a 62 us row at 16K ids -- and of the masked passes after it.
+// tau: the bin (13 key bits) of the m-th largest of the first kLowDepth stripes' per-thread maxima,
+// m three times the K-th's share of that sample (penalised candidates may fall below tau).
+// Returns false, with nothing written, for a row it does not decide (too few or too many
+// candidates, a NaN or +inf, a threshold below tau): the caller runs the penalty pass.
+// Measured (1024 fp32 rows of 151936, top-k 50, histories up to 32768): 255.0 -> 160.7 us a launch.
+constexpr int kLowK = 192;       // top-k served
+constexpr int kLowDepth = 2;     // stripes sampled
+constexpr int kLowCap = 1023;    // staged candidates: one a thread, and one for the draft id
+constexpr int kLowSlots = 4096;  // hash table
+
+// Sorts c[0, n), n <= kThreads, into out[0, min(n, kSortCap)): descending value, ascending id (each
+// entry's rank is the count of larger keys). `kk` holds n staged keys; the result is visible on
+// return.
+__device__ __forceinline__ void sort_top(const Cand* c, int n, u64* kk, Cand* out) {
+  const int i = threadIdx.x;
+  Cand me{0.0f, 0};
+  u64 km = 0;
+  if (i < n) {
+    me = c[i];
+    km = (static_cast<u64>(key_of(me.x)) << 32) | (0xFFFFFFFFu - static_cast<uint32_t>(me.id));
+    kk[i] = km;
+  }
+  lds_barrier();
+  if (i < n) {
+    uint32_t rank = 0;
+#pragma unroll 8
+    for (int j = 0; j < n; ++j) rank += kk[j] > km ? 1u : 0u;  // (j uniform: one broadcast read per wave)
+    if (rank < static_cast<uint32_t>(kSortCap)) out[rank] = me;
+  }
+  lds_barrier();
+}
+
+template <class Tin>
+__device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, Row<Tin> row, const RowParams& p, GenericSmem& g,
+                                                 int r) {
+  const int tid = threadIdx.x;
+  const int V = row.V;
+  const int L = p.h1 - p.h0;
+  // (uniform)
+  if (!(p.T > 0.0f) || p.K < 1 || p.K >= V || p.K > kLowK || L < 1 || a.out_probs) return false;
+  if (!(p.rep >= 1.0f && p.rep < INFINITY && p.pres >= 0.0f && p.freq >= 0.0f)) return false;
+  if (p.rep == 1.0f && p.pres == 0.0f && p.freq == 0.0f) return false;  // (no penalties: the generic path's own stream)
+  if (V / kBlk / kThreads < kLowDepth) return false;
+  uint32_t* const area = reinterpret_cast<uint32_t*>(&g);
+  uint32_t* const hkey = area + kBitmapOffset;      // the hash table's ids
+  uint32_t* const hcnt = hkey + kLowSlots;          // and counts
+  uint32_t* const h13 = area + kMatchOffset;        // the sample's bins, then:
+  Cand* const cand = reinterpret_cast<Cand*>(h13);  // the penalised candidates,
+  u64* const kk = reinterpret_cast<u64*>(h13 + 2048);       // their sort keys
+  Cand* const srt = reinterpret_cast<Cand*>(h13 + 4096);    // and the sorted list
+  constexpr int kBins = 8192;
+  Cand* const stage = reinterpret_cast<Cand*>(h13 + kBins);
+  static_assert(kMatchOffset + kBins + 2 * (kLowCap + 1) <= kChunk && 2 * kLowSlots <= kMatchOffset - kBitmapOffset &&
+                    4096 + 2 * kSortCap <= kBins && kLowCap < kThreads,
+                "the row's LDS areas");
+  uint32_t* const sh = g.rdx.bk;  // [0] the bin, [1] above it, [2] candidates, [3] a NaN or +inf
+  WholeBlock<Tin> q[kLowDepth];
+#pragma unroll
+  for (int k = 0; k < kLowDepth; ++k) q[k].load(row.p, k * kThreads + tid);
+  for (int i = tid; i < kBins / 4; i += kThreads) reinterpret_cast<uint4*>(h13)[i] = make_uint4(0, 0, 0, 0);
+  for (int i = tid; i < kLowSlots / 4; i += kThreads) {
+    reinterpret_cast<uint4*>(hkey)[i] = make_uint4(kEmpty, kEmpty, kEmpty, kEmpty);
+    reinterpret_cast<uint4*>(hcnt)[i] = make_uint4(0, 0, 0, 0);
+  }
+  if (tid < 4) sh[tid] = 0;
+  lds_barrier();
+  float v[kLowDepth][kBlk];
+  float mx = -INFINITY;  // (IEEE maximum: a NaN stays)
+#pragma unroll
+  for (int k = 0; k < kLowDepth; ++k) {
+    q[k].values(v[k]);
+    mx = __builtin_elementwise_maximum(mx, max_of8(v[k]));
+  }
+  atomicAdd(&h13[key_of(mx) >> 19], 1u);
+  lds_barrier();
+  {
+    // the bin of the m-th largest maximum (thread t sums bins 8191 - 8t .. 8184 - 8t, descending)
+    constexpr u64 kSample = static_cast<u64>(kLowDepth) * kThreads * kBlk;
+    const uint32_t m =
+        static_cast<uint32_t>((3ull * static_cast<u64>(p.K) * kSample + static_cast<u64>(V) - 1) / static_cast<u64>(V)) + 2u;
+    uint32_t c8[8], s8 = 0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const uint4 w = reinterpret_cast<const uint4*>(h13)[kBins / 4 - 1 - 2 * tid - h];
+      c8[4 * h] = w.w;
+      c8[4 * h + 1] = w.z;
+      c8[4 * h + 2] = w.y;
+      c8[4 * h + 3] = w.x;
+      s8 += w.x + w.y + w.z + w.w;
+    }
+    uint32_t tot;
+    uint32_t run = block_excl_scan<uint32_t>(s8, g.rdx.hcnt, &tot);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (run < m && m <= run + c8[i]) sh[0] = static_cast<uint32_t>(kBins - 1 - 8 * tid - i);
+      run += c8[i];
+    }
+  }
+  lds_barrier();
+  const float tau = val_of(max(sh[0] << 19, key_of(-INFINITY)));  // (the bin's least value; bin 0: none found)
+  if (!(tau > -INFINITY && tau < INFINITY)) return false;         // (uniform)
+  auto append = [&](float x, int id) {
+    const bool c = x >= tau;
+    const u64 bal = __ballot(c);  // (one counter update per wave round)
+    if (bal) {
+      const int leader = __ffsll(static_cast<long long>(bal)) - 1;
+      uint32_t at = 0;
+      if (lane_id() == leader) at = atomicAdd(&sh[2], static_cast<uint32_t>(__popcll(bal)));
+      at = __builtin_amdgcn_readlane(at, leader) + lanes_below(bal);
+      if (c && at < static_cast<uint32_t>(kLowCap)) stage[at] = Cand{x, id};
+    }
+  };
+  if (__ballot(!(mx < tau))) {
+#pragma unroll
+    for (int k = 0; k < kLowDepth; ++k)
+#pragma unroll
+      for (int i = 0; i < kBlk; ++i) append(v[k][i], (k * kThreads + tid) * kBlk + i);
+  }
+  for_each_block_ahead(row, [&](const float (&w)[kBlk], uint32_t out, int b) {
+    float x[kBlk];
+#pragma unroll
+    for (int i = 0; i < kBlk; ++i) x[i] = out & (1u << i) ? -INFINITY : w[i];
+    const float bx = max_of8(x);
+    mx = __builtin_elementwise_maximum(mx, bx);
+    if (__ballot(!(bx < tau))) {  // (uniform over the wave)
+#pragma unroll
+      for (int i = 0; i < kBlk; ++i) append(x[i], b * kBlk + i);
+    }
+  }, kLowDepth);
+  if (!(mx < INFINITY)) sh[3] = 1;
+  lds_barrier();
+  const uint32_t n0 = sh[2];
+  const uint32_t K = static_cast<uint32_t>(p.K);
+  if (sh[3] || n0 < K || n0 > static_cast<uint32_t>(kLowCap)) return false;  // (uniform)
+  // the candidates' ids (and the draft's) into the table: thread t the t-th, the last thread the draft's
+  const bool want_draft = p.draft >= 0 && p.draft < V && a.out_dprob;  // (uniform)
+  const bool mine = tid < static_cast<int>(n0);
+  const bool drafts = want_draft && tid == kThreads - 1;
+  Cand me{0.0f, 0};
+  if (mine) me = stage[tid];
+  if (drafts) me = Cand{load_one<Tin>(row.p, p.draft), p.draft};
+  uint32_t slot = (static_cast<uint32_t>(me.id) * 2654435761u) >> (32 - 12);
+  static_assert(kLowSlots == 1 << 12, "hash bits");
+  if (mine || drafts) {
+    // (at most 1024 of 4096 slots are taken: every probe sequence ends)
+    while (true) {
+      const uint32_t prev = atomicCAS(&hkey[slot], kEmpty, static_cast<uint32_t>(me.id));
+      if (prev == kEmpty || prev == static_cast<uint32_t>(me.id)) break;
+      slot = (slot + 1) & (kLowSlots - 1);
+    }
+  }
+  if (tid == 0) sh[2] = 0;
+  lds_barrier();
+  for_each_id(a.pen.hist + p.h0, L, [&](int id, int) {
+    uint32_t h = (static_cast<uint32_t>(id) * 2654435761u) >> (32 - 12);
+    while (true) {
+      const uint32_t key = hkey[h];
+      if (key == kEmpty) break;  // (an id of -1 too)
+      if (key == static_cast<uint32_t>(id)) {
+        atomicAdd(&hcnt[h], 1u);
+        break;
+      }
+      h = (h + 1) & (kLowSlots - 1);
+    }
+  });
+  lds_barrier();
+  // penalised values: the candidates' that stay >= tau, and the draft's (the row's only "exception")
+  int32_t* const xid = reinterpret_cast<int32_t*>(g.rdx.hcnt) + 64;  // (past sorted_tail's results)
+  float* const xval = reinterpret_cast<float*>(xid + 1);
+  const int c = mine || drafts ? static_cast<int>(hcnt[slot]) : 0;
+  const float xp = c > 0 ? apply_penalty(me.x, c, p.rep, p.pres, p.freq) : me.x;
+  if (drafts) {
+    xid[0] = p.draft;
+    xval[0] = xp;
+  }
+  {
+    const bool in = mine && xp >= tau;
+    const u64 bal = __ballot(in);
+    if (bal) {
+      const int leader = __ffsll(static_cast<long long>(bal)) - 1;
+      uint32_t at = 0;
+      if (lane_id() == leader) at = atomicAdd(&sh[2], static_cast<uint32_t>(__popcll(bal)));
+      at = __builtin_amdgcn_readlane(at, leader) + lanes_below(bal);
+      if (in) cand[at] = Cand{xp, me.id};
+    }
+  }
+  lds_barrier();
+  const int n = static_cast<int>(sh[2]);
+  if (n < p.K) return false;  // (uniform)
+  sort_top(cand, n, kk, srt);
+  const float T = p.T;
+  const float mz = srt[0].x / T;
+  if (!(mz > -INFINITY && mz < INFINITY)) return false;  // (uniform) point rows
+  // the exact thresholds: the K-th largest's z, and min-p's
+  if (tid < kWave) {
+    const uint32_t lo_key = key_of(-INFINITY);
+    const float kx = srt[p.K - 1].x;
+    const float kz = kx / T;
+    float x0 = val_of(wave_bisect(lo_key, key_of(kx), key_of(kz * T), [&](float x) { return x / T >= kz; }));
+    if (p.mp > 0.0f) {
+      const double dmp = static_cast<double>(p.mp);
+      const float xm = val_of(wave_bisect(lo_key, key_of(srt[0].x), key_of(T * (mz + __logf(p.mp))),
+                                          [&](float x) { return ptilde(x, T, mz) >= dmp; }));
+      x0 = xm > x0 ? xm : x0;
+    }
+    if (tid == 0) reinterpret_cast<float*>(sh)[3] = x0;
+  }
+  lds_barrier();
+  Kept k;
+  k.x0 = reinterpret_cast<const float*>(sh)[3];
+  // every element >= x0 must be in the sorted list
+  if (!(k.x0 >= tau) || (n > kSortCap && srt[kSortCap - 1].x >= k.x0)) return false;  // (uniform)
+  row.eid = xid;
+  row.eval = xval;
+  row.nexc = want_draft ? 1 : 0;
+  return sorted_tail<false>(a, row, p, g, g.srch, srt, min(n, kSortCap), mz, k, r);
+}
+
 // have_bitmap: the penalty pass left the penalised ids' bitmap at kBitmapOffset.
 template <bool STATE, class Tin>
 __device__ __forceinline__ void generic_row(const SampleArgs& a, Row<Tin> row, const RowParams& p, GenericSmem& g,
@@ -1909,41 +2171,6 @@ __device__ __forceinline__ WalkResult wave_walk(const uint32_t* hist, FastSmem& 
   res.q = readlane64(hi ? eq[1] : eq[0], at);
   res.above = readlane64(hi ? acc_h[1] : acc_h[0], at);
   return res;
-}
-
-// Smallest key K in [lo, hi] with pred(val_of(K)) (pred(val_of(hi)) must hold; pred is false
-// below the answer and true from it on), by the 64 lanes of one wave: 64 probes per round.
-// `guess` is an estimate of the answer: the first round probes the 64 keys around it.
-template <class P>
-__device__ __forceinline__ uint32_t wave_bisect(uint32_t lo, uint32_t hi, uint32_t guess, P pred) {
-  const uint32_t l = lane_id();
-  if (lo < hi) {
-    const uint32_t g = guess < lo ? lo : (guess > hi ? hi : guess);
-    const uint32_t g0 = g - lo >= 32u ? g - 32u : lo;  // probes g0 .. g0 + 63, clamped to hi
-    const u64 p64 = static_cast<u64>(g0) + l;
-    const uint32_t probe = p64 < hi ? static_cast<uint32_t>(p64) : hi;
-    const u64 hm = __ballot(pred(val_of(probe)));
-    const int first = hm ? __ffsll(static_cast<long long>(hm)) - 1 : 64;
-    // (first comes from a ballot: the same in every lane, so the lanes are read directly)
-    if (first < 64) hi = __builtin_amdgcn_readlane(probe, first);
-    if (first > 0) lo = __builtin_amdgcn_readlane(probe, first - 1) + 1;
-    if (first == 0) lo = lo < hi ? lo : hi;
-  }
-  while (lo < hi) {
-    // probes lo + step*(l+1) - 1 for l = 0..63 split [lo, hi] into 64 pieces
-    const u64 span = static_cast<u64>(hi) - lo;
-    const u64 step = (span + 63) / 64;
-    const u64 probe64 = static_cast<u64>(lo) + step * (l + 1) - 1;
-    const uint32_t probe = probe64 < hi ? static_cast<uint32_t>(probe64) : hi;
-    const u64 hm = __ballot(pred(val_of(probe)));
-    // the first probe that holds bounds the answer from above; the one before it from below
-    const int first = hm ? __ffsll(static_cast<long long>(hm)) - 1 : 64;
-    const uint32_t nhi = first < 64 ? __builtin_amdgcn_readlane(probe, first) : hi;
-    const uint32_t nlo = first > 0 ? __builtin_amdgcn_readlane(probe, first - 1) + 1 : lo;
-    lo = nlo;
-    hi = nhi;
-  }
-  return hi;
 }
 
 // The id of the j-th (0-based, ascending id) token whose penalised value is vd: bulk positions
@@ -3426,6 +3653,10 @@ __device__ __forceinline__ void sample_row(const SampleArgs& a, int r, uint32_t 
   }
   RowParams p = f.prm;
   p.u = p.u >= 0.0f ? p.u : 0.0f;
+  if constexpr (PEN && !STATE && sizeof(Tin) == 4) {
+    if (lowered_topk_row<Tin>(a, row, p, g, r)) return;
+    lds_barrier();  // (every thread is done with its LDS)
+  }
   // the generic path: the penalty pass writes the penalised ids and values to the workspace
   int ne = 0;
   bool have_bitmap = false;
