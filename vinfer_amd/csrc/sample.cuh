@@ -3643,6 +3643,12 @@ __device__ __forceinline__ void sample_row(const SampleArgs& a, int r, uint32_t 
       if (tile_row<PEN, Tin>(a, row, pt, g, r)) return;
       lds_barrier();  // (every thread is done with the tile path's LDS)
     }
+    if constexpr (PEN && sizeof(Tin) == 2) {
+      // (bf16 rows here, whose parameters are at hand: no histogram and no member search either;
+      // in the plain launch the histogram's first loads go out before the parameters are known)
+      if (lowered_topk_row<Tin>(a, row, pt, g, r)) return;
+      lds_barrier();  // (every thread is done with its LDS)
+    }
   }
   if constexpr (sizeof(Tin) == 2) {
     if (__builtin_expect(fast_row<PEN, STATE, SPLIT>(a, row, f.prm, big, f, g.srch, pw, r), 1)) return;
