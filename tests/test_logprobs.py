@@ -131,3 +131,44 @@ def test_gpu_logprobs_on_unaligned_strided_rows(dtype):
         assert ids[b].tolist() == wids
         fin = np.isfinite(wv)
         np.testing.assert_allclose(lps[b].cpu().numpy()[fin], wv[fin], rtol=1e-6, atol=2e-6)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=str)
+@pytest.mark.parametrize("V", [16383, 16384, 16385, 33000])  # two whole stripes of 8192 are sampled
+def test_gpu_logprobs_around_the_sampled_bound(V, dtype):
+    # rows the one-pass form decides and rows it hands on: the max far above the sample's, ties past its
+    # list, -inf but for a few, NaN and infinities outside the sample; against torch in 64 bits
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(V)
+    x = torch.randn(12, V, generator=g, device=dev) * 2
+    x[1, V - 1] += 40.0  # (past the sample where V > 16384)
+    x[2, V - 1] += 90.0
+    x[3] = (x[3] * 0.5).round()
+    x[4] = 0.25
+    x[5] = -math.inf
+    x[5, V - 9 : V - 2] = 1.0
+    x[6, V - 1] = math.nan
+    x[7, V - 1] = math.inf
+    x[8] = -math.inf
+    x[9] = x[9] * 0.01 - 500.0
+    x[10, ::3] = -0.0
+    x[10, 1::3] = -5.0
+    x[10, 2::3] = 0.0
+    x[11] = x[11].sort().values  # ascending: the largest last
+    logits = x.to(dtype)
+    tokens = torch.randint(0, V, (12,), generator=g, device=dev).to(torch.int32)
+    s = SAMPLER.resolve("hip", BackendContext(dev, dtype))
+    for n in (0, 1, 20, 32):
+        print(f"logprobs sampled bound V={V} {dtype} n={n}", flush=True)
+        tok, ids, lps = s.logprobs(logits, tokens, n)
+        want = torch.log_softmax(logits.double(), dim=1)
+        order = logits.double().sort(dim=1, descending=True, stable=True)
+        for r in range(12):
+            if r in (6, 7, 8):
+                assert tok[r].isnan() and lps[r].isnan().all()
+                continue
+            # (fp32 exponentials summed in fp64: 1e-7 of the sum; the result rounded to fp32 once)
+            torch.testing.assert_close(tok[r].double(), want[r, tokens[r].long()], rtol=2e-6, atol=1e-6)
+            assert torch.equal(ids[r].long(), order.indices[r, :n])
+            torch.testing.assert_close(lps[r].double(), want[r, order.indices[r, :n]], rtol=2e-6, atol=1e-6)

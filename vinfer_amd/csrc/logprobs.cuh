@@ -4,7 +4,9 @@
 // ascending id). The sum adds fp32 exponentials in fp64; a row whose max is not finite reports
 // NaN throughout.
 //
-// One workgroup per row: a pass for the max and a histogram of the keys' top 13 bits, which
+// One workgroup per row. Rows of at least two stripes take one pass (lp_stream). The others, and the
+// rows it does not serve: for bf16 one pass over a 16-bit key histogram (lp_one_pass), and for the
+// rest a pass for the max and a histogram of the keys' top 13 bits, which
 // gives the bin of the n-th largest key; a pass that sums the exponentials and copies every
 // element of that bin and the bins above to LDS (at most kCandCap); the n-th largest key by a
 // radix descent over that list, and the top n from it. A row whose top bins hold more than
@@ -189,11 +191,124 @@ __device__ __forceinline__ bool lp_one_pass(const LogprobArgs& a, const Row<uint
   return ok;
 }
 
+// Rows of at least two stripes, in one pass and without a histogram: each element's fp32
+// exponential against the sample's max M0 is added in fp64 as it is read, but for the elements >= tau
+// (the bin of about the 3n-th largest of the row, from the first two stripes' per-thread maxima),
+// which are staged: they hold the row's max and its top n, and their exponentials are taken in
+// fp64 against the row's max M, so that M0's distance from M costs the large terms no precision.
+// Their sum is in fixed point: the staging order varies, the sum does not. Returns false, with
+// nothing written, for a row it does not serve (a NaN, an infinite or no finite max, an M more than
+// 60 above M0, fewer staged elements than n or more than kLpCap: massive ties).
+// A histogram's LDS atomic an element (about 9 clocks a wave) and a thread's three largest kept
+// an element bound the pass below it; this one is bound by the reads and the exponentials.
+// Measured (256 bf16 rows of 151936, top 20, half certain and half flat): 27-52 us a call with
+// lp_one_pass, by how many rows' lists were complete, 25.3-28.5 for all of them now (12.5 of it SIMD
+// time).
+constexpr int kLpCap = 1023;
+constexpr int kLpDepth = 2;
+constexpr int kLpBins = 8192;
+constexpr int kLpWords = kLpBins + 2 * (kLpCap + 1);  // LDS words: bins (then sort keys and list), staged elements
+template <class Tin>
+__device__ __forceinline__ bool lp_stream(const LogprobArgs& a, const Row<Tin>& row, int r, uint32_t* area, uint32_t* sh,
+                                          uint32_t* red32, u64* red64) {
+  const int tid = threadIdx.x;
+  const int V = row.V;
+  const int n = a.n_top;
+  if (V / kBlk / kThreads < kLpDepth) return false;  // (uniform)
+  Cand* const stage = reinterpret_cast<Cand*>(area + kLpBins);
+  WholeBlock<Tin> q[kLpDepth];
+#pragma unroll
+  for (int k = 0; k < kLpDepth; ++k) q[k].load(row.p, k * kThreads + tid);
+  for (int i = tid; i < kLpBins / 4; i += kThreads) reinterpret_cast<uint4*>(area)[i] = make_uint4(0, 0, 0, 0);
+  if (tid < 8) sh[tid] = 0;  // [0] the bin, [2] staged, [3] a NaN or +inf, [4] M0's key, [5] M's
+  __syncthreads();           // (the exp table too)
+  float v[kLpDepth][kBlk];
+  float mx = -INFINITY;  // (IEEE maximum: a NaN stays)
+#pragma unroll
+  for (int k = 0; k < kLpDepth; ++k) {
+    q[k].values(v[k]);
+    mx = __builtin_elementwise_maximum(mx, max_of8(v[k]));
+  }
+  auto umax = [](uint32_t x, uint32_t y) { return x > y ? x : y; };
+  atomicAdd(&area[key_of(mx) >> 19], 1u);
+  {
+    const uint32_t wm = dpp::reduce(key_of(mx), umax);
+    if (lane_id() == 0) atomicMax(&sh[4], wm);
+  }
+  __syncthreads();
+  const uint32_t nn = static_cast<uint32_t>(n) < static_cast<uint32_t>(V) ? static_cast<uint32_t>(n) : static_cast<uint32_t>(V);
+  find_top_bin(area, kLpBins, sample_rank<kLpDepth>(nn, V), red32, &sh[0]);
+  __syncthreads();
+  const float tau = val_of(max(sh[0] << 19, key_of(-INFINITY)));  // (the bin's least value; bin 0: none found)
+  const float M0 = val_of(sh[4]);
+  if (!(tau > -INFINITY && M0 < INFINITY)) return false;  // (uniform; a NaN M0 too)
+  double s = 0.0;
+  auto block = [&](float (&x)[kBlk], float bx, int b) {
+    if (__ballot(!(bx < tau))) {  // (uniform over the wave)
+#pragma unroll
+      for (int i = 0; i < kBlk; ++i) {
+        const bool c = x[i] >= tau;
+        const u64 bal = __ballot(c);  // (one counter update per wave round)
+        if (bal) {
+          const int leader = __ffsll(static_cast<long long>(bal)) - 1;
+          uint32_t at = 0;
+          if (lane_id() == leader) at = atomicAdd(&sh[2], static_cast<uint32_t>(__popcll(bal)));
+          at = __builtin_amdgcn_readlane(at, leader) + lanes_below(bal);
+          if (c && at < static_cast<uint32_t>(kLpCap)) stage[at] = Cand{x[i], b * kBlk + i};
+          if (c) x[i] = -INFINITY;
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kBlk; ++i) s += static_cast<double>(__expf(x[i] - M0));
+  };
+#pragma unroll
+  for (int k = 0; k < kLpDepth; ++k) block(v[k], max_of8(v[k]), k * kThreads + tid);
+  for_each_block_ahead(row, [&](const float (&w)[kBlk], uint32_t out, int b) {
+    float x[kBlk];
+#pragma unroll
+    for (int i = 0; i < kBlk; ++i) x[i] = out & (1u << i) ? -INFINITY : w[i];
+    const float bx = max_of8(x);
+    mx = __builtin_elementwise_maximum(mx, bx);
+    block(x, bx, b);
+  }, kLpDepth);
+  if (!(mx < INFINITY)) sh[3] = 1;
+  {
+    const uint32_t wm = dpp::reduce(key_of(mx), umax);
+    if (lane_id() == 0) atomicMax(&sh[5], wm);
+  }
+  __syncthreads();
+  const uint32_t n0 = sh[2];
+  const float M = val_of(sh[5]);
+  if (sh[3] || n0 < nn || n0 < 1 || n0 > static_cast<uint32_t>(kLpCap) || !(M - M0 <= 60.0f)) return false;  // (uniform)
+  u64 qc = 0;
+  if (tid < static_cast<int>(n0)) qc = mass_q(exp_nonpos(static_cast<double>(stage[tid].x) - static_cast<double>(M)));
+  qc = block_sum<u64>(qc, red64);
+  s = block_sum<double>(s, reinterpret_cast<double*>(red64));
+  const double lse = static_cast<double>(M) + log(s * exp_nonpos(static_cast<double>(M0) - static_cast<double>(M)) +
+                                                  static_cast<double>(qc) * (1.0 / kMassScale));
+  auto lp = [&](float x) -> float { return static_cast<float>(static_cast<double>(x) - lse); };
+  if (tid == 0 && a.out_token && a.tokens) {
+    const int t = a.tokens[r];
+    a.out_token[r] = t >= 0 && t < V ? lp(load_one<Tin>(row.p, t)) : NAN;
+  }
+  if (n <= 0) return true;
+  Cand* const srt = reinterpret_cast<Cand*>(area + 2 * (kLpCap + 1));
+  static_assert(kMaxTop <= kSortCap && 2 * (kLpCap + 1) + 2 * kSortCap <= kLpBins, "the sort lies over the bins");
+  sort_top(stage, static_cast<int>(n0), reinterpret_cast<u64*>(area), srt);
+  for (int i = tid; i < n; i += kThreads) {
+    const bool in = i < static_cast<int>(nn);  // (n > V: the rest are empty)
+    a.out_top_ids[static_cast<int64_t>(r) * n + i] = in ? srt[i].id : -1;
+    a.out_top[static_cast<int64_t>(r) * n + i] = in ? lp(srt[i].x) : -INFINITY;
+  }
+  return true;
+}
+
 template <class Tin, bool TILES = false>
 __global__ __launch_bounds__(kThreads) void k_logprobs(LogprobArgs a) {
   constexpr int kBins = 8192;  // by the top 13 bits of the ordered key
   constexpr bool kOnePass = sizeof(Tin) == 2 && !TILES;  // (bf16 rows: one pass over a 16-bit histogram)
-  __shared__ uint32_t h13[kOnePass ? 32768 : kBins];  // (then the candidate list: kCandCap 8-byte entries)
+  __shared__ __align__(16) uint32_t h13[kOnePass ? 32768 : TILES ? kBins : kLpWords];  // (then the candidate list: kCandCap 8-byte entries)
   __shared__ Radix rdx;
   __shared__ Search srch;
   __shared__ Cand top[kMaxTop];
@@ -211,7 +326,11 @@ __global__ __launch_bounds__(kThreads) void k_logprobs(LogprobArgs a) {
   row.eval = nullptr;
   row.nexc = 0;
   const int n = a.n_top;
-  if constexpr (TILES) exp_table_init();  // (published by the first barrier below)
+  exp_table_init();  // (published by the first barrier below)
+  if constexpr (!TILES) {
+    if (lp_stream<Tin>(a, row, r, h13, sh, rdx.hcnt, srch.red64)) return;  // (uniform)
+    __syncthreads();  // (every thread is done with its LDS)
+  }
   Cand* cand = reinterpret_cast<Cand*>(h13);
   float M = 0.0f;
   bool finite = false;

@@ -1313,6 +1313,38 @@ __device__ __forceinline__ bool sorted_tail(const SampleArgs& a, const Row<Tin>&
   return true;
 }
 
+// ---- a bound on a row's largest elements from a sample -------------------------------------------
+// The rank, among the per-thread maxima of the first DEPTH stripes (16 elements each at DEPTH 2),
+// that about three times the n largest of the row lie above.
+template <int DEPTH>
+__device__ __forceinline__ uint32_t sample_rank(uint32_t n, int V) {
+  constexpr u64 kSample = static_cast<u64>(DEPTH) * kThreads * kBlk;
+  return static_cast<uint32_t>((3ull * n * kSample + static_cast<u64>(V) - 1) / static_cast<u64>(V)) + 2u;
+}
+// The bin of the m-th largest of the 8192 counted keys, to *bin (left alone when fewer were
+// counted); every thread calls, a barrier publishes. Thread t sums bins 8191 - 8t .. 8184 - 8t,
+// descending.
+__device__ __forceinline__ void find_top_bin(const uint32_t* h13, int bins, uint32_t m, uint32_t* red, uint32_t* bin) {
+  const int tid = threadIdx.x;
+  uint32_t c8[8], s8 = 0;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const uint4 w = reinterpret_cast<const uint4*>(h13)[bins / 4 - 1 - 2 * tid - h];
+    c8[4 * h] = w.w;
+    c8[4 * h + 1] = w.z;
+    c8[4 * h + 2] = w.y;
+    c8[4 * h + 3] = w.x;
+    s8 += w.x + w.y + w.z + w.w;
+  }
+  uint32_t tot;
+  uint32_t run = block_excl_scan<uint32_t>(s8, red, &tot);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    if (run < m && m <= run + c8[i]) *bin = static_cast<uint32_t>(bins - 1 - 8 * tid - i);
+    run += c8[i];
+  }
+}
+
 // ---- top-k rows whose penalties only lower values ----------------------------------------------
 // With rep >= 1, pres >= 0 and freq >= 0 no penalised value is above its original (each step of
 // apply_penalty rounds a value no larger). So every token whose penalised value reaches a bound
@@ -1365,6 +1397,7 @@ __device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, Row<Tin> r
   if (!(p.rep >= 1.0f && p.rep < INFINITY && p.pres >= 0.0f && p.freq >= 0.0f)) return false;
   if (p.rep == 1.0f && p.pres == 0.0f && p.freq == 0.0f) return false;  // (no penalties: the generic path's own stream)
   if (V / kBlk / kThreads < kLowDepth) return false;
+  const uint32_t K = static_cast<uint32_t>(p.K);
   uint32_t* const area = reinterpret_cast<uint32_t*>(&g);
   uint32_t* const hkey = area + kBitmapOffset;      // the hash table's ids
   uint32_t* const hcnt = hkey + kLowSlots;          // and counts
@@ -1397,29 +1430,7 @@ __device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, Row<Tin> r
   }
   atomicAdd(&h13[key_of(mx) >> 19], 1u);
   lds_barrier();
-  {
-    // the bin of the m-th largest maximum (thread t sums bins 8191 - 8t .. 8184 - 8t, descending)
-    constexpr u64 kSample = static_cast<u64>(kLowDepth) * kThreads * kBlk;
-    const uint32_t m =
-        static_cast<uint32_t>((3ull * static_cast<u64>(p.K) * kSample + static_cast<u64>(V) - 1) / static_cast<u64>(V)) + 2u;
-    uint32_t c8[8], s8 = 0;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const uint4 w = reinterpret_cast<const uint4*>(h13)[kBins / 4 - 1 - 2 * tid - h];
-      c8[4 * h] = w.w;
-      c8[4 * h + 1] = w.z;
-      c8[4 * h + 2] = w.y;
-      c8[4 * h + 3] = w.x;
-      s8 += w.x + w.y + w.z + w.w;
-    }
-    uint32_t tot;
-    uint32_t run = block_excl_scan<uint32_t>(s8, g.rdx.hcnt, &tot);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      if (run < m && m <= run + c8[i]) sh[0] = static_cast<uint32_t>(kBins - 1 - 8 * tid - i);
-      run += c8[i];
-    }
-  }
+  find_top_bin(h13, kBins, sample_rank<kLowDepth>(K, V), g.rdx.hcnt, &sh[0]);
   lds_barrier();
   const float tau = val_of(max(sh[0] << 19, key_of(-INFINITY)));  // (the bin's least value; bin 0: none found)
   if (!(tau > -INFINITY && tau < INFINITY)) return false;         // (uniform)
@@ -1454,7 +1465,6 @@ __device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, Row<Tin> r
   if (!(mx < INFINITY)) sh[3] = 1;
   lds_barrier();
   const uint32_t n0 = sh[2];
-  const uint32_t K = static_cast<uint32_t>(p.K);
   if (sh[3] || n0 < K || n0 > static_cast<uint32_t>(kLowCap)) return false;  // (uniform)
   // the candidates' ids (and the draft's) into the table: thread t the t-th, the last thread the draft's
   const bool want_draft = p.draft >= 0 && p.draft < V && a.out_dprob;  // (uniform)
