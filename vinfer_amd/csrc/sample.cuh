@@ -1974,6 +1974,9 @@ __device__ __forceinline__ float val16(uint32_t ok) {
 __device__ __forceinline__ uint32_t hcount(const uint32_t* h, uint32_t ok) {
   return (h[ok >> 1] >> ((ok & 1u) << 4)) & 0xFFFFu;
 }
+// The word whose high half counts -0.0 (key 0x7FFF), and its chunk; +0.0's key is the next.
+constexpr uint32_t kNeg0Word = 0x3FFF;
+constexpr int kNeg0Chunk = 512;
 // Chunk c holds keys 65535 - 64c - 63 .. 65535 - 64c; lane l of a chunk walk is key 65535-64c-l.
 __device__ __forceinline__ int chunk_of16(uint32_t ok) { return static_cast<int>((65535u - ok) >> 6); }
 
@@ -2304,8 +2307,8 @@ __device__ __forceinline__ int select_member(const Row<uint16_t>& row, FastSmem&
           if (m0 + k < nm) mark(tid + (m0 + k) * kThreads, q[k]);
       }
     }
-    lds_barrier();  // (the byte stores above land before the word atomics below)
     // the rest: a ragged tail
+    if (nfull * kBlk < V) lds_barrier();  // (uniform; the byte stores above land before the word atomics below)
     if (cand) {
       for (int i = nfull * kBlk + tid; i < V; i += kThreads) {
         const uint32_t raw = base[i];
@@ -2313,7 +2316,7 @@ __device__ __forceinline__ int select_member(const Row<uint16_t>& row, FastSmem&
       }
     }
   }
-  lds_barrier();  // (every bulk mark is in before the corrections)
+  if (ne > 0) lds_barrier();  // (uniform; every bulk mark is in before the corrections)
   // this thread's penalised entries (at e0, e0 + estep, ... in the order of sl): members by
   // their new value, not their original one
   uint32_t e = e0;
@@ -2717,18 +2720,6 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, Row<uint16_t> row,
   const int ne = static_cast<int>(nexc);
   row.nexc = ne;
   lds_barrier();
-  // fold -0.0 (key 0x7FFF, high half of word 0x3FFF) onto +0.0 (key 0x8000, low half of 0x4000)
-  if (tid == 0) {
-    const uint32_t neg0 = hist[0x3FFF] >> 16;
-    const uint32_t pos0 = hist[0x4000] & 0xFFFFu;
-    f.si[1] = 0;
-    if (neg0) {
-      if (pos0 + neg0 > 0xFFFFu) f.si[1] = 1;  // would overflow: generic path
-      hist[0x3FFF] &= 0xFFFFu;
-      hist[0x4000] += neg0;
-    }
-  }
-  lds_barrier();
   // The rest alternates parallel phases (all threads, one barrier each) with decisions taken by
   // wave 0 alone (no workgroup barrier inside), which it publishes in f.plan.
   // ---- 2. [all] per-chunk counts, NaNs, the top chunk, the penalised max ---------------------
@@ -2745,6 +2736,9 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, Row<uint16_t> row,
       cnt = __builtin_amdgcn_udot2(__builtin_bit_cast(ushort2_t, q4.z), ones2(), cnt, false);
       cnt = __builtin_amdgcn_udot2(__builtin_bit_cast(ushort2_t, q4.w), ones2(), cnt, false);
     }
+    // (-0.0 counts as +0.0: wave 0 folds its key onto +0.0's below, before any other read of either)
+    if (tid == kNeg0Chunk) cnt -= hist[kNeg0Word] >> 16;
+    if (tid == kNeg0Chunk - 1) cnt += hist[kNeg0Word] >> 16;
     // NaN keys: all of chunks 0 and 1023 (keys >= 0xFFC0, <= 0x003F), and chunks 1 and 1022
     // but for +inf (0xFF80) and -inf (0x007F)
     if (tid == 0 || tid == 1023) nan = cnt;
@@ -2785,10 +2779,22 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, Row<uint16_t> row,
     const uint32_t nnan = wave_sum<uint32_t>(wq.y);
     const uint32_t cm = dpp::reduce(wq.z, umax);
     const uint32_t em = dpp::reduce(wq.w, umax);
+    // fold -0.0 (the high half of word 0x3FFF) onto +0.0 (the low half of the next): the other waves
+    // read the histogram again only after the next barrier
+    const uint32_t neg0 = hist[kNeg0Word] >> 16;
+    const uint32_t pos0 = hist[kNeg0Word + 1] & 0xFFFFu;
+    if (neg0) {  // (uniform)
+      wave_lds_sync();  // (every lane has read both words)
+      if (l == 0) {
+        hist[kNeg0Word] &= 0xFFFFu;
+        hist[kNeg0Word + 1] += neg0;  // (past 16 bits: the row takes the generic path)
+      }
+      wave_lds_sync();
+    }
     int status = kPlanFast;
     uint32_t mkey = 0;
     float x0 = -INFINITY, mz = 0.0f;
-    if (f.si[1] || total != static_cast<uint32_t>(V - ne)) {
+    if (pos0 + neg0 > 0xFFFFu || total != static_cast<uint32_t>(V - ne)) {
       status = kPlanGeneric;  // a key count past 65535
     } else {
       // the bulk max: the top populated key of the top populated chunk
