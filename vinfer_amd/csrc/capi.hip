@@ -314,9 +314,9 @@ int run_sample(const vsamp_args* a, float* probs, int64_t probs_stride, hipStrea
     s.tile_G = tile_G;
     const dim3 grid(a->batch * (tile_arrive ? tile_G : 1));
     if (pen)
-      hipLaunchKernelGGL((vs::k_sample<Tin, true, false, false, true>), grid, dim3(vs::kThreads), 0, st, s);
+      hipLaunchKernelGGL((vs::k_sample<Tin, true, false, false, true>), grid, dim3(vs::kThreads), 0, st, s, vs::OwnRow{});
     else
-      hipLaunchKernelGGL((vs::k_sample<Tin, false, false, false, true>), grid, dim3(vs::kThreads), 0, st, s);
+      hipLaunchKernelGGL((vs::k_sample<Tin, false, false, false, true>), grid, dim3(vs::kThreads), 0, st, s, vs::OwnRow{});
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? VSAMP_OK : hip_fail(e, "launch k_sample (tile maxima)");
   }
@@ -332,22 +332,22 @@ int run_sample(const vsamp_args* a, float* probs, int64_t probs_stride, hipStrea
     s.epoch = next_epoch();
     s.G = G;
     if (pen)
-      hipLaunchKernelGGL((vs::k_sample<Tin, true, false, true>), dim3(a->batch * G), dim3(vs::kThreads), 0, st, s);
+      hipLaunchKernelGGL((vs::k_sample<Tin, true, false, true>), dim3(a->batch * G), dim3(vs::kThreads), 0, st, s, vs::OwnRow{});
     else
-      hipLaunchKernelGGL((vs::k_sample<Tin, false, false, true>), dim3(a->batch * G), dim3(vs::kThreads), 0, st, s);
+      hipLaunchKernelGGL((vs::k_sample<Tin, false, false, true>), dim3(a->batch * G), dim3(vs::kThreads), 0, st, s, vs::OwnRow{});
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? VSAMP_OK : hip_fail(e, "launch k_sample (split rows)");
   }
   // One launch per step: the penalty phase runs at the start of the same kernel.
   if (state && pen)  // (probabilities)
-    hipLaunchKernelGGL((vs::k_sample<Tin, true, true>), dim3(a->batch), dim3(vs::kThreads), 0, st, s);
+    hipLaunchKernelGGL((vs::k_sample<Tin, true, true>), dim3(a->batch), dim3(vs::kThreads), 0, st, s, vs::OwnRow{});
   else if (state)
     hipLaunchKernelGGL((vs::k_sample<Tin, false, true>),
-                       dim3(skip_every ? a->batch / (skip_every + 1) * skip_every : a->batch), dim3(vs::kThreads), 0, st, s);
+                       dim3(skip_every ? a->batch / (skip_every + 1) * skip_every : a->batch), dim3(vs::kThreads), 0, st, s, vs::OwnRow{});
   else if (pen)
-    hipLaunchKernelGGL((vs::k_sample<Tin, true>), dim3(a->batch), dim3(vs::kThreads), 0, st, s);
+    hipLaunchKernelGGL((vs::k_sample<Tin, true>), dim3(a->batch), dim3(vs::kThreads), 0, st, s, vs::OwnRow{});
   else
-    hipLaunchKernelGGL((vs::k_sample<Tin, false>), dim3(a->batch), dim3(vs::kThreads), 0, st, s);
+    hipLaunchKernelGGL((vs::k_sample<Tin, false>), dim3(a->batch), dim3(vs::kThreads), 0, st, s, vs::OwnRow{});
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? VSAMP_OK : hip_fail(e, "launch k_sample");
 }
@@ -640,10 +640,12 @@ int vsamp_verify(const vsamp_verify_args* v, void* stream) {
   s.param_div = K + 1;
   if (bf) {
     hipLaunchKernelGGL(vs::k_verify_accept<uint16_t>, dim3(1), dim3(vs::kThreads), 0, st, a);
-    hipLaunchKernelGGL(vs::k_verify_finish<uint16_t>, gr, dim3(vs::kThreads), 0, st, a, s);
+    hipLaunchKernelGGL((vs::k_sample<uint16_t, false, false, false, false, vs::VerifyRow>), gr, dim3(vs::kThreads), 0,
+                       st, s, vs::VerifyRow{a});
   } else {
     hipLaunchKernelGGL(vs::k_verify_accept<float>, dim3(1), dim3(vs::kThreads), 0, st, a);
-    hipLaunchKernelGGL(vs::k_verify_finish<float>, gr, dim3(vs::kThreads), 0, st, a, s);
+    hipLaunchKernelGGL((vs::k_sample<float, false, false, false, false, vs::VerifyRow>), gr, dim3(vs::kThreads), 0, st,
+                       s, vs::VerifyRow{a});
   }
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? VSAMP_OK : hip_fail(e, "launch k_verify");

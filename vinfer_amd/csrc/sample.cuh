@@ -3622,15 +3622,42 @@ __device__ __forceinline__ SampleArgs globalized(SampleArgs a) {
   return a;
 }
 
-// Row r by the calling workgroup, its parameter words loaded (pw). `big` is 128 KB: the key
-// histogram (or the generic path's penalty counts), then the id-search / radix scratch. The
-// template parameters are k_sample's.
-template <class Tin, bool PEN, bool STATE, bool SPLIT, bool TILES>
-__device__ __forceinline__ void sample_row(const SampleArgs& a, int r, uint32_t pw, bool fused, uint32_t* big,
-                                           FastSmem& f) {
+// STATE: write each row's RowState (the speculative verify's launches, without PEN, and the
+// probabilities' first launch; with a.out_probs set nothing is drawn).
+// SPLIT: a bf16 split-row launch (grid B * G).
+// TILES: rows (bf16 or fp32) with their tile maxima (a.tile_max): the rows tile_row can decide
+// are decided from a few tiles, the others take the row passes.
+// PICK: which row a workgroup takes (OwnRow: by its place in the grid).
+struct OwnRow {
+  static constexpr bool kOwn = true;
+};
+template <class Tin, bool PEN, bool STATE = false, bool SPLIT = false, bool TILES = false, class PICK = OwnRow>
+__global__ __launch_bounds__(kThreads) void k_sample(SampleArgs a_, PICK pick) {
+  const SampleArgs a = globalized(a_);
+  // 128 KB: the key histogram (or the generic path's penalty counts), then the id-search /
+  // radix scratch
+  __shared__ __align__(16) uint32_t big[kChunk];
+  __shared__ FastSmem f;
   static_assert(sizeof(GenericSmem) <= sizeof(uint32_t) * kBitmapOffset, "scratch must fit below the bitmap");
   static_assert(kMatchOffset + kMatchWords <= kChunk, "count cells must fit");
+  const bool fused = TILES && a.tile_arrive != nullptr;  // (uniform)
   const int tid = threadIdx.x;
+  exp_table_init();  // (published by the first barrier of either path)
+  int r;
+  if constexpr (PICK::kOwn) {
+    r = SPLIT ? row_index(a)
+        : fused ? static_cast<int>(blockIdx.x) / a.tile_G
+        : STATE ? state_row_index(a)
+                : static_cast<int>(blockIdx.x);
+  } else {
+    r = pick.template row<Tin>(big, f);
+    if (r < 0) return;  // (uniform)
+  }
+  // the row's parameters: thread w < kParamWords loads word w, the others word 0 (every thread
+  // loads: a load on one branch only would make later waits wait for every load in flight)
+  const uint32_t pw = param_word<PEN, STATE || !PICK::kOwn>(a, r, tid < kParamWords ? tid : 0);
+  __builtin_amdgcn_sched_barrier(0);  // (issued before the row's first loads)
+
   Row<Tin> row;
   row.p = static_cast<const Tin*>(a.logits) + static_cast<int64_t>(r) * a.stride;
   row.V = a.V;
@@ -3690,30 +3717,6 @@ __device__ __forceinline__ void sample_row(const SampleArgs& a, int r, uint32_t 
     row.eval = a.ws.exc_val + p.h0;
   }
   generic_row<STATE>(a, row, p, g, f, r, have_bitmap);
-}
-
-// STATE: write each row's RowState (the speculative verify's launches, without PEN, and the
-// probabilities' first launch; with a.out_probs set nothing is drawn).
-// SPLIT: a bf16 split-row launch (grid B * G).
-// TILES: rows (bf16 or fp32) with their tile maxima (a.tile_max): the rows tile_row can decide
-// are decided from a few tiles, the others take the row passes.
-template <class Tin, bool PEN, bool STATE = false, bool SPLIT = false, bool TILES = false>
-__global__ __launch_bounds__(kThreads) void k_sample(SampleArgs a_) {
-  const SampleArgs a = globalized(a_);
-  __shared__ __align__(16) uint32_t big[kChunk];
-  __shared__ FastSmem f;
-  const bool fused = TILES && a.tile_arrive != nullptr;  // (uniform)
-  const int r = SPLIT ? row_index(a)
-                : fused ? static_cast<int>(blockIdx.x) / a.tile_G
-                : STATE ? state_row_index(a)
-                        : static_cast<int>(blockIdx.x);
-  const int tid = threadIdx.x;
-  exp_table_init();  // (published by the first barrier of either path)
-  // the row's parameters: thread w < kParamWords loads word w, the others word 0 (every thread
-  // loads: a load on one branch only would make later waits wait for every load in flight)
-  const uint32_t pw = param_word<PEN, STATE>(a, r, tid < kParamWords ? tid : 0);
-  __builtin_amdgcn_sched_barrier(0);  // (issued before the row's first loads)
-  sample_row<Tin, PEN, STATE, SPLIT, TILES>(a, r, pw, fused, big, f);
 }
 
 }  // namespace vs

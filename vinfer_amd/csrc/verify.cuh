@@ -128,7 +128,7 @@ struct ResidualSide {
 
 // One workgroup, a thread per sequence: the acceptance chain. Writes the accepted drafts and, when
 // all are accepted, the count; leaves the first rejected position in jr, clears the row's slice
-// counter and lists the rejected and the accepted sequences (ascending) for k_verify_finish.
+// counter and lists the rejected and the accepted sequences (ascending) for the last launch.
 template <class Tin>
 __global__ __launch_bounds__(kThreads) void k_verify_accept(VerifyArgs a) {
   __shared__ uint32_t red[kWaves];
@@ -156,7 +156,7 @@ __global__ __launch_bounds__(kThreads) void k_verify_accept(VerifyArgs a) {
       }
       int32_t* out = a.out_tokens + static_cast<int64_t>(b) * (K + 1);
       for (int i = 0; i <= K; ++i) out[i] = i < j ? a.drafts[b * K + i] : -1;
-      if (j == K) a.out_count[b] = K + 1;  // (k_verify_finish draws the bonus token)
+      if (j == K) a.out_count[b] = K + 1;  // (the last launch draws the bonus token)
       a.jr[b] = j;
       a.done[b] = 0;
     }
@@ -537,38 +537,33 @@ __device__ __forceinline__ bool residual_item(const VerifyArgs& a, int b, int sl
   return residual(std::false_type{});
 }
 
-// The bonus rows of the accepted sequences (k_sample's row code, one workgroup a row) and the
-// residual draws of the rejected ones, (row, slice) items row-major over their list, one item a
-// workgroup: the grid is the larger of B and the CUs the items can use (the LDS holds one
-// workgroup a CU), and the slices are chosen to fit it. (No loop over the items: with one the
-// compiler kept both kinds' values live across it and spilled, 640 bytes a lane, 72-78 us.)
-// `s_` describes the target rows, its out_ids the emitted tokens: row (b, j)'s draw is token (b, j).
-template <class Tin>
-__global__ __launch_bounds__(kThreads) void k_verify_finish(VerifyArgs a, SampleArgs s_) {
-  __shared__ __align__(16) uint32_t big[kChunk];
-  __shared__ FastSmem f;
-  exp_table_init();
-  const int nrej = *a.nrej;
-  const int nacc = a.B - nrej;
-  const int item = blockIdx.x;
-  int r;  // (uniform) the target row to draw from
-  if (item < nacc) {
-    r = a.acc[item] * (a.K + 1) + a.K;
-  } else {
+// The last launch's rows: the bonus rows of the accepted sequences (k_sample's row code, one
+// workgroup a row) and the residual draws of the rejected ones, (row, slice) items row-major over
+// their list, one item a workgroup: the grid is the larger of B and the CUs the items can use (the
+// LDS holds one workgroup a CU), and the slices are chosen to fit it. (No loop over the items: with
+// one the compiler kept both kinds' values live across it and spilled, 640 bytes a lane, 72-78 us.)
+// The launch's SampleArgs describe the target rows, its out_ids the emitted tokens: row (b, j)'s
+// draw is token (b, j).
+struct VerifyRow {
+  static constexpr bool kOwn = false;
+  VerifyArgs a;
+  // The target row this workgroup draws from: a bonus row, or a rejected one without residual mass
+  // (after its residual); -1: none.
+  template <class Tin>
+  __device__ __forceinline__ int row(uint32_t* big, FastSmem& f) const {
+    const int nrej = *a.nrej;
+    const int nacc = a.B - nrej;
+    const int item = blockIdx.x;
+    if (item < nacc) return a.acc[item] * (a.K + 1) + a.K;
     const int slices = residual_slices(nrej, static_cast<int>(gridDim.x) - nacc, a.max_slices);
     const int q = item - nacc;
-    if (q >= nrej * slices) return;
+    if (q >= nrej * slices) return -1;
     const int b = a.rej[q / slices];
     __syncthreads();  // (publishes the exp table)
-    if (!residual_item<Tin>(a, b, q % slices, slices, big, *reinterpret_cast<ResidualSmem*>(&f))) return;  // (uniform)
-    r = b * (a.K + 1) + a.jr[b];
+    if (!residual_item<Tin>(a, b, q % slices, slices, big, *reinterpret_cast<ResidualSmem*>(&f))) return -1;  // (uniform)
     __syncthreads();  // (the residual's LDS is free)
+    return b * (a.K + 1) + a.jr[b];
   }
-  const SampleArgs s = globalized(s_);
-  const int tid = threadIdx.x;
-  const uint32_t pw = param_word<false, true>(s, r, tid < kParamWords ? tid : 0);
-  __builtin_amdgcn_sched_barrier(0);  // (issued before the row's first loads)
-  sample_row<Tin, false, false, false, false>(s, r, pw, false, big, f);
-}
+};
 
 }  // namespace vs
