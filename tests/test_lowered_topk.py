@@ -77,3 +77,33 @@ def test_lowered_top_k_rows_match_the_oracle(V, dtype):
         _, bad = compare_ids(got, oracle(w), dp)
         assert not bad, (tiles, bad[:8])
     s.tile_pass = True
+
+
+@pytest.mark.parametrize("V", [16384, 20011])
+def test_more_fp32_rows_than_cus_equal_smaller_batches(V):
+    # above one row a CU the candidates' rows and the others take a launch each; the same rows in
+    # batches of 200 take the one launch
+    s = SAMPLER.resolve("hip", BackendContext(DEV, torch.float32))
+    cus = torch.cuda.get_device_properties(DEV).multi_processor_count
+    g = torch.Generator(device=DEV).manual_seed(V)
+    rng = np.random.default_rng(V)
+    for B in (cus, cus + 1, 2 * cus + 5):
+        x = torch.randn(B, V, generator=g, device=DEV) * 2.5
+        x[5, V - 1] = math.nan
+        rows = [SamplingParams(temperature=(0.8, 0.0, 1.1)[b % 3], top_k=(50, 20, 0, 192, 400)[b % 5], top_p=0.9,
+                               repetition_penalty=(1.1, 0.95)[b % 7 == 0], presence_penalty=0.3, frequency_penalty=0.1)
+                for b in range(B)]
+        hist = [rng.integers(0, V, int(rng.integers(0, 400))).tolist() for _ in range(B)]
+        u = torch.rand(B, generator=g, device=DEV)
+        draft = torch.randint(0, V, (B,), generator=g, device=DEV).to(torch.int32)
+        print(f"fp32 rows past the CUs B={B} V={V}", flush=True)
+
+        def run(lo, hi):
+            ids, off = pack_history(hist[lo:hi], DEV)
+            return s.sample_batch(x[lo:hi], pack_params(rows[lo:hi]).to(DEV), u[lo:hi], ids, off, draft[lo:hi])
+
+        got = run(0, B)
+        parts = [run(lo, min(B, lo + 200)) for lo in range(0, B, 200)]
+        torch.cuda.synchronize()
+        assert torch.equal(got[0], torch.cat([p[0] for p in parts]))
+        assert torch.equal(got[1], torch.cat([p[1] for p in parts]))

@@ -1358,11 +1358,13 @@ __device__ __forceinline__ void find_top_bin(const uint32_t* h13, int bins, uint
 // m three times the K-th's share of that sample (penalised candidates may fall below tau).
 // Returns false, with nothing written, for a row it does not decide (too few or too many
 // candidates, a NaN or +inf, a threshold below tau): the caller runs the penalty pass.
-// Measured (1024 fp32 rows of 151936, top-k 50, histories up to 32768): 255.0 -> 160.7 us a launch.
+// Measured (1024 fp32 rows of 151936, top-k 50, histories up to 32768): 255.0 -> 160.7 us in one
+// launch, 136.6 with two workgroups a CU (k_lowered).
 constexpr int kLowK = 192;       // top-k served
 constexpr int kLowDepth = 2;     // stripes sampled
 constexpr int kLowCap = 1023;    // staged candidates: one a thread, and one for the draft id
 constexpr int kLowSlots = 4096;  // hash table
+constexpr int kLowWords = kBitmapOffset + 8192 + 2 * 1024;  // LDS words from the scratch's start: 60 KB
 
 // Sorts c[0, n), n <= kThreads, into out[0, min(n, kSortCap)): descending value, ascending id (each
 // entry's rank is the count of larger keys). `kk` holds n staged keys; the result is visible on
@@ -1398,16 +1400,15 @@ __device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, Row<Tin> r
   if (p.rep == 1.0f && p.pres == 0.0f && p.freq == 0.0f) return false;  // (no penalties: the generic path's own stream)
   if (V / kBlk / kThreads < kLowDepth) return false;
   const uint32_t K = static_cast<uint32_t>(p.K);
-  uint32_t* const area = reinterpret_cast<uint32_t*>(&g);
-  uint32_t* const hkey = area + kBitmapOffset;      // the hash table's ids
-  uint32_t* const hcnt = hkey + kLowSlots;          // and counts
-  uint32_t* const h13 = area + kMatchOffset;        // the sample's bins, then:
+  uint32_t* const h13 = reinterpret_cast<uint32_t*>(&g) + kBitmapOffset;  // the sample's bins, then:
+  uint32_t* const hkey = h13;                       // the hash table's ids
+  uint32_t* const hcnt = hkey + kLowSlots;          // and counts, then:
   Cand* const cand = reinterpret_cast<Cand*>(h13);  // the penalised candidates,
   u64* const kk = reinterpret_cast<u64*>(h13 + 2048);       // their sort keys
   Cand* const srt = reinterpret_cast<Cand*>(h13 + 4096);    // and the sorted list
   constexpr int kBins = 8192;
   Cand* const stage = reinterpret_cast<Cand*>(h13 + kBins);
-  static_assert(kMatchOffset + kBins + 2 * (kLowCap + 1) <= kChunk && 2 * kLowSlots <= kMatchOffset - kBitmapOffset &&
+  static_assert(kBitmapOffset + kBins + 2 * (kLowCap + 1) <= kLowWords && 2 * kLowSlots <= kBins &&
                     4096 + 2 * kSortCap <= kBins && kLowCap < kThreads,
                 "the row's LDS areas");
   uint32_t* const sh = g.rdx.bk;  // [0] the bin, [1] above it, [2] candidates, [3] a NaN or +inf
@@ -1415,10 +1416,6 @@ __device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, Row<Tin> r
 #pragma unroll
   for (int k = 0; k < kLowDepth; ++k) q[k].load(row.p, k * kThreads + tid);
   for (int i = tid; i < kBins / 4; i += kThreads) reinterpret_cast<uint4*>(h13)[i] = make_uint4(0, 0, 0, 0);
-  for (int i = tid; i < kLowSlots / 4; i += kThreads) {
-    reinterpret_cast<uint4*>(hkey)[i] = make_uint4(kEmpty, kEmpty, kEmpty, kEmpty);
-    reinterpret_cast<uint4*>(hcnt)[i] = make_uint4(0, 0, 0, 0);
-  }
   if (tid < 4) sh[tid] = 0;
   lds_barrier();
   float v[kLowDepth][kBlk];
@@ -1434,6 +1431,10 @@ __device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, Row<Tin> r
   lds_barrier();
   const float tau = val_of(max(sh[0] << 19, key_of(-INFINITY)));  // (the bin's least value; bin 0: none found)
   if (!(tau > -INFINITY && tau < INFINITY)) return false;         // (uniform)
+  for (int i = tid; i < kLowSlots / 4; i += kThreads) {  // (the bins are dead; published after the pass)
+    reinterpret_cast<uint4*>(hkey)[i] = make_uint4(kEmpty, kEmpty, kEmpty, kEmpty);
+    reinterpret_cast<uint4*>(hcnt)[i] = make_uint4(0, 0, 0, 0);
+  }
   auto append = [&](float x, int id) {
     const bool c = x >= tau;
     const u64 bal = __ballot(c);  // (one counter update per wave round)
@@ -1502,6 +1503,7 @@ __device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, Row<Tin> r
   int32_t* const xid = reinterpret_cast<int32_t*>(g.rdx.hcnt) + 64;  // (past sorted_tail's results)
   float* const xval = reinterpret_cast<float*>(xid + 1);
   const int c = mine || drafts ? static_cast<int>(hcnt[slot]) : 0;
+  lds_barrier();  // (every thread has its count: the candidates go over the table)
   const float xp = c > 0 ? apply_penalty(me.x, c, p.rep, p.pres, p.freq) : me.x;
   if (drafts) {
     xid[0] = p.draft;
@@ -3702,7 +3704,7 @@ __global__ __launch_bounds__(kThreads) void k_sample(SampleArgs a_, PICK pick) {
   }
   RowParams p = f.prm;
   p.u = p.u >= 0.0f ? p.u : 0.0f;
-  if constexpr (PEN && !STATE && sizeof(Tin) == 4) {
+  if constexpr (PEN && !STATE && sizeof(Tin) == 4 && PICK::kOwn) {
     if (lowered_topk_row<Tin>(a, row, p, g, r)) return;
     lds_barrier();  // (every thread is done with its LDS)
   }
@@ -3718,5 +3720,47 @@ __global__ __launch_bounds__(kThreads) void k_sample(SampleArgs a_, PICK pick) {
   }
   generic_row<STATE>(a, row, p, g, f, r, have_bitmap);
 }
+
+// ---- fp32 batches of more rows than CUs, with penalties ------------------------------------------
+// lowered_topk_row alone, two workgroups a CU (60 KB of LDS, at most 64 VGPRs), so that one row's
+// decisions run while the other's row streams; k_sample holds one (160 KB). A row it decides is
+// marked in the workspace's n_exc, and k_sample with UndecidedRow takes the others in a launch after
+// it. Measured (1024 rows of 151936, top-k 50, histories up to 32768): 161.0 us in the one launch,
+// 136.6 in the two (131-135 and 4); 512 rows none of which it decides (top-k 1000): 261.0 and 262.2.
+constexpr uint32_t kRowDecided = 0xFFFFFFFFu;
+template <class Tin>
+__global__ __launch_bounds__(kThreads, 8) void k_lowered(SampleArgs a_) {
+  const SampleArgs a = globalized(a_);
+  __shared__ __align__(16) uint32_t mem[kLowWords];
+  __shared__ RowParams prm;
+  exp_table_init();
+  const int r = blockIdx.x;
+  const int tid = threadIdx.x;
+  const uint32_t pw = param_word<true>(a, r, tid < kParamWords ? tid : 0);
+  if (tid < kParamWords) reinterpret_cast<uint32_t*>(&prm)[tid] = pw;
+  lds_barrier();
+  RowParams p = prm;
+  p.u = p.u >= 0.0f ? p.u : 0.0f;
+  Row<Tin> row;
+  row.p = static_cast<const Tin*>(a.logits) + static_cast<int64_t>(r) * a.stride;
+  row.V = a.V;
+  row.nblk = (a.V + kBlk - 1) / kBlk;
+  row.nstripes = (row.nblk + kThreads - 1) / kThreads;
+  row.bm = nullptr;
+  row.eid = nullptr;
+  row.eval = nullptr;
+  row.nexc = 0;
+  const bool done = lowered_topk_row<Tin>(a, row, p, *reinterpret_cast<GenericSmem*>(mem), r);  // (uniform)
+  if (tid == 0) a.ws.n_exc[r] = done ? kRowDecided : 0u;
+}
+struct UndecidedRow {
+  static constexpr bool kOwn = false;
+  const uint32_t* marks;
+  template <class Tin>
+  __device__ __forceinline__ int row(uint32_t*, FastSmem&) const {
+    const int r = static_cast<int>(blockIdx.x);
+    return ld_global(marks + r) == kRowDecided ? -1 : r;
+  }
+};
 
 }  // namespace vs
