@@ -24,7 +24,7 @@
 // drafted positions' rows are not drawn from (but in the rare row without residual mass), and the
 // bonus rows and the residuals share one launch: 192 sequences of one draft, V = 262144, 137.4 us
 // a call when every target row was sampled first (384 rows, one and a half rounds on 256 CUs) and
-// the residuals took a launch of their own, 91 us now.
+// the residuals took a launch of their own, 89 us now.
 // A bf16 row holds at most 65536 distinct values, and its kept ones sit in a short run of keys
 // below the row's max: the two terms of w are tabulated per key in LDS for the top kTab keys
 // of each row (a kept token below that run is computed directly), so the residual pass costs
