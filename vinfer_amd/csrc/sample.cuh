@@ -1411,7 +1411,9 @@ __device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, Row<Tin> r
   static_assert(kBitmapOffset + kBins + 2 * (kLowCap + 1) <= kLowWords && 2 * kLowSlots <= kBins &&
                     4096 + 2 * kSortCap <= kBins && kLowCap < kThreads,
                 "the row's LDS areas");
-  uint32_t* const sh = g.rdx.bk;  // [0] the bin, [1] above it, [2] candidates, [3] a NaN or +inf
+  // [0] the bin, [1] penalised candidates, [2] candidates, [3] a NaN or +inf, then the threshold (a word of
+  // its own for each count: every thread decides by [2], so nothing may reset it before they all have)
+  uint32_t* const sh = g.rdx.bk;
   WholeBlock<Tin> q[kLowDepth];
 #pragma unroll
   for (int k = 0; k < kLowDepth; ++k) q[k].load(row.p, k * kThreads + tid);
@@ -1484,7 +1486,6 @@ __device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, Row<Tin> r
       slot = (slot + 1) & (kLowSlots - 1);
     }
   }
-  if (tid == 0) sh[2] = 0;
   lds_barrier();
   for_each_id(a.pen.hist + p.h0, L, [&](int id, int) {
     uint32_t h = (static_cast<uint32_t>(id) * 2654435761u) >> (32 - 12);
@@ -1515,13 +1516,13 @@ __device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, Row<Tin> r
     if (bal) {
       const int leader = __ffsll(static_cast<long long>(bal)) - 1;
       uint32_t at = 0;
-      if (lane_id() == leader) at = atomicAdd(&sh[2], static_cast<uint32_t>(__popcll(bal)));
+      if (lane_id() == leader) at = atomicAdd(&sh[1], static_cast<uint32_t>(__popcll(bal)));
       at = __builtin_amdgcn_readlane(at, leader) + lanes_below(bal);
       if (in) cand[at] = Cand{xp, me.id};
     }
   }
   lds_barrier();
-  const int n = static_cast<int>(sh[2]);
+  const int n = static_cast<int>(sh[1]);
   if (n < p.K) return false;  // (uniform)
   sort_top(cand, n, kk, srt);
   const float T = p.T;
