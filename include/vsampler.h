@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define VSAMP_ABI_VERSION 11
+#define VSAMP_ABI_VERSION 12
 
 /* Bytes of one row's sampling state (vsamp_sample_states), an opaque record. */
 #define VSAMP_ROW_STATE_BYTES 40
@@ -134,7 +134,7 @@ size_t vsamp_split_workspace_bytes(int32_t batch, int32_t vocab, int64_t hist_to
 
 /* Workspace bytes of a vsamp_probs call that writes its rows over the whole chip (the rows' states
  * after the penalty part); a call with less (vsamp_workspace_bytes()) writes each row from one
- * workgroup, with the same results. No counterpart in the engine. */
+ * workgroup, with the same results. (ABI version 12; no counterpart in the engine.) */
 size_t vsamp_probs_workspace_bytes(int32_t batch, int32_t vocab, int64_t hist_total);
 
 /* Sample one token per row: penalties, temperature, top-k, softmax, min-p, top-p, then the

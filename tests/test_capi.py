@@ -35,6 +35,12 @@ def test_abi_version_is_one_number_everywhere():
     assert header == _lib.ABI_VERSION == snippet
 
 
+def test_a_changed_surface_has_a_new_abi_version():
+    # a library of an earlier version must fail on its number, not on a symbol that it lacks: whoever adds an
+    # entry point changes this pair, both numbers of it
+    assert (_lib.ABI_VERSION, len(declared())) == (12, 22)
+
+
 def test_every_declared_symbol_is_exported():
     names = declared()
     assert names == sorted(_lib.EXPORTS)
