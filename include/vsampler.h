@@ -51,6 +51,13 @@ extern "C" {
  * counterpart: for callers that keep per-row histories on the device (a batched decode loop).
  * Needs penalties on (a history and a penalty column). */
 #define VSAMP_HIST_APPEND 4u
+/* Row states in the workspace (vsamp_probs only; ABI version 12): the call may keep its rows' states
+ * there between two launches, so that it writes the rows over the whole chip, when the workspace holds
+ * vsamp_probs_workspace_bytes(). The workspace is then in use until the call's work is done, with or
+ * without histories: calls that overlap each need their own. Without it a call that applies no
+ * penalties leaves the workspace alone, and one workgroup writes each row. The results are identical
+ * either way. No reference counterpart. */
+#define VSAMP_PROBS_STATES 8u
 
 enum vsamp_dtype { VSAMP_BF16 = 0, VSAMP_F32 = 1 };
 
@@ -112,7 +119,7 @@ typedef struct vsamp_args {
   void* workspace;
   size_t workspace_bytes;
 
-  uint32_t flags; /* VSAMP_HIST_RANGES, VSAMP_SPLIT_ROWS, VSAMP_HIST_APPEND, or 0 */
+  uint32_t flags; /* VSAMP_HIST_RANGES, VSAMP_SPLIT_ROWS, VSAMP_HIST_APPEND, VSAMP_PROBS_STATES, or 0 */
   uint32_t reserved1;
 } vsamp_args;
 
@@ -132,8 +139,8 @@ size_t vsamp_workspace_bytes(int32_t batch, int32_t vocab, int64_t hist_total);
  * need no clearing: each launch tags them. No counterpart in the engine. */
 size_t vsamp_split_workspace_bytes(int32_t batch, int32_t vocab, int64_t hist_total);
 
-/* Workspace bytes of a vsamp_probs call that writes its rows over the whole chip (the rows' states
- * after the penalty part); a call with less (vsamp_workspace_bytes()) writes each row from one
+/* Workspace bytes of a vsamp_probs call with VSAMP_PROBS_STATES (the rows' states after the penalty
+ * part); a call with less (vsamp_workspace_bytes()) writes each row from one
  * workgroup, with the same results. (ABI version 12; no counterpart in the engine.) */
 size_t vsamp_probs_workspace_bytes(int32_t batch, int32_t vocab, int64_t hist_total);
 

@@ -115,6 +115,16 @@ def test_bad_arguments_are_rejected_with_their_code(kw, code, msg):
         _lib.check(rc)
 
 
+def test_the_row_states_flag_goes_with_the_probabilities_alone():
+    lib = _lib.load()
+    a = _args(flags=_lib.VSAMP_PROBS_STATES, batch=0)
+    assert lib.vsamp_probs(ctypes.byref(a), 0x6000, 100, None) == 0
+    assert lib.vsamp_penalized_logits(ctypes.byref(a), 0x6000, None, 100, None) == 1
+    assert lib.vsamp_sample(ctypes.byref(a), None) == 1
+    a.flags = 16
+    assert lib.vsamp_probs(ctypes.byref(a), 0x6000, 100, None) == 1
+
+
 def test_empty_batch_is_a_no_op():
     lib = _lib.load()
     assert lib.vsamp_sample(ctypes.byref(_args(batch=0)), None) == 0

@@ -63,3 +63,30 @@ def test_two_launches_equal_one(V, offset, dtype, pen):
     rows = [(r, int((got[r] != want[r]).sum()), got[r][got[r] != want[r]][:3].tolist(), want[r][got[r] != want[r]][:3].tolist())
             for r in range(B) if not torch.equal(got[r], want[r])]
     assert not rows, rows
+
+
+@pytest.mark.parametrize("pen", [False, True], ids=["plain", "penalties"])
+def test_a_workspace_is_used_past_the_penalties_only_when_given_for_it(pen):
+    # (without the flag, calls that apply no penalties may share one workspace on several streams)
+    s = SAMPLER.resolve("hip", BackendContext(DEV, torch.float32))
+    B, V = 5, 20000
+    g = torch.Generator(device=DEV).manual_seed(3)
+    logits = torch.randn(B, V, generator=g, device=DEV) * 3.0
+    f = lambda v: torch.full((B,), v, device=DEV)  # noqa: E731
+    params = PackedParams(temperature=f(0.8), top_k=torch.zeros(B, dtype=torch.int32, device=DEV), top_p=f(0.9), min_p=f(0.0),
+                          repetition_penalty=f(1.1), presence_penalty=f(0.5), frequency_penalty=f(0.2))
+    ids = torch.randint(0, V, (50 * B,), generator=g, device=DEV).to(torch.int32) if pen else None
+    off = torch.arange(0, 50 * B + 1, 50, dtype=torch.int32, device=DEV) if pen else None
+    want = one_launch(s, logits, params, ids, off)
+    for flag in (0, _lib.VSAMP_PROBS_STATES):
+        a, keep = s._args(logits, params, ids, off)
+        need = int(s._lib.vsamp_probs_workspace_bytes(B, V, a.hist_total))
+        kept = int(s._lib.vsamp_workspace_bytes(B, V, a.hist_total)) if pen else 0
+        ws = torch.full((need + 512,), 0xA5, dtype=torch.uint8, device=DEV)
+        at = (ws.data_ptr() + 255 & ~255) - ws.data_ptr()
+        a.workspace, a.workspace_bytes, a.flags = ws.data_ptr() + at, need, a.flags | flag
+        out = torch.empty(B, V, device=DEV)
+        _lib.check(s._lib.vsamp_probs(ctypes.byref(a), out.data_ptr(), V, s._stream(DEV)))
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        assert bool((ws[at + kept:at + need] == 0xA5).all()) == (flag == 0)

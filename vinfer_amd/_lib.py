@@ -19,6 +19,7 @@ VSAMP_F32 = 1
 VSAMP_HIST_RANGES = 1
 VSAMP_SPLIT_ROWS = 2
 VSAMP_HIST_APPEND = 4
+VSAMP_PROBS_STATES = 8
 
 STATUS = {0: "ok", 1: "VSAMP_E_ARG", 2: "VSAMP_E_DTYPE", 3: "VSAMP_E_HIP", 4: "VSAMP_E_WORKSPACE", 5: "VSAMP_E_DEVICE"}
 

@@ -180,9 +180,10 @@ int scratch_of_current_device(void** out) {
 
 bool wants_penalties(const vsamp_args* a);
 
-int validate(const vsamp_args* a, bool need_draw) {
+// extra: a flags bit that this call takes besides the common ones.
+int validate(const vsamp_args* a, bool need_draw, uint32_t extra = 0) {
   if (!a) return fail(VSAMP_E_ARG, "args is NULL");
-  if (a->flags & ~(VSAMP_HIST_RANGES | VSAMP_SPLIT_ROWS | VSAMP_HIST_APPEND))
+  if (a->flags & ~extra & ~(VSAMP_HIST_RANGES | VSAMP_SPLIT_ROWS | VSAMP_HIST_APPEND))
     return fail(VSAMP_E_ARG,
                 "flags must be a combination of VSAMP_HIST_RANGES, VSAMP_SPLIT_ROWS and VSAMP_HIST_APPEND, got %u",
                 a->flags);
@@ -381,12 +382,13 @@ size_t probs_total(int64_t B, int64_t V, int64_t H) {
   return probs_states(B, V, H) + sizeof(vs::RowState) * static_cast<size_t>(B);
 }
 
-// Probabilities: with a workspace that holds the row states, the states' launch and a launch that
-// writes the rows over the whole chip (32 bf16 rows of 151936: 104.8 -> 32.3 us); otherwise one
+// Probabilities: where the caller gives a workspace for the row states (VSAMP_PROBS_STATES: a call
+// without histories may otherwise share its workspace with others), the states' launch and a launch
+// that writes the rows over the whole chip (32 bf16 rows of 151936: 104.8 -> 32.3 us); otherwise one
 // launch, each row written by its own workgroup.
 template <class Tin>
 int run_probs(const vsamp_args* a, float* out, int64_t out_stride, hipStream_t st) {
-  if (!a->workspace || (reinterpret_cast<uintptr_t>(a->workspace) & 255u) ||
+  if (!(a->flags & VSAMP_PROBS_STATES) || !a->workspace || (reinterpret_cast<uintptr_t>(a->workspace) & 255u) ||
       a->workspace_bytes < probs_total(a->batch, a->vocab, a->hist_total) || a->batch > 65535)
     return run_sample<Tin>(a, out, out_stride, st);
   char* w = static_cast<char*>(a->workspace);
@@ -515,7 +517,7 @@ int vsamp_sample_noalloc(const vsamp_args* a, void* stream) {
 
 int vsamp_probs(const vsamp_args* a, float* out, int64_t out_stride, void* stream) {
   g_err.clear();
-  if (int rc = validate(a, false)) return rc;
+  if (int rc = validate(a, false, VSAMP_PROBS_STATES)) return rc;
   if (a->batch == 0) return VSAMP_OK;
   if (!out) return fail(VSAMP_E_ARG, "out is NULL");
   if (out_stride < a->vocab) return fail(VSAMP_E_ARG, "out_stride must be >= vocab");

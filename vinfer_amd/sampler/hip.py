@@ -212,6 +212,7 @@ class HipSampler:
         B, V = logits.shape
         out = torch.empty(B, V, dtype=torch.float32, device=logits.device)
         # (the call's own workspace: the rows' states live in it between its two launches)
+        a.flags |= _lib.VSAMP_PROBS_STATES
         a.workspace_bytes = int(self._lib.vsamp_probs_workspace_bytes(B, V, a.hist_total))
         ws = torch.empty(a.workspace_bytes + 256, dtype=torch.uint8, device=logits.device)
         a.workspace = (ws.data_ptr() + 255) & ~255
