@@ -11,11 +11,14 @@ always rejected, and the replacement is then p's own inverse-CDF draw over ascen
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 from oracle.sampler_oracle import sample_row, token_masses, verify_row
+from vinfer_amd import _lib
 from vinfer_amd.registry import BackendContext
 from vinfer_amd.sampler import SAMPLER
 from vinfer_amd.sampling import SamplingParams, pack_params
@@ -304,12 +307,13 @@ def test_gpu_verify_residual_over_signed_zeros(dtype):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=str)
-@pytest.mark.parametrize("B,K,V", [(1, 1, 7), (3, 2, 4099), (40, 3, 8195), (300, 1, 2048)])
+@pytest.mark.parametrize("B,K,V", [(1, 1, 7), (3, 2, 4099), (40, 3, 8195), (300, 1, 2048), (64, 3, 2049), (65, 3, 2049), (3, 64, 520), (16, 4, 140000),
+                                   (128, 1, 40000)])
 def test_gpu_rows_without_residual_mass_take_the_targets_draw(dtype, B, K, V):
     # the draft's logits are the target's: a rejected draft (outside the vocabulary, at a position of its
     # own for every sequence) leaves no residual, so the target's own draw at that position is emitted, and
     # sequences without one get the bonus draw; both are those of a batched draw from the same row (300
-    # sequences: more rows than CUs)
+    # sequences, 65 of 3: more rows than CUs; 64 of 3: one row a CU)
     dev = torch.device("cuda", 0)
     s = SAMPLER.resolve("hip", BackendContext(dev, dtype))
     g = torch.Generator(device=dev).manual_seed(B * K + V)
@@ -328,3 +332,36 @@ def test_gpu_rows_without_residual_mass_take_the_targets_draw(dtype, B, K, V):
     assert torch.equal(counts.long(), first + 1)
     keep = torch.arange(K + 1, device=dev)[None, :] <= first[:, None]
     assert torch.equal(tokens, torch.where(keep, draws, -1).to(torch.int32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("past", [0, 1], ids=["one round", "more rows"])
+def test_gpu_bonus_rows_join_the_first_launch_while_the_rows_fit_the_cus(past):
+    # (an accepted sequence is then done after it; in more rounds only the accepted ones' are drawn from, last)
+    dev = torch.device("cuda", 0)
+    s = SAMPLER.resolve("hip", BackendContext(dev, torch.bfloat16))
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    K, V = 3, 1024
+    B = cus // (K + 1) + past
+    g = torch.Generator(device=dev).manual_seed(past)
+    target = (torch.randn(B * (K + 1), V, generator=g, device=dev) * 2).to(torch.bfloat16)
+    params = pack_params([SamplingParams(temperature=0.9)] * B).to(dev)
+    ta, keep = s._args(target, params, None, None, torch.rand(B, generator=g, device=dev), param_rows=B)
+    da, keep2 = s._args(target[:B * K], params, None, None, None, param_rows=B)
+    need = int(s._lib.vsamp_verify_workspace_bytes(B, K))
+    ws = torch.full((need + 256,), 0xA5, dtype=torch.uint8, device=dev)
+    at = (ws.data_ptr() + 255 & ~255) - ws.data_ptr()
+    v = _lib.VsampVerifyArgs()
+    v.target, v.draft, v.batch, v.num_draft = ta, da, B, K
+    drafts = torch.zeros(B, K, dtype=torch.int32, device=dev)
+    u = torch.rand(2, B, K, generator=g, device=dev)
+    tokens, counts = (torch.empty(n, dtype=torch.int32, device=dev) for n in (B * (K + 1), B))
+    v.draft_tokens, v.u_accept, v.u_residual = drafts.data_ptr(), u[0].data_ptr(), u[1].data_ptr()
+    v.out_tokens, v.out_count = tokens.data_ptr(), counts.data_ptr()
+    v.workspace, v.workspace_bytes = ws.data_ptr() + at, need
+    _lib.check(s._lib.vsamp_verify(ctypes.byref(v), s._stream(dev)))
+    torch.cuda.synchronize()
+    # the workspace opens with the target rows' states
+    states = ws[at:at + B * (K + 1) * _lib.ROW_STATE_BYTES].view(B, K + 1, _lib.ROW_STATE_BYTES)
+    assert not (states[:, :K] == 0xA5).all(dim=2).any()
+    assert bool((states[:, K] == 0xA5).all()) == bool(past)

@@ -283,11 +283,12 @@ vs::SampleArgs sample_args(const vsamp_args* a) {
 }
 
 // state: the rows' states are written too; with probs also set, they alone, and nothing is drawn.
-// skip_every (with state): of every skip_every + 1 rows the last is left out.
+// skip_every (with state): of every skip_every + 1 rows the last is left out. bonus (with state and
+// probs, without penalties): which rows are drawn from all the same.
 template <class Tin>
 int run_sample(const vsamp_args* a, float* probs, int64_t probs_stride, hipStream_t st,
                vs::RowState* state = nullptr, int param_div = 1, const float* tile_max = nullptr,
-               uint32_t* tile_arrive = nullptr, int tile_G = 1, int skip_every = 0) {
+               uint32_t* tile_arrive = nullptr, int tile_G = 1, int skip_every = 0, const vs::BonusDraws* bonus = nullptr) {
   const bool pen = wants_penalties(a);
   if (state && pen && !probs) return fail(VSAMP_E_ARG, "row states are written without penalties only");
   if ((a->flags & VSAMP_HIST_APPEND) && (state || probs))
@@ -342,6 +343,9 @@ int run_sample(const vsamp_args* a, float* probs, int64_t probs_stride, hipStrea
   // One launch per step: the penalty phase runs at the start of the same kernel.
   if (state && pen)  // (probabilities)
     hipLaunchKernelGGL((vs::k_sample<Tin, true, true>), dim3(a->batch), dim3(vs::kThreads), 0, st, s, vs::OwnRow{});
+  else if (bonus)
+    hipLaunchKernelGGL((vs::k_sample<Tin, false, true, false, false, vs::BonusDraws>), dim3(a->batch), dim3(vs::kThreads),
+                       0, st, s, *bonus);
   else if (state)
     hipLaunchKernelGGL((vs::k_sample<Tin, false, true>),
                        dim3(skip_every ? a->batch / (skip_every + 1) * skip_every : a->batch), dim3(vs::kThreads), 0, st, s, vs::OwnRow{});
@@ -594,7 +598,7 @@ int vsamp_verify(const vsamp_verify_args* v, void* stream) {
   char* w = static_cast<char*>(v->workspace);
   vs::RowState* ts = reinterpret_cast<vs::RowState*>(w + L.ts);
   vs::RowState* ds = reinterpret_cast<vs::RowState*>(w + L.ds);
-  t.out_ids = d.out_ids = v->out_tokens;  // (the draft rows write none)
+  t.out_ids = d.out_ids = v->out_tokens;  // (row (b, j) of the target: token (b, j); the draft rows write none)
   if (int rc = validate(&t, true)) return rc;
   if (int rc = validate(&d, true)) return rc;
   if (B == 0) return VSAMP_OK;
@@ -602,18 +606,20 @@ int vsamp_verify(const vsamp_verify_args* v, void* stream) {
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool bf = t.dtype == VSAMP_BF16;
   // parameters and uniforms: one entry per sequence for all of its rows. The states of the target
-  // rows at the drafted positions and of the draft rows; nothing is drawn yet (`probs` only marks
-  // that).
-  auto states_of = [&](const vsamp_args& q, vs::RowState* out, int rows, int skip) {
+  // rows at the drafted positions and of the draft rows, from which nothing is drawn yet (`probs`
+  // only marks that); the bonus rows join them while all target rows fit one round on the CUs.
+  const bool one_round = t.batch <= current_cus() && t.batch <= vs::kThreads;  // (ResidualRow: a thread per draft)
+  const vs::BonusDraws bonus{K + 1, reinterpret_cast<uint32_t*>(w + L.done)};
+  auto states_of = [&](const vsamp_args& q, vs::RowState* out, int rows, int skip, const vs::BonusDraws* draws) {
     float* mark = reinterpret_cast<float*>(out);
-    return bf ? run_sample<uint16_t>(&q, mark, 0, st, out, rows, nullptr, nullptr, 1, skip)
-              : run_sample<float>(&q, mark, 0, st, out, rows, nullptr, nullptr, 1, skip);
+    return bf ? run_sample<uint16_t>(&q, mark, 0, st, out, rows, nullptr, nullptr, 1, skip, draws)
+              : run_sample<float>(&q, mark, 0, st, out, rows, nullptr, nullptr, 1, skip, draws);
   };
-  if (int rc = states_of(t, ts, K + 1, K)) return rc;
+  if (int rc = one_round ? states_of(t, ts, K + 1, 0, &bonus) : states_of(t, ts, K + 1, K, nullptr)) return rc;
   if (v->draft_states) {
     if (reinterpret_cast<uintptr_t>(v->draft_states) & 7u) return fail(VSAMP_E_ARG, "draft_states must be 8-byte aligned");
     ds = static_cast<vs::RowState*>(const_cast<void*>(v->draft_states));
-  } else if (int rc = states_of(d, ds, K, 0)) {
+  } else if (int rc = states_of(d, ds, K, 0, nullptr)) {
     return rc;
   }
   vs::VerifyArgs a;
@@ -646,6 +652,16 @@ int vsamp_verify(const vsamp_verify_args* v, void* stream) {
   const dim3 gr(static_cast<unsigned>(on_cus > B ? on_cus : B));
   vs::SampleArgs s = sample_args(&t);
   s.param_div = K + 1;
+  if (one_round) {
+    if (bf)
+      hipLaunchKernelGGL((vs::k_sample<uint16_t, false, false, false, false, vs::ResidualRow>), gr, dim3(vs::kThreads), 0,
+                         st, s, vs::ResidualRow{a});
+    else
+      hipLaunchKernelGGL((vs::k_sample<float, false, false, false, false, vs::ResidualRow>), gr, dim3(vs::kThreads), 0, st,
+                         s, vs::ResidualRow{a});
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? VSAMP_OK : hip_fail(e, "launch k_sample (verify)");
+  }
   if (bf) {
     hipLaunchKernelGGL(vs::k_verify_accept<uint16_t>, dim3(1), dim3(vs::kThreads), 0, st, a);
     hipLaunchKernelGGL((vs::k_sample<uint16_t, false, false, false, false, vs::VerifyRow>), gr, dim3(vs::kThreads), 0,

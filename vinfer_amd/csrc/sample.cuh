@@ -3630,13 +3630,15 @@ __device__ __forceinline__ SampleArgs globalized(SampleArgs a) {
 // SPLIT: a bf16 split-row launch (grid B * G).
 // TILES: rows (bf16 or fp32) with their tile maxima (a.tile_max): the rows tile_row can decide
 // are decided from a few tiles, the others take the row passes.
-// PICK: which row a workgroup takes (OwnRow: by its place in the grid).
+// PICK: which row a workgroup takes (OwnRow: by its place in the grid), and with kDraws which rows of a
+// launch that draws nothing are drawn from all the same.
 struct OwnRow {
   static constexpr bool kOwn = true;
+  static constexpr bool kDraws = false;
 };
 template <class Tin, bool PEN, bool STATE = false, bool SPLIT = false, bool TILES = false, class PICK = OwnRow>
 __global__ __launch_bounds__(kThreads) void k_sample(SampleArgs a_, PICK pick) {
-  const SampleArgs a = globalized(a_);
+  SampleArgs a = globalized(a_);
   // 128 KB: the key histogram (or the generic path's penalty counts), then the id-search /
   // radix scratch
   __shared__ __align__(16) uint32_t big[kChunk];
@@ -3655,6 +3657,9 @@ __global__ __launch_bounds__(kThreads) void k_sample(SampleArgs a_, PICK pick) {
   } else {
     r = pick.template row<Tin>(big, f);
     if (r < 0) return;  // (uniform)
+  }
+  if constexpr (PICK::kDraws) {
+    if (pick.draws(r)) a.out_probs = nullptr;  // (uniform)
   }
   // the row's parameters: thread w < kParamWords loads word w, the others word 0 (every thread
   // loads: a load on one branch only would make later waits wait for every load in flight)
@@ -3756,6 +3761,7 @@ __global__ __launch_bounds__(kThreads, 8) void k_lowered(SampleArgs a_) {
 }
 struct UndecidedRow {
   static constexpr bool kOwn = false;
+  static constexpr bool kDraws = false;
   const uint32_t* marks;
   template <class Tin>
   __device__ __forceinline__ int row(uint32_t*, FastSmem&) const {

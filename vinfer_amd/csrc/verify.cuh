@@ -15,16 +15,22 @@
 // whose inclusive prefix of w exceeds floor(m * R / 2^24), R the sum. A point-mass row (greedy,
 // degenerate) has mass 2^42 at its token and S = 2^42.
 //
-// The sampling kernel has already run over the target rows at the drafted positions and the draft
-// rows (its RowState output gives each row's kept set, max and S), so these kernels read logits
-// only where they decide: the drafted tokens' two values per position, for a rejected position
-// the target and draft rows, once to sum the residual and once more inside the stripe that holds
-// the token, and for a sequence whose drafts were all accepted the bonus position's row, which is
-// sampled then. So the rows at the bonus position cost nothing where a draft is rejected, the
-// drafted positions' rows are not drawn from (but in the rare row without residual mass), and the
-// bonus rows and the residuals share one launch: 192 sequences of one draft, V = 262144, 137.4 us
-// a call when every target row was sampled first (384 rows, one and a half rounds on 256 CUs) and
-// the residuals took a launch of their own, 89 us now.
+// The sampling kernel has already run over the target rows and the draft rows (its RowState output
+// gives each row's kept set, max and S), so these kernels read logits only where they decide: the
+// drafted tokens' two values per position and, for a rejected position, the target and draft rows,
+// once to sum the residual and once more inside the stripe that holds the token. The drafted
+// positions' rows are not drawn from (but in the rare row without residual mass). The bonus position's
+// row is drawn from where it costs least:
+//   * while the target rows fit one round on the CUs, in that launch (BonusDraws), which one more
+//     workgroup a sequence makes ~4 us longer; the residuals' launch then works out the acceptance
+//     itself (ResidualRow), and a fully accepted sequence is done. V = 151936, us a call in this form
+//     against the other one: 8 sequences of 1 draft 30.4/47.2 against 49.1/48.8 (all accepted / drafts
+//     from a close draft model), 64 of 2 33.3/52.7 against 53.7/54.5, 128 of 1 34.2/56.1 against
+//     52.8/53.6; where every sequence is rejected it is slower by those 4 us;
+//   * past one round, where those rows would cost rounds of their own, only after all drafts were
+//     accepted (k_verify_accept), in one launch with the residual draws (VerifyRow): 192 sequences
+//     of one draft, V = 262144, 137.4 us a call when every target row was sampled first (384 rows, one
+//     and a half rounds on 256 CUs) and the residuals took a launch of their own, 89 us now.
 // A bf16 row holds at most 65536 distinct values, and its kept ones sit in a short run of keys
 // below the row's max: the two terms of w are tabulated per key in LDS for the top kTab keys
 // of each row (a kept token below that run is computed directly), so the residual pass costs
@@ -126,6 +132,22 @@ struct ResidualSide {
   }
 };
 
+// Whether draft j of sequence b is accepted.
+template <class Tin>
+__device__ __forceinline__ bool accepts(const VerifyArgs& a, int b, int j) {
+  const int K = a.K;
+  const int d = a.drafts[b * K + j];
+  if (d < 0 || d >= a.V) return false;  // a token outside the vocabulary is never accepted
+  const RowState st = a.ts[b * (K + 1) + j];
+  const RowState sd = a.ds[b * K + j];
+  const float xt = load_one<Tin>(static_cast<const Tin*>(a.tgt) + static_cast<int64_t>(b * (K + 1) + j) * a.tstride, d);
+  const float xd = load_one<Tin>(static_cast<const Tin*>(a.drf) + static_cast<int64_t>(b * K + j) * a.dstride, d);
+  const u64 P = token_mass(xt, d, st), Q = token_mass(xd, d, sd);
+  const u128 lhs = static_cast<u128>(u24(a.u_acc[b * K + j])) * Q * kept_mass(st);  // < 2^127
+  const u128 rhs = (static_cast<u128>(P) * kept_mass(sd)) << 24;
+  return lhs < rhs;
+}
+
 // One workgroup, a thread per sequence: the acceptance chain. Writes the accepted drafts and, when
 // all are accepted, the count; leaves the first rejected position in jr, clears the row's slice
 // counter and lists the rejected and the accepted sequences (ascending) for the last launch.
@@ -135,24 +157,12 @@ __global__ __launch_bounds__(kThreads) void k_verify_accept(VerifyArgs a) {
   exp_table_init();
   __syncthreads();
   const int K = a.K, B = a.B;
-  const Tin* tgt = static_cast<const Tin*>(a.tgt);
-  const Tin* drf = static_cast<const Tin*>(a.drf);
   uint32_t listed = 0;
   for (int b0 = 0; b0 < B; b0 += kThreads) {
     const int b = b0 + static_cast<int>(threadIdx.x);
     int j = K;
     if (b < B) {
-      for (j = 0; j < K; ++j) {
-        const int d = a.drafts[b * K + j];
-        if (d < 0 || d >= a.V) break;  // a token outside the vocabulary is never accepted
-        const RowState st = a.ts[b * (K + 1) + j];
-        const RowState sd = a.ds[b * K + j];
-        const float xt = load_one<Tin>(tgt + static_cast<int64_t>(b * (K + 1) + j) * a.tstride, d);
-        const float xd = load_one<Tin>(drf + static_cast<int64_t>(b * K + j) * a.dstride, d);
-        const u64 P = token_mass(xt, d, st), Q = token_mass(xd, d, sd);
-        const u128 lhs = static_cast<u128>(u24(a.u_acc[b * K + j])) * Q * kept_mass(st);  // < 2^127
-        const u128 rhs = (static_cast<u128>(P) * kept_mass(sd)) << 24;
-        if (!(lhs < rhs)) break;
+      for (j = 0; j < K && accepts<Tin>(a, b, j); ++j) {
       }
       int32_t* out = a.out_tokens + static_cast<int64_t>(b) * (K + 1);
       for (int i = 0; i <= K; ++i) out[i] = i < j ? a.drafts[b * K + i] : -1;
@@ -189,13 +199,13 @@ struct ResidualSmem {
 static_assert(sizeof(ResidualSmem) <= sizeof(FastSmem), "the residual's scratch lies over FastSmem");
 static_assert(2 * kTab * sizeof(u64) <= kChunk * sizeof(uint32_t), "the tables lie over the histogram");
 
-// One (row, slice) item of the residual draw of rejected sequence b: the slice sums the residual
+// One (row, slice) item of the residual draw of sequence b, rejected at position jr: the slice sums the residual
 // over its share of the row's stripes; the last slice of the row to finish finds the stripe that
 // holds floor(m * R / 2^24) and the token inside it. Returns true (in every thread of the last
 // slice's workgroup) when the row has no residual mass: the caller draws from the target row.
 template <class Tin>
-__device__ __forceinline__ bool residual_item(const VerifyArgs& a, int b, int slice, int slices, uint32_t* big,
-                                              ResidualSmem& m) {
+__device__ __forceinline__ bool residual_item(const VerifyArgs& a, int b, int jr, int slice, int slices,
+                                              uint32_t* big, ResidualSmem& m) {
   constexpr bool kBf16 = sizeof(Tin) == 2;
   auto& cell = m.cell;
   auto& red = m.red;
@@ -205,7 +215,6 @@ __device__ __forceinline__ bool residual_item(const VerifyArgs& a, int b, int sl
   const int tid = threadIdx.x;
   const int wv = tid / kWave;
   const int K = a.K;
-  const int jr = a.jr[b];
   const Tin* tgt = static_cast<const Tin*>(a.tgt);
   const Tin* drf = static_cast<const Tin*>(a.drf);
   int32_t* out = a.out_tokens + static_cast<int64_t>(b) * (K + 1);
@@ -537,15 +546,16 @@ __device__ __forceinline__ bool residual_item(const VerifyArgs& a, int b, int sl
   return residual(std::false_type{});
 }
 
-// The last launch's rows: the bonus rows of the accepted sequences (k_sample's row code, one
-// workgroup a row) and the residual draws of the rejected ones, (row, slice) items row-major over
-// their list, one item a workgroup: the grid is the larger of B and the CUs the items can use (the
-// LDS holds one workgroup a CU), and the slices are chosen to fit it. (No loop over the items: with
-// one the compiler kept both kinds' values live across it and spilled, 640 bytes a lane, 72-78 us.)
-// The launch's SampleArgs describe the target rows, its out_ids the emitted tokens: row (b, j)'s
-// draw is token (b, j).
+// Target rows past one round on the CUs: the last launch's rows, the bonus rows of the accepted
+// sequences (k_sample's row code, one workgroup a row) and the residual draws of the rejected ones,
+// (row, slice) items row-major over their list, one item a workgroup: the grid is the larger of B and
+// the CUs the items can use (the LDS holds one workgroup a CU), and the slices are chosen to fit it.
+// (No loop over the items: with one the compiler kept both kinds' values live across it and spilled,
+// 640 bytes a lane, 72-78 us.) The launch's SampleArgs describe the target rows, its out_ids the
+// emitted tokens: row (b, j)'s draw is token (b, j).
 struct VerifyRow {
   static constexpr bool kOwn = false;
+  static constexpr bool kDraws = false;
   VerifyArgs a;
   // The target row this workgroup draws from: a bonus row, or a rejected one without residual mass
   // (after its residual); -1: none.
@@ -559,10 +569,86 @@ struct VerifyRow {
     const int q = item - nacc;
     if (q >= nrej * slices) return -1;
     const int b = a.rej[q / slices];
+    const int jr = a.jr[b];
     __syncthreads();  // (publishes the exp table)
-    if (!residual_item<Tin>(a, b, q % slices, slices, big, *reinterpret_cast<ResidualSmem*>(&f))) return -1;  // (uniform)
+    if (!residual_item<Tin>(a, b, jr, q % slices, slices, big, *reinterpret_cast<ResidualSmem*>(&f))) return -1;  // (uniform)
     __syncthreads();  // (the residual's LDS is free)
-    return b * (a.K + 1) + a.jr[b];
+    return b * (a.K + 1) + jr;
+  }
+};
+
+// Target rows of one round: all in the first launch, each sequence's last (its bonus row) also drawn
+// from, and the slice counters of the last launch cleared by its workgroup.
+struct BonusDraws {
+  static constexpr bool kOwn = false;
+  static constexpr bool kDraws = true;
+  int K1;  // K + 1
+  uint32_t* done;
+  template <class Tin>
+  __device__ __forceinline__ int row(uint32_t*, FastSmem&) const {
+    const int r = static_cast<int>(blockIdx.x);
+    if (draws(r) && threadIdx.x == 0) done[r / K1] = 0;
+    return r;
+  }
+  __device__ __forceinline__ bool draws(int r) const { return r % K1 == K1 - 1; }
+};
+
+// Then the launch after the states': the residuals' (row, slice) items, each workgroup working out for
+// itself which is its own; an accepted sequence has its tokens already. (The lists of k_verify_accept
+// would cost a launch of one workgroup, ~6 us, before this one.)
+struct ResidualRow {
+  static constexpr bool kOwn = false;
+  static constexpr bool kDraws = false;
+  VerifyArgs a;
+  // Token i of sequence b, first rejected at j: but for token j, which is the bonus token, already
+  // there, or the residual's.
+  __device__ __forceinline__ void tokens(int b, int j) const {
+    const int i = threadIdx.x;
+    if (i <= a.K && i != j) a.out_tokens[static_cast<int64_t>(b) * (a.K + 1) + i] = i < j ? a.drafts[b * a.K + i] : -1;
+    if (i == 0 && j == a.K) a.out_count[b] = a.K + 1;
+  }
+  // A target row without residual mass, to draw from (after its residual); -1: none.
+  template <class Tin>
+  __device__ __forceinline__ int row(uint32_t* big, FastSmem& f) const {
+    const int K = a.K, B = a.B;
+    const int tid = threadIdx.x;
+    const int item = blockIdx.x;
+    int b, jr, slice, slices = a.max_slices;  // (uniform)
+    if (B * slices <= static_cast<int>(gridDim.x)) {
+      // every sequence has all of its slices: only its own acceptance counts (a lane per draft, K <= 64)
+      b = item / slices;
+      slice = item % slices;
+      const int l = static_cast<int>(lane_id());
+      __syncthreads();  // (publishes the exp table)
+      const u64 no = __ballot(l < K && !accepts<Tin>(a, b, l));
+      jr = no ? __ffsll(static_cast<long long>(no)) - 1 : K;
+      if (slice == 0) tokens(b, jr);
+      if (jr == K) return -1;
+    } else {
+      // the whole batch's acceptance (a thread per draft, B K < kThreads), and the rejected rows split
+      // as far as the grid goes
+      int* const first = reinterpret_cast<int*>(big);  // [B] the first rejected position (K: none)
+      int* const rej = first + kThreads;               // the rejected sequences, ascending
+      if (tid < B) first[tid] = K;
+      __syncthreads();  // (publishes the exp table too)
+      if (tid < B * K && !accepts<Tin>(a, tid / K, tid % K)) atomicMin(&first[tid / K], tid % K);
+      __syncthreads();
+      const bool r = tid < B && first[tid] < K;
+      uint32_t nrej;
+      const uint32_t at = block_excl_scan<uint32_t>(r ? 1u : 0u, f.red32, &nrej);
+      if (r) rej[at] = tid;
+      if (item < B) tokens(item, first[item]);
+      slices = residual_slices(static_cast<int>(nrej), static_cast<int>(gridDim.x), slices);
+      if (item >= static_cast<int>(nrej) * slices) return -1;
+      __syncthreads();
+      b = __builtin_amdgcn_readfirstlane(rej[item / slices]);
+      jr = __builtin_amdgcn_readfirstlane(first[b]);
+      slice = item % slices;
+      __syncthreads();  // (the residual's tables go over the lists)
+    }
+    if (!residual_item<Tin>(a, b, jr, slice, slices, big, *reinterpret_cast<ResidualSmem*>(&f))) return -1;  // (uniform)
+    __syncthreads();  // (the residual's LDS is free)
+    return b * (K + 1) + jr;
   }
 };
 
