@@ -4,6 +4,7 @@ oracle, at the sizes and parameters where the route changes."""
 
 from __future__ import annotations
 
+import ctypes
 import math
 
 import numpy as np
@@ -107,3 +108,34 @@ def test_more_fp32_rows_than_cus_equal_smaller_batches(V):
         torch.cuda.synchronize()
         assert torch.equal(got[0], torch.cat([p[0] for p in parts]))
         assert torch.equal(got[1], torch.cat([p[1] for p in parts]))
+
+
+def launches(fn) -> int:
+    """Kernels of one call, from a captured graph (which is not run)."""
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g):
+        fn()
+    n = ctypes.c_size_t()
+    hip = ctypes.CDLL("libamdhip64.so")
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    return n.value
+
+
+def penalised_step(s, B, V, mean=0.0, std=2.0, K=50, history=300, seed=0, **kw):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    x = torch.randn(B, V, generator=g, device=DEV) * std + mean
+    ids = torch.randint(0, V, (B * history,), generator=g, device=DEV).to(torch.int32)
+    off = torch.arange(0, B * history + 1, history, dtype=torch.int32, device=DEV)
+    p = pack_params([SamplingParams(**{"temperature": 0.8, "top_k": K, "top_p": 0.9, "repetition_penalty": 1.05,
+                                       "presence_penalty": 0.3, "frequency_penalty": 0.1, **kw})] * B).to(DEV)
+    return s.prepare_batch(x, p, torch.rand(B, generator=g, device=DEV), ids, off)
+
+
+def test_two_launches_only_past_one_row_a_cu_and_from_the_sample_on():
+    s = SAMPLER.resolve("hip", BackendContext(DEV, torch.float32))
+    cus = torch.cuda.get_device_properties(DEV).multi_processor_count
+    for B, V, want in ((cus, 16384, 1), (cus + 1, 16384, 2), (cus + 1, 16383, 1), (cus + 1, 8192, 1)):
+        step = penalised_step(s, B, V)
+        step.launch()
+        torch.cuda.synchronize()
+        assert launches(step.launch) == want, (B, V)

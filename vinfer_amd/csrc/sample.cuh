@@ -1362,6 +1362,7 @@ __device__ __forceinline__ void find_top_bin(const uint32_t* h13, int bins, uint
 // launch, 136.6 with two workgroups a CU (k_lowered).
 constexpr int kLowK = 192;       // top-k served
 constexpr int kLowDepth = 2;     // stripes sampled
+constexpr int kLowVocab = kLowDepth * kThreads * kBlk;  // the shortest row served: the sample
 constexpr int kLowCap = 1023;    // staged candidates: one a thread, and one for the draft id
 constexpr int kLowSlots = 4096;  // hash table
 constexpr int kLowWords = kBitmapOffset + 8192 + 2 * 1024;  // LDS words from the scratch's start: 60 KB
@@ -1398,7 +1399,7 @@ __device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, Row<Tin> r
   if (!(p.T > 0.0f) || p.K < 1 || p.K >= V || p.K > kLowK || L < 1 || a.out_probs) return false;
   if (!(p.rep >= 1.0f && p.rep < INFINITY && p.pres >= 0.0f && p.freq >= 0.0f)) return false;
   if (p.rep == 1.0f && p.pres == 0.0f && p.freq == 0.0f) return false;  // (no penalties: the generic path's own stream)
-  if (V / kBlk / kThreads < kLowDepth) return false;
+  if (V < kLowVocab) return false;
   const uint32_t K = static_cast<uint32_t>(p.K);
   uint32_t* const h13 = reinterpret_cast<uint32_t*>(&g) + kBitmapOffset;  // the sample's bins, then:
   uint32_t* const hkey = h13;                       // the hash table's ids
