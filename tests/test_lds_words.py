@@ -12,7 +12,7 @@ import pytest
 
 CSRC = Path(__file__).resolve().parents[1] / "vinfer_amd" / "csrc"
 BARRIERS = ("lds_barrier", "__syncthreads", "block_excl_scan", "block_sum", "block_max_u64", "sort_top", "sort_cands",
-            "find_top_bin")
+            "sample_bound")
 TOKEN = re.compile(r"\b(?P<barrier>" + "|".join(BARRIERS) + r")\s*[<(]"
                    r"|(?P<rmw>&)?\bsh\[(?P<word>[^\]]+)\](?P<store>\s*=(?!=))?"
                    r"|(?P<guard>\bif\s*\((?:tid < kWave|tid == 0|l == i)\))"

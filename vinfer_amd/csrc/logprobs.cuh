@@ -193,7 +193,7 @@ __device__ __forceinline__ bool lp_one_pass(const LogprobArgs& a, const Row<uint
 
 // Rows of at least two stripes, in one pass and without a histogram: each element's fp32
 // exponential against the sample's max M0 is added in fp64 as it is read, but for the elements >= tau
-// (the bin of about the 3n-th largest of the row, from the first two stripes' per-thread maxima),
+// (about the 3n-th largest of the row, from the first two stripes' per-thread maxima),
 // which are staged: they hold the row's max and its top n, and their exponentials are taken in
 // fp64 against the row's max M, so that M0's distance from M costs the large terms no precision.
 // Their sum is in fixed point: the staging order varies, the sum does not. Returns false, with
@@ -210,7 +210,7 @@ constexpr int kLpBins = 8192;
 constexpr int kLpWords = kLpBins + 2 * (kLpCap + 1);  // LDS words: bins (then sort keys and list), staged elements
 template <class Tin>
 __device__ __forceinline__ bool lp_stream(const LogprobArgs& a, const Row<Tin>& row, int r, uint32_t* area, uint32_t* sh,
-                                          uint32_t* red32, u64* red64) {
+                                          uint32_t* words, u64* red64) {
   const int tid = threadIdx.x;
   const int V = row.V;
   const int n = a.n_top;
@@ -219,8 +219,8 @@ __device__ __forceinline__ bool lp_stream(const LogprobArgs& a, const Row<Tin>& 
   WholeBlock<Tin> q[kLpDepth];
 #pragma unroll
   for (int k = 0; k < kLpDepth; ++k) q[k].load(row.p, k * kThreads + tid);
-  for (int i = tid; i < kLpBins / 4; i += kThreads) reinterpret_cast<uint4*>(area)[i] = make_uint4(0, 0, 0, 0);
-  if (tid < 8) sh[tid] = 0;  // [0] the bin, [2] staged, [3] a NaN or +inf, [4] M0's key, [5] M's
+  for (int i = tid; i < kBoundWords / 4; i += kThreads) reinterpret_cast<uint4*>(area)[i] = make_uint4(0, 0, 0, 0);
+  if (tid < 8) sh[tid] = 0;  // [2] staged, [3] a NaN or +inf, [4] M0's key, [5] M's
   __syncthreads();           // (the exp table too)
   float v[kLpDepth][kBlk];
   float mx = -INFINITY;  // (IEEE maximum: a NaN stays)
@@ -230,16 +230,12 @@ __device__ __forceinline__ bool lp_stream(const LogprobArgs& a, const Row<Tin>& 
     mx = __builtin_elementwise_maximum(mx, max_of8(v[k]));
   }
   auto umax = [](uint32_t x, uint32_t y) { return x > y ? x : y; };
-  atomicAdd(&area[key_of(mx) >> 19], 1u);
   {
     const uint32_t wm = dpp::reduce(key_of(mx), umax);
     if (lane_id() == 0) atomicMax(&sh[4], wm);
   }
-  __syncthreads();
   const uint32_t nn = static_cast<uint32_t>(n) < static_cast<uint32_t>(V) ? static_cast<uint32_t>(n) : static_cast<uint32_t>(V);
-  find_top_bin(area, kLpBins, sample_rank<kLpDepth>(nn, V), red32, &sh[0]);
-  __syncthreads();
-  const float tau = val_of(max(sh[0] << 19, key_of(-INFINITY)));  // (the bin's least value; bin 0: none found)
+  const float tau = sample_bound<kLpDepth>(area, mx, nn, V, kLpCap, words);
   const float M0 = val_of(sh[4]);
   if (!(tau > -INFINITY && M0 < INFINITY)) return false;  // (uniform; a NaN M0 too)
   double s = 0.0;
@@ -328,7 +324,7 @@ __global__ __launch_bounds__(kThreads) void k_logprobs(LogprobArgs a) {
   const int n = a.n_top;
   exp_table_init();  // (published by the first barrier below)
   if constexpr (!TILES) {
-    if (lp_stream<Tin>(a, row, r, h13, sh, rdx.hcnt, srch.red64)) return;  // (uniform)
+    if (lp_stream<Tin>(a, row, r, h13, sh, rdx.bk, srch.red64)) return;  // (uniform)
     __syncthreads();  // (every thread is done with its LDS)
   }
   Cand* cand = reinterpret_cast<Cand*>(h13);

@@ -1313,6 +1313,53 @@ __device__ __forceinline__ bool sorted_tail(const SampleArgs& a, const Row<Tin>&
   return true;
 }
 
+// ---- the k-th largest of counted keys ------------------------------------------------------------
+// (wave 0) Of 4096 bins that count keys by their top 12 bits, the one that holds the k-th largest
+// (1-based; at least k are counted), to *bin, and the count of the bins above it, to *above.
+__device__ __forceinline__ void top_bin12(const uint32_t* h12, uint32_t k, uint32_t* bin, uint32_t* above) {
+  // lane l sums bins 4095 - 64 l - 63 .. 4095 - 64 l (lane 0 the top ones), then lane i of the crossing
+  // lane's 64 bins takes bin 4095 - 64 L - i
+  const int l = static_cast<int>(lane_id());
+  uint32_t sum = 0;
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    const uint4 v = reinterpret_cast<const uint4*>(h12 + 4032 - 64 * l)[q];
+    sum += v.x + v.y + v.z + v.w;
+  }
+  const uint32_t incl = wave_incl_scan<uint32_t>(sum);
+  const int L = __ffsll(static_cast<long long>(__ballot(incl >= k))) - 1;
+  const uint32_t over = __builtin_amdgcn_readlane(incl, L) - __builtin_amdgcn_readlane(sum, L);
+  const uint32_t c = h12[4095 - 64 * L - l];
+  const uint32_t incl2 = over + wave_incl_scan<uint32_t>(c);
+  const int i = __ffsll(static_cast<long long>(__ballot(incl2 >= k))) - 1;
+  if (l == i) {
+    *bin = static_cast<uint32_t>(4095 - 64 * L - i);
+    *above = incl2 - c;
+  }
+}
+// (wave 0) The same of the 256 sub-bins that count that bin's keys by their next 8 bits, `above` keys
+// above them: the sub-bin, and in *reach how many keys lie in it or above (both uniform).
+__device__ __forceinline__ uint32_t top_sub8(const uint32_t* h8, uint32_t k, uint32_t above, uint32_t* reach) {
+  // lane l: sub-bins 255 - 4 l .. 252 - 4 l, descending
+  const int l = static_cast<int>(lane_id());
+  const uint4 v = reinterpret_cast<const uint4*>(h8)[63 - l];
+  const uint32_t c4[4] = {v.w, v.z, v.y, v.x};
+  const uint32_t s4 = v.x + v.y + v.z + v.w;
+  uint32_t run = above + wave_incl_scan<uint32_t>(s4) - s4;
+  uint32_t sub = 0xFFFFFFFFu, got = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (run < k && k <= run + c4[i]) {
+      sub = static_cast<uint32_t>(255 - 4 * l - i);
+      got = run + c4[i];
+    }
+    run += c4[i];
+  }
+  const int L = __ffsll(static_cast<long long>(__ballot(sub != 0xFFFFFFFFu))) - 1;  // (one lane holds it)
+  *reach = __builtin_amdgcn_readlane(got, L);
+  return __builtin_amdgcn_readlane(sub, L);
+}
+
 // ---- a bound on a row's largest elements from a sample -------------------------------------------
 // The rank, among the per-thread maxima of the first DEPTH stripes (16 elements each at DEPTH 2),
 // that about three times the n largest of the row lie above.
@@ -1321,28 +1368,35 @@ __device__ __forceinline__ uint32_t sample_rank(uint32_t n, int V) {
   constexpr u64 kSample = static_cast<u64>(DEPTH) * kThreads * kBlk;
   return static_cast<uint32_t>((3ull * n * kSample + static_cast<u64>(V) - 1) / static_cast<u64>(V)) + 2u;
 }
-// The bin of the m-th largest of the 8192 counted keys, to *bin (left alone when fewer were
-// counted); every thread calls, a barrier publishes. Thread t sums bins 8191 - 8t .. 8184 - 8t,
-// descending.
-__device__ __forceinline__ void find_top_bin(const uint32_t* h13, int bins, uint32_t m, uint32_t* red, uint32_t* bin) {
+// The value of that rank to 20 bits of its key (the lowest value with those bits), `mx` being the
+// calling thread's maximum; -inf where the row would have more than `cap` elements that reach it (ties:
+// as many as the maxima that do, a row of independent elements, tell). Every thread calls, the result
+// is the same in all. `h`: kBoundWords zeroed words, `w` three words, both free afterwards.
+// To 13 bits, as one scan of 8192 bins gave it, a bin of [16, 32) is 1 wide: at N(20, 1) and n = 50 most
+// rows of 151936 had more elements at its floor than can be staged, and were read for nothing.
+constexpr int kBoundWords = 4096 + 256;
+template <int DEPTH>
+__device__ __forceinline__ float sample_bound(uint32_t* h, float mx, uint32_t n, int V, uint32_t cap, uint32_t* w) {
   const int tid = threadIdx.x;
-  uint32_t c8[8], s8 = 0;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const uint4 w = reinterpret_cast<const uint4*>(h13)[bins / 4 - 1 - 2 * tid - h];
-    c8[4 * h] = w.w;
-    c8[4 * h + 1] = w.z;
-    c8[4 * h + 2] = w.y;
-    c8[4 * h + 3] = w.x;
-    s8 += w.x + w.y + w.z + w.w;
+  uint32_t* const h8 = h + 4096;
+  const uint32_t key = key_of(mx);
+  const uint32_t m = sample_rank<DEPTH>(n, V);
+  atomicAdd(&h[key >> 20], 1u);
+  lds_barrier();
+  if (tid < kWave) top_bin12(h, m, &w[0], &w[1]);
+  lds_barrier();
+  if ((key >> 20) == w[0]) atomicAdd(&h8[(key >> 12) & 255u], 1u);
+  lds_barrier();
+  if (tid < kWave) {
+    uint32_t reach;
+    const uint32_t k32 = (w[0] << 20) | (top_sub8(h8, m, w[1], &reach) << 12);
+    // a share f of the threads' maxima reach it: about -ln(1 - f) elements a thread do
+    const float each = -__logf(1.0f - static_cast<float>(reach) * (1.0f / kThreads));
+    const bool fits = each * static_cast<float>(V) <= static_cast<float>(cap) * (DEPTH * kBlk);
+    if (tid == 0) w[2] = fits ? k32 : 0u;
   }
-  uint32_t tot;
-  uint32_t run = block_excl_scan<uint32_t>(s8, red, &tot);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    if (run < m && m <= run + c8[i]) *bin = static_cast<uint32_t>(bins - 1 - 8 * tid - i);
-    run += c8[i];
-  }
+  lds_barrier();
+  return val_of(max(w[2], key_of(-INFINITY)));
 }
 
 // ---- top-k rows whose penalties only lower values ----------------------------------------------
@@ -1354,8 +1408,8 @@ __device__ __forceinline__ void find_top_bin(const uint32_t* h13, int bins, uint
 // least K of them, hold the top K (and the row's max). In place of the penalty pass -- the whole
 // history's presence bitmap, ranks, counts, (id, count) pairs and a gather of every distinct id's
 // value, ~30 us of a 62 us row at 16K ids -- and of the masked passes after it.
-// tau: the bin (13 key bits) of the m-th largest of the first kLowDepth stripes' per-thread maxima,
-// m three times the K-th's share of that sample (penalised candidates may fall below tau).
+// tau: the m-th largest of the first kLowDepth stripes' per-thread maxima to 20 bits, m three times the
+// K-th's share of that sample (penalised candidates may fall below tau).
 // Returns false, with nothing written, for a row it does not decide (too few or too many
 // candidates, a NaN or +inf, a threshold below tau): the caller runs the penalty pass.
 // Measured (1024 fp32 rows of 151936, top-k 50, histories up to 32768): 255.0 -> 160.7 us in one
@@ -1401,24 +1455,24 @@ __device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, Row<Tin> r
   if (p.rep == 1.0f && p.pres == 0.0f && p.freq == 0.0f) return false;  // (no penalties: the generic path's own stream)
   if (V < kLowVocab) return false;
   const uint32_t K = static_cast<uint32_t>(p.K);
-  uint32_t* const h13 = reinterpret_cast<uint32_t*>(&g) + kBitmapOffset;  // the sample's bins, then:
-  uint32_t* const hkey = h13;                       // the hash table's ids
-  uint32_t* const hcnt = hkey + kLowSlots;          // and counts, then:
-  Cand* const cand = reinterpret_cast<Cand*>(h13);  // the penalised candidates,
-  u64* const kk = reinterpret_cast<u64*>(h13 + 2048);       // their sort keys
-  Cand* const srt = reinterpret_cast<Cand*>(h13 + 4096);    // and the sorted list
-  constexpr int kBins = 8192;
-  Cand* const stage = reinterpret_cast<Cand*>(h13 + kBins);
-  static_assert(kBitmapOffset + kBins + 2 * (kLowCap + 1) <= kLowWords && 2 * kLowSlots <= kBins &&
-                    4096 + 2 * kSortCap <= kBins && kLowCap < kThreads,
+  uint32_t* const bins = reinterpret_cast<uint32_t*>(&g) + kBitmapOffset;  // the sample's bins, then:
+  uint32_t* const hkey = bins;                       // the hash table's ids
+  uint32_t* const hcnt = hkey + kLowSlots;           // and counts, then:
+  Cand* const cand = reinterpret_cast<Cand*>(bins);  // the penalised candidates,
+  u64* const kk = reinterpret_cast<u64*>(bins + 2048);     // their sort keys
+  Cand* const srt = reinterpret_cast<Cand*>(bins + 4096);  // and the sorted list
+  constexpr int kTable = 2 * kLowSlots;
+  Cand* const stage = reinterpret_cast<Cand*>(hkey + kTable);
+  static_assert(kBitmapOffset + kTable + 2 * (kLowCap + 1) <= kLowWords && kBoundWords <= kTable &&
+                    4096 + 2 * kSortCap <= kTable && kLowCap < kThreads,
                 "the row's LDS areas");
-  // [0] the bin, [1] penalised candidates, [2] candidates, [3] a NaN or +inf, then the threshold (a word of
-  // its own for each count: every thread decides by [2], so nothing may reset it before they all have)
+  // [1] penalised candidates, [2] candidates, [3] a NaN or +inf, then the threshold (a word of its own for
+  // each count: every thread decides by [2], so nothing may reset it before they all have)
   uint32_t* const sh = g.rdx.bk;
   WholeBlock<Tin> q[kLowDepth];
 #pragma unroll
   for (int k = 0; k < kLowDepth; ++k) q[k].load(row.p, k * kThreads + tid);
-  for (int i = tid; i < kBins / 4; i += kThreads) reinterpret_cast<uint4*>(h13)[i] = make_uint4(0, 0, 0, 0);
+  for (int i = tid; i < kBoundWords / 4; i += kThreads) reinterpret_cast<uint4*>(bins)[i] = make_uint4(0, 0, 0, 0);
   if (tid < 4) sh[tid] = 0;
   lds_barrier();
   float v[kLowDepth][kBlk];
@@ -1428,12 +1482,8 @@ __device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, Row<Tin> r
     q[k].values(v[k]);
     mx = __builtin_elementwise_maximum(mx, max_of8(v[k]));
   }
-  atomicAdd(&h13[key_of(mx) >> 19], 1u);
-  lds_barrier();
-  find_top_bin(h13, kBins, sample_rank<kLowDepth>(K, V), g.rdx.hcnt, &sh[0]);
-  lds_barrier();
-  const float tau = val_of(max(sh[0] << 19, key_of(-INFINITY)));  // (the bin's least value; bin 0: none found)
-  if (!(tau > -INFINITY && tau < INFINITY)) return false;         // (uniform)
+  const float tau = sample_bound<kLowDepth>(bins, mx, K, V, kLowCap, reinterpret_cast<uint32_t*>(g.rdx.bq));
+  if (!(tau > -INFINITY && tau < INFINITY)) return false;  // (uniform)
   for (int i = tid; i < kLowSlots / 4; i += kThreads) {  // (the bins are dead; published after the pass)
     reinterpret_cast<uint4*>(hkey)[i] = make_uint4(kEmpty, kEmpty, kEmpty, kEmpty);
     reinterpret_cast<uint4*>(hcnt)[i] = make_uint4(0, 0, 0, 0);
@@ -3473,28 +3523,7 @@ __device__ __forceinline__ bool tile_row(const SampleArgs& a, const Row<Tin>& ro
   // xlo: no kept token lies below it (wave 0 decides; the others wait at the barrier)
   const uint32_t lo_key = key_of(-INFINITY);
   if (topk) {  // (uniform)
-    if (tid < kWave) {
-      // the bin of the K-th largest: lane l sums bins 4095 - 64 l - 63 .. 4095 - 64 l (lane 0
-      // the top ones), then lane i of the crossing lane's 64 bins takes bin 4095 - 64 L - i
-      const uint32_t K = static_cast<uint32_t>(p.K);
-      const int l = tid;
-      uint32_t sum = 0;
-#pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const uint4 v = reinterpret_cast<const uint4*>(h12 + 4032 - 64 * l)[q];
-        sum += v.x + v.y + v.z + v.w;
-      }
-      const uint32_t incl = wave_incl_scan<uint32_t>(sum);
-      const int L = __ffsll(static_cast<long long>(__ballot(incl >= K))) - 1;  // (K <= nT: some lane crosses)
-      const uint32_t above = __builtin_amdgcn_readlane(incl, L) - __builtin_amdgcn_readlane(sum, L);
-      const uint32_t c = h12[4095 - 64 * L - l];
-      const uint32_t incl2 = above + wave_incl_scan<uint32_t>(c);
-      const int i = __ffsll(static_cast<long long>(__ballot(incl2 >= K))) - 1;
-      if (l == i) {
-        sh[2] = static_cast<uint32_t>(4095 - 64 * L - i);
-        sh[3] = incl2 - c;  // tile maxima above the bin
-      }
-    }
+    if (tid < kWave) top_bin12(h12, static_cast<uint32_t>(p.K), &sh[2], &sh[3]);  // (K <= nT)
     lds_barrier();
     const uint32_t bin = sh[2];
 #pragma unroll
@@ -3505,20 +3534,8 @@ __device__ __forceinline__ bool tile_row(const SampleArgs& a, const Row<Tin>& ro
   if (tid < kWave) {
     float xlo = -INFINITY, xm = -INFINITY;
     if (topk) {
-      // lane l: the bin's sub-bins 255 - 4 l .. 252 - 4 l, descending
-      const uint32_t K = static_cast<uint32_t>(p.K);
-      const uint4 v = reinterpret_cast<const uint4*>(h8)[63 - tid];
-      const uint32_t c4[4] = {v.w, v.z, v.y, v.x};
-      const uint32_t s4 = v.x + v.y + v.z + v.w;
-      uint32_t run = sh[3] + wave_incl_scan<uint32_t>(s4) - s4;
-      uint32_t sub = 0xFFFFFFFFu;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (run < K && K <= run + c4[i]) sub = static_cast<uint32_t>(255 - 4 * tid - i);
-        run += c4[i];
-      }
-      const int L = __ffsll(static_cast<long long>(__ballot(sub != 0xFFFFFFFFu))) - 1;  // (one lane holds it)
-      const uint32_t k32 = (sh[2] << 20) | (__builtin_amdgcn_readlane(sub, L) << 12);
+      uint32_t reach;
+      const uint32_t k32 = (sh[2] << 20) | (top_sub8(h8, static_cast<uint32_t>(p.K), sh[3], &reach) << 12);
       const float theta = val_of(k32 > lo_key ? k32 : lo_key);
       const float zt = theta / T;
       xlo = val_of(wave_bisect(lo_key, key_of(theta), key_of(zt * T), [&](float x) { return x / T >= zt; }));
