@@ -6,6 +6,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+from dataclasses import fields
 
 import numpy as np
 import pytest
@@ -14,7 +15,7 @@ import torch
 from tests.parity import compare_ids, oracle
 from vinfer_amd.registry import BackendContext
 from vinfer_amd.sampler import SAMPLER
-from vinfer_amd.sampling import SamplingParams, pack_history, pack_params
+from vinfer_amd.sampling import PackedParams, SamplingParams, pack_history, pack_params
 from vinfer_amd.workloads import Workload
 
 pytestmark = pytest.mark.gpu
@@ -121,21 +122,53 @@ def launches(fn) -> int:
     return n.value
 
 
-def penalised_step(s, B, V, mean=0.0, std=2.0, K=50, history=300, seed=0, **kw):
+def penalised_step(s, B, V, mean=0.0, std=2.0, K=50, history=300, best=0, seed=0, **kw):
+    """A prepared step of fp32 rows N(mean, std) whose histories hold random ids, the row's `best` largest
+    twice among them; and its inputs as a Workload."""
     g = torch.Generator(device=DEV).manual_seed(seed)
     x = torch.randn(B, V, generator=g, device=DEV) * std + mean
-    ids = torch.randint(0, V, (B * history,), generator=g, device=DEV).to(torch.int32)
+    ids = torch.randint(0, V, (B, history), generator=g, device=DEV).to(torch.int32)
+    if best:
+        ids[:, :2 * best] = x.topk(best, dim=1).indices.to(torch.int32).repeat(1, 2)
     off = torch.arange(0, B * history + 1, history, dtype=torch.int32, device=DEV)
     p = pack_params([SamplingParams(**{"temperature": 0.8, "top_k": K, "top_p": 0.9, "repetition_penalty": 1.05,
                                        "presence_penalty": 0.3, "frequency_penalty": 0.1, **kw})] * B).to(DEV)
-    return s.prepare_batch(x, p, torch.rand(B, generator=g, device=DEV), ids, off)
+    w = Workload("penalised", x, p, torch.rand(B, generator=g, device=DEV), ids.view(-1), off, None)
+    return s.prepare_batch(w.logits, w.params, w.uniforms, w.hist_ids, w.hist_offsets), w
 
 
 def test_two_launches_only_past_one_row_a_cu_and_from_the_sample_on():
     s = SAMPLER.resolve("hip", BackendContext(DEV, torch.float32))
     cus = torch.cuda.get_device_properties(DEV).multi_processor_count
     for B, V, want in ((cus, 16384, 1), (cus + 1, 16384, 2), (cus + 1, 16383, 1), (cus + 1, 8192, 1)):
-        step = penalised_step(s, B, V)
+        step, _ = penalised_step(s, B, V)
         step.launch()
         torch.cuda.synchronize()
         assert launches(step.launch) == want, (B, V)
+
+
+@pytest.mark.parametrize("kw,decided", [
+    ({}, True), ({"K": 1}, True), ({"K": 192}, True), ({"K": 193}, False),
+    # (bounds between powers of two, where values of one bin of a few key bits are many)
+    ({"mean": 20.0, "std": 1.0}, True), ({"mean": 20.0, "std": 1.0, "K": 192}, True), ({"mean": -40.0, "std": 1.0}, True),
+    ({"mean": 10.0, "std": 3.0, "K": 192}, True),
+    ({"repetition_penalty": 0.95}, False), ({"std": 0.0}, False),
+], ids=str)
+def test_the_rows_that_the_candidates_decide(kw, decided):
+    # (the first launch marks them, in the workspace's first words; the second leaves the marks)
+    s = SAMPLER.resolve("hip", BackendContext(DEV, torch.float32))
+    B, V = torch.cuda.get_device_properties(DEV).multi_processor_count + 8, 40000
+    print(f"rows the candidates decide {kw}", flush=True)
+    step, w = penalised_step(s, B, V, **kw)
+    step.launch()
+    torch.cuda.synchronize()
+    ws = step._keep[-1]
+    at = step._args.workspace - ws.data_ptr()
+    marks = ws[at:at + 4 * B].view(torch.int32)
+    assert bool((marks == -1).all()) == decided and bool((marks == -1).any()) == decided
+    few = slice(0, 8)
+    n = int(w.hist_offsets[8])
+    part = Workload("part", w.logits[few], PackedParams(**{f.name: getattr(w.params, f.name)[few] for f in fields(w.params)}), w.uniforms[few],
+                    w.hist_ids[:n], w.hist_offsets[:9], None)
+    _, bad = compare_ids(step.ids[few], oracle(part))
+    assert not bad, bad
