@@ -12,7 +12,7 @@ import pytest
 
 CSRC = Path(__file__).resolve().parents[1] / "vinfer_amd" / "csrc"
 BARRIERS = ("lds_barrier", "__syncthreads", "block_excl_scan", "block_sum", "block_max_u64", "sort_top", "sort_cands",
-            "sample_bound")
+            "sample_bound", "kth_key20")
 TOKEN = re.compile(r"\b(?P<barrier>" + "|".join(BARRIERS) + r")\s*[<(]"
                    r"|(?P<rmw>&)?\bsh\[(?P<word>[^\]]+)\](?P<store>\s*=(?!=))?"
                    r"|(?P<guard>\bif\s*\((?:tid < kWave|tid == 0|l == i)\))"
@@ -65,7 +65,7 @@ def conflicts(body: str) -> list[tuple[str, int]]:
 @pytest.mark.parametrize("name", ["sample.cuh", "logprobs.cuh"])
 def test_no_shared_word_is_read_and_written_between_two_barriers(name):
     seen = dict(functions((CSRC / name).read_text()))
-    assert {"sample.cuh": {"tile_row", "lowered_topk_row"}, "logprobs.cuh": {"lp_stream", "lp_one_pass"}}[name] <= set(seen)
+    assert {"sample.cuh": {"tile_row", "lowered_pass"}, "logprobs.cuh": {"lp_stream", "lp_one_pass"}}[name] <= set(seen)
     assert {f: c for f, b in seen.items() if (c := conflicts(b))} == {}
 
 

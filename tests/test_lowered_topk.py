@@ -152,6 +152,10 @@ def test_two_launches_only_past_one_row_a_cu_and_from_the_sample_on():
     # (bounds between powers of two, where values of one bin of a few key bits are many)
     ({"mean": 20.0, "std": 1.0}, True), ({"mean": 20.0, "std": 1.0, "K": 192}, True), ({"mean": -40.0, "std": 1.0}, True),
     ({"mean": 10.0, "std": 3.0, "K": 192}, True),
+    # (the best tokens penalised: fewer than K stay above the sample's bound, a second pass takes the bound that
+    # they give; pushed so far down that it would hold a third of the row, none does)
+    ({"history": 800, "best": 400, "presence_penalty": 1.0}, True),
+    ({"history": 800, "best": 400, "frequency_penalty": 3.0}, False),
     ({"repetition_penalty": 0.95}, False), ({"std": 0.0}, False),
 ], ids=str)
 def test_the_rows_that_the_candidates_decide(kw, decided):

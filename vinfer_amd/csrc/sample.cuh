@@ -1360,6 +1360,38 @@ __device__ __forceinline__ uint32_t top_sub8(const uint32_t* h8, uint32_t k, uin
   return __builtin_amdgcn_readlane(sub, L);
 }
 
+// The k-th largest of the workgroup's keys (of the threads with `count`, at least k of them) to 20 bits:
+// the lowest key with those bits, and how many keys reach it. Every thread calls, the result is the same
+// in all. `h`: kBoundWords zeroed words, `w` four words, both free afterwards.
+constexpr int kBoundWords = 4096 + 256;
+struct KthKey {
+  uint32_t key, reach;
+};
+__device__ __forceinline__ KthKey kth_key20(uint32_t* h, uint32_t key, bool count, uint32_t k, uint32_t* w) {
+  const int tid = threadIdx.x;
+  uint32_t* const h8 = h + 4096;
+  if (count) atomicAdd(&h[key >> 20], 1u);
+  lds_barrier();
+  if (tid < kWave) top_bin12(h, k, &w[0], &w[1]);
+  lds_barrier();
+  if (count && (key >> 20) == w[0]) atomicAdd(&h8[(key >> 12) & 255u], 1u);
+  lds_barrier();
+  if (tid < kWave) {
+    uint32_t reach;
+    const uint32_t sub = top_sub8(h8, k, w[1], &reach);
+    if (tid == 0) {
+      w[2] = (w[0] << 20) | (sub << 12);
+      w[3] = reach;
+    }
+  }
+  lds_barrier();
+  return KthKey{w[2], w[3]};
+}
+// Elements a thread that reach a bound, when `reach` of the threads' maxima do.
+__device__ __forceinline__ float elements_a_thread(uint32_t reach) {
+  return -__logf(1.0f - static_cast<float>(reach) * (1.0f / kThreads));
+}
+
 // ---- a bound on a row's largest elements from a sample -------------------------------------------
 // The rank, among the per-thread maxima of the first DEPTH stripes (16 elements each at DEPTH 2),
 // that about three times the n largest of the row lie above.
@@ -1368,35 +1400,16 @@ __device__ __forceinline__ uint32_t sample_rank(uint32_t n, int V) {
   constexpr u64 kSample = static_cast<u64>(DEPTH) * kThreads * kBlk;
   return static_cast<uint32_t>((3ull * n * kSample + static_cast<u64>(V) - 1) / static_cast<u64>(V)) + 2u;
 }
-// The value of that rank to 20 bits of its key (the lowest value with those bits), `mx` being the
-// calling thread's maximum; -inf where the row would have more than `cap` elements that reach it (ties:
-// as many as the maxima that do, a row of independent elements, tell). Every thread calls, the result
-// is the same in all. `h`: kBoundWords zeroed words, `w` three words, both free afterwards.
+// The value of that rank, or -inf where the row would have more than `cap` elements that reach it (ties:
+// as many as the maxima that do, a row of independent elements, tell); `mx` is the calling thread's
+// maximum, `h` and `w` as kth_key20's.
 // To 13 bits, as one scan of 8192 bins gave it, a bin of [16, 32) is 1 wide: at N(20, 1) and n = 50 most
 // rows of 151936 had more elements at its floor than can be staged, and were read for nothing.
-constexpr int kBoundWords = 4096 + 256;
 template <int DEPTH>
 __device__ __forceinline__ float sample_bound(uint32_t* h, float mx, uint32_t n, int V, uint32_t cap, uint32_t* w) {
-  const int tid = threadIdx.x;
-  uint32_t* const h8 = h + 4096;
-  const uint32_t key = key_of(mx);
-  const uint32_t m = sample_rank<DEPTH>(n, V);
-  atomicAdd(&h[key >> 20], 1u);
-  lds_barrier();
-  if (tid < kWave) top_bin12(h, m, &w[0], &w[1]);
-  lds_barrier();
-  if ((key >> 20) == w[0]) atomicAdd(&h8[(key >> 12) & 255u], 1u);
-  lds_barrier();
-  if (tid < kWave) {
-    uint32_t reach;
-    const uint32_t k32 = (w[0] << 20) | (top_sub8(h8, m, w[1], &reach) << 12);
-    // a share f of the threads' maxima reach it: about -ln(1 - f) elements a thread do
-    const float each = -__logf(1.0f - static_cast<float>(reach) * (1.0f / kThreads));
-    const bool fits = each * static_cast<float>(V) <= static_cast<float>(cap) * (DEPTH * kBlk);
-    if (tid == 0) w[2] = fits ? k32 : 0u;
-  }
-  lds_barrier();
-  return val_of(max(w[2], key_of(-INFINITY)));
+  const KthKey t = kth_key20(h, key_of(mx), true, sample_rank<DEPTH>(n, V), w);
+  const float fits = static_cast<float>(cap) * (DEPTH * kBlk) / static_cast<float>(V);
+  return elements_a_thread(t.reach) <= fits ? val_of(max(t.key, key_of(-INFINITY))) : -INFINITY;
 }
 
 // ---- top-k rows whose penalties only lower values ----------------------------------------------
@@ -1410,8 +1423,12 @@ __device__ __forceinline__ float sample_bound(uint32_t* h, float mx, uint32_t n,
 // value, ~30 us of a 62 us row at 16K ids -- and of the masked passes after it.
 // tau: the m-th largest of the first kLowDepth stripes' per-thread maxima to 20 bits, m three times the
 // K-th's share of that sample (penalised candidates may fall below tau).
-// Returns false, with nothing written, for a row it does not decide (too few or too many
-// candidates, a NaN or +inf, a threshold below tau): the caller runs the penalty pass.
+// Where fewer than K candidates stay >= tau (the row's best tokens are in its history), the K-th largest
+// of their penalised values is a bound that K tokens reach, and a second pass takes it for tau: rows whose
+// 300 best are there twice, top-k 50, 327 us for 1024 fp32 rows of 151936 when they were handed on (210
+// with the penalty pass alone), 205 now; 256 rows 82, 56 and 62; one bf16 row 90, 81 and 30.
+// Returns false, with nothing written, for a row it does not decide (too many candidates, a NaN or
+// +inf, a threshold below tau): the caller runs the penalty pass.
 // Measured (1024 fp32 rows of 151936, top-k 50, histories up to 32768): 255.0 -> 160.7 us in one
 // launch, 136.6 with two workgroups a CU (k_lowered).
 constexpr int kLowK = 192;       // top-k served
@@ -1443,17 +1460,14 @@ __device__ __forceinline__ void sort_top(const Cand* c, int n, u64* kk, Cand* ou
   lds_barrier();
 }
 
-template <class Tin>
-__device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, Row<Tin> row, const RowParams& p, GenericSmem& g,
-                                                 int r) {
+// One pass. FIRST: the bound from the sample; where too few candidates stay above it, `bound` is the key
+// of the next one (0: none worth a pass). Else the bound is `bound`.
+template <bool FIRST, class Tin>
+__device__ __forceinline__ bool lowered_pass(const SampleArgs& a, Row<Tin> row, const RowParams& p, GenericSmem& g, int r,
+                                             uint32_t& bound) {
   const int tid = threadIdx.x;
   const int V = row.V;
   const int L = p.h1 - p.h0;
-  // (uniform)
-  if (!(p.T > 0.0f) || p.K < 1 || p.K >= V || p.K > kLowK || L < 1 || a.out_probs) return false;
-  if (!(p.rep >= 1.0f && p.rep < INFINITY && p.pres >= 0.0f && p.freq >= 0.0f)) return false;
-  if (p.rep == 1.0f && p.pres == 0.0f && p.freq == 0.0f) return false;  // (no penalties: the generic path's own stream)
-  if (V < kLowVocab) return false;
   const uint32_t K = static_cast<uint32_t>(p.K);
   uint32_t* const bins = reinterpret_cast<uint32_t*>(&g) + kBitmapOffset;  // the sample's bins, then:
   uint32_t* const hkey = bins;                       // the hash table's ids
@@ -1469,24 +1483,29 @@ __device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, Row<Tin> r
   // [1] penalised candidates, [2] candidates, [3] a NaN or +inf, then the threshold (a word of its own for
   // each count: every thread decides by [2], so nothing may reset it before they all have)
   uint32_t* const sh = g.rdx.bk;
-  WholeBlock<Tin> q[kLowDepth];
-#pragma unroll
-  for (int k = 0; k < kLowDepth; ++k) q[k].load(row.p, k * kThreads + tid);
-  for (int i = tid; i < kBoundWords / 4; i += kThreads) reinterpret_cast<uint4*>(bins)[i] = make_uint4(0, 0, 0, 0);
-  if (tid < 4) sh[tid] = 0;
-  lds_barrier();
-  float v[kLowDepth][kBlk];
+  uint32_t* const w = reinterpret_cast<uint32_t*>(g.rdx.bq);  // [0, 4) kth_key20's, [4] maxima that reach a bound
+  float v[FIRST ? kLowDepth : 1][kBlk];
   float mx = -INFINITY;  // (IEEE maximum: a NaN stays)
+  float tau;
+  if constexpr (FIRST) {
+    WholeBlock<Tin> q[kLowDepth];
 #pragma unroll
-  for (int k = 0; k < kLowDepth; ++k) {
-    q[k].values(v[k]);
-    mx = __builtin_elementwise_maximum(mx, max_of8(v[k]));
-  }
-  const float tau = sample_bound<kLowDepth>(bins, mx, K, V, kLowCap, reinterpret_cast<uint32_t*>(g.rdx.bq));
-  if (!(tau > -INFINITY && tau < INFINITY)) return false;  // (uniform)
-  for (int i = tid; i < kLowSlots / 4; i += kThreads) {  // (the bins are dead; published after the pass)
-    reinterpret_cast<uint4*>(hkey)[i] = make_uint4(kEmpty, kEmpty, kEmpty, kEmpty);
-    reinterpret_cast<uint4*>(hcnt)[i] = make_uint4(0, 0, 0, 0);
+    for (int k = 0; k < kLowDepth; ++k) q[k].load(row.p, k * kThreads + tid);
+    for (int i = tid; i < kBoundWords / 4; i += kThreads) reinterpret_cast<uint4*>(bins)[i] = make_uint4(0, 0, 0, 0);
+    if (tid < 4) sh[tid] = 0;
+    if (tid == 4) w[4] = 0;
+    lds_barrier();
+#pragma unroll
+    for (int k = 0; k < kLowDepth; ++k) {
+      q[k].values(v[k]);
+      mx = __builtin_elementwise_maximum(mx, max_of8(v[k]));
+    }
+    tau = sample_bound<kLowDepth>(bins, mx, K, V, kLowCap, w);
+    if (!(tau > -INFINITY && tau < INFINITY)) return false;  // (uniform)
+  } else {
+    if (tid < 4) sh[tid] = 0;
+    tau = val_of(bound);
+    lds_barrier();
   }
   auto append = [&](float x, int id) {
     const bool c = x >= tau;
@@ -1499,36 +1518,44 @@ __device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, Row<Tin> r
       if (c && at < static_cast<uint32_t>(kLowCap)) stage[at] = Cand{x, id};
     }
   };
-  if (__ballot(!(mx < tau))) {
-#pragma unroll
-    for (int k = 0; k < kLowDepth; ++k)
-#pragma unroll
-      for (int i = 0; i < kBlk; ++i) append(v[k][i], (k * kThreads + tid) * kBlk + i);
+  const bool want_draft = p.draft >= 0 && p.draft < V && a.out_dprob;  // (uniform)
+  const bool drafts = want_draft && tid == kThreads - 1;
+  int32_t* const xid = reinterpret_cast<int32_t*>(g.rdx.hcnt) + 64;  // (past sorted_tail's results)
+  float* const xval = reinterpret_cast<float*>(xid + 1);
+  static_assert(kLowSlots == 1 << 12, "hash bits");
+  for (int i = tid; i < kLowSlots / 4; i += kThreads) {  // (the bins are dead; published after the pass)
+    reinterpret_cast<uint4*>(hkey)[i] = make_uint4(kEmpty, kEmpty, kEmpty, kEmpty);
+    reinterpret_cast<uint4*>(hcnt)[i] = make_uint4(0, 0, 0, 0);
   }
-  for_each_block_ahead(row, [&](const float (&w)[kBlk], uint32_t out, int b) {
+  if constexpr (FIRST) {
+    if (__ballot(!(mx < tau))) {
+#pragma unroll
+      for (int k = 0; k < kLowDepth; ++k)
+#pragma unroll
+        for (int i = 0; i < kBlk; ++i) append(v[k][i], (k * kThreads + tid) * kBlk + i);
+    }
+  }
+  for_each_block_ahead(row, [&](const float (&y)[kBlk], uint32_t out, int b) {
     float x[kBlk];
 #pragma unroll
-    for (int i = 0; i < kBlk; ++i) x[i] = out & (1u << i) ? -INFINITY : w[i];
+    for (int i = 0; i < kBlk; ++i) x[i] = out & (1u << i) ? -INFINITY : y[i];
     const float bx = max_of8(x);
     mx = __builtin_elementwise_maximum(mx, bx);
     if (__ballot(!(bx < tau))) {  // (uniform over the wave)
 #pragma unroll
       for (int i = 0; i < kBlk; ++i) append(x[i], b * kBlk + i);
     }
-  }, kLowDepth);
+  }, FIRST ? kLowDepth : 0);
   if (!(mx < INFINITY)) sh[3] = 1;
   lds_barrier();
   const uint32_t n0 = sh[2];
   if (sh[3] || n0 < K || n0 > static_cast<uint32_t>(kLowCap)) return false;  // (uniform)
   // the candidates' ids (and the draft's) into the table: thread t the t-th, the last thread the draft's
-  const bool want_draft = p.draft >= 0 && p.draft < V && a.out_dprob;  // (uniform)
   const bool mine = tid < static_cast<int>(n0);
-  const bool drafts = want_draft && tid == kThreads - 1;
   Cand me{0.0f, 0};
   if (mine) me = stage[tid];
   if (drafts) me = Cand{load_one<Tin>(row.p, p.draft), p.draft};
   uint32_t slot = (static_cast<uint32_t>(me.id) * 2654435761u) >> (32 - 12);
-  static_assert(kLowSlots == 1 << 12, "hash bits");
   if (mine || drafts) {
     // (at most 1024 of 4096 slots are taken: every probe sequence ends)
     while (true) {
@@ -1552,8 +1579,6 @@ __device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, Row<Tin> r
   });
   lds_barrier();
   // penalised values: the candidates' that stay >= tau, and the draft's (the row's only "exception")
-  int32_t* const xid = reinterpret_cast<int32_t*>(g.rdx.hcnt) + 64;  // (past sorted_tail's results)
-  float* const xval = reinterpret_cast<float*>(xid + 1);
   const int c = mine || drafts ? static_cast<int>(hcnt[slot]) : 0;
   lds_barrier();  // (every thread has its count: the candidates go over the table)
   const float xp = c > 0 ? apply_penalty(me.x, c, p.rep, p.pres, p.freq) : me.x;
@@ -1574,7 +1599,19 @@ __device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, Row<Tin> r
   }
   lds_barrier();
   const int n = static_cast<int>(sh[1]);
-  if (n < p.K) return false;  // (uniform)
+  if (n < p.K) {  // (uniform)
+    if constexpr (FIRST) {
+      // the K-th largest of the candidates' penalised values: K tokens reach it
+      for (int i = tid; i < kBoundWords / 4; i += kThreads) reinterpret_cast<uint4*>(bins)[i] = make_uint4(0, 0, 0, 0);
+      lds_barrier();
+      const uint32_t key = max(kth_key20(bins, key_of(xp), mine, K, w).key, key_of(-INFINITY));
+      const u64 reach = __ballot(mx >= val_of(key));  // (mx is by now the maximum of all of the thread's elements)
+      if (lane_id() == 0) atomicAdd(&w[4], static_cast<uint32_t>(__popcll(reach)));
+      lds_barrier();
+      if (key > key_of(-INFINITY) && elements_a_thread(w[4]) * kThreads <= static_cast<float>(kLowCap)) bound = key;
+    }
+    return false;
+  }
   sort_top(cand, n, kk, srt);
   const float T = p.T;
   const float mz = srt[0].x / T;
@@ -1602,6 +1639,23 @@ __device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, Row<Tin> r
   row.eval = xval;
   row.nexc = want_draft ? 1 : 0;
   return sorted_tail<false>(a, row, p, g, g.srch, srt, min(n, kSortCap), mz, k, r);
+}
+
+template <class Tin>
+__device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, const Row<Tin>& row, const RowParams& p,
+                                                 GenericSmem& g, int r) {
+  const int V = row.V;
+  const int L = p.h1 - p.h0;
+  // (uniform)
+  if (!(p.T > 0.0f) || p.K < 1 || p.K >= V || p.K > kLowK || L < 1 || a.out_probs) return false;
+  if (!(p.rep >= 1.0f && p.rep < INFINITY && p.pres >= 0.0f && p.freq >= 0.0f)) return false;
+  if (p.rep == 1.0f && p.pres == 0.0f && p.freq == 0.0f) return false;  // (no penalties: the generic path's own stream)
+  if (V < kLowVocab) return false;
+  uint32_t bound = 0;
+  if (lowered_pass<true>(a, row, p, g, r, bound)) return true;
+  if (bound == 0) return false;
+  lds_barrier();  // (every thread is done with its LDS)
+  return lowered_pass<false>(a, row, p, g, r, bound);
 }
 
 // have_bitmap: the penalty pass left the penalised ids' bitmap at kBitmapOffset.
@@ -3763,7 +3817,14 @@ __global__ __launch_bounds__(kThreads, 8) void k_lowered(SampleArgs a_) {
   const uint32_t pw = param_word<true>(a, r, tid < kParamWords ? tid : 0);
   if (tid < kParamWords) reinterpret_cast<uint32_t*>(&prm)[tid] = pw;
   lds_barrier();
-  RowParams p = prm;
+  // (in scalar registers: in vector ones the second pass's copies spilled, 115 -> 136 us)
+  struct Words {
+    uint32_t w[kParamWords];
+  };
+  Words words = __builtin_bit_cast(Words, prm);
+#pragma unroll
+  for (int i = 0; i < kParamWords; ++i) words.w[i] = __builtin_amdgcn_readfirstlane(words.w[i]);
+  RowParams p = __builtin_bit_cast(RowParams, words);
   p.u = p.u >= 0.0f ? p.u : 0.0f;
   Row<Tin> row;
   row.p = static_cast<const Tin*>(a.logits) + static_cast<int64_t>(r) * a.stride;
