@@ -90,3 +90,23 @@ def test_a_workspace_is_used_past_the_penalties_only_when_given_for_it(pen):
         torch.cuda.synchronize()
         assert torch.equal(out, want)
         assert bool((ws[at + kept:at + need] == 0xA5).all()) == (flag == 0)
+
+
+def test_a_call_makes_one_workspace():
+    # (the thread's kept workspace, which the draws use, neither grows nor is made for the probabilities)
+    s = SAMPLER.resolve("hip", BackendContext(DEV, torch.float32))
+    B, V = 3, 3000
+    g = torch.Generator(device=DEV).manual_seed(4)
+    logits = torch.randn(B, V, generator=g, device=DEV)
+    f = lambda v: torch.full((B,), v, device=DEV)  # noqa: E731
+    params = PackedParams(temperature=f(0.8), top_k=torch.zeros(B, dtype=torch.int32, device=DEV), top_p=f(0.9), min_p=f(0.0),
+                          repetition_penalty=f(1.1), presence_penalty=f(0.5), frequency_penalty=f(0.2))
+    kept = s._local.__dict__.get("workspaces", {}).get(DEV)
+    most = 0 if kept is None else kept.numel() // 12
+    off = torch.arange(0, 3 * (most + 4000) + 1, most + 4000, dtype=torch.int32, device=DEV)
+    ids = torch.randint(0, V, (int(off[-1]),), generator=g, device=DEV).to(torch.int32)
+    got = s.probs(logits, params, ids, off)
+    torch.cuda.synchronize()
+    after = s._local.__dict__.get("workspaces", {}).get(DEV)
+    assert after is kept
+    assert torch.equal(got, one_launch(s, logits, params, ids, off))

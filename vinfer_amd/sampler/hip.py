@@ -82,7 +82,7 @@ class HipSampler:
         return t.contiguous()
 
     def _args(self, logits, params, hist_ids, hist_offsets, uniforms=None, draft_ids=None, param_rows=None,
-              append_history=False):
+              append_history=False, own_workspace=False):
         dev = self._device(logits)
         B, V = logits.shape
         P = B if param_rows is None else param_rows  # parameter entries (verify: one per sequence)
@@ -139,6 +139,8 @@ class HipSampler:
         if draft_ids is not None:
             draft_ids = self._vec(draft_ids, B, torch.int32, dev, "draft_ids")
             a.draft_ids = _ptr(draft_ids)
+        if own_workspace:  # (the caller makes the call's)
+            return a, (logits, cols, hist_ids, hist_offsets, uniforms, draft_ids)
         # (histories' penalty lists and, with split rows, the slices' records)
         ws_bytes = self._lib.vsamp_split_workspace_bytes if self.split_rows else self._lib.vsamp_workspace_bytes
         need = int(ws_bytes(B, V, hist_total))
@@ -208,7 +210,7 @@ class HipSampler:
                 and B * ((_n_tiles(V) + 63) // 64) <= _TILE_FUSED_WORKGROUPS)
 
     def probs(self, logits, params, hist_ids=None, hist_offsets=None):
-        a, keep = self._args(logits, params, hist_ids, hist_offsets)
+        a, keep = self._args(logits, params, hist_ids, hist_offsets, own_workspace=True)
         B, V = logits.shape
         out = torch.empty(B, V, dtype=torch.float32, device=logits.device)
         # (the call's own workspace: the rows' states live in it between its two launches)
