@@ -176,3 +176,32 @@ def test_the_rows_that_the_candidates_decide(kw, decided):
                     w.hist_ids[:n], w.hist_offsets[:9], None)
     _, bad = compare_ids(step.ids[few], oracle(part))
     assert not bad, bad
+
+
+def test_history_append_where_the_rows_take_two_launches():
+    # per-row ranges with a spare entry each, rows of the first launch and rows of the second: the draws are those
+    # of the same call without append, each drawn id lands behind its row's range, nothing else is written
+    s = SAMPLER.resolve("hip", BackendContext(DEV, torch.float32))
+    B, V, room = torch.cuda.get_device_properties(DEV).multi_processor_count + 5, 17000, 260
+    g = torch.Generator(device=DEV).manual_seed(11)
+    x = torch.randn(B, V, generator=g, device=DEV) * 2.5
+    x[7, 100] = math.nan
+    hist = torch.randint(0, V, (B * room,), generator=g, device=DEV).to(torch.int32)
+    start = torch.randperm(B, generator=g, device=DEV) * room  # (the rows' regions in any order)
+    length = torch.arange(B, device=DEV) % room  # 0 .. room - 1
+    off = torch.stack([start, start + length], 1).to(torch.int32)
+    p = pack_params([SamplingParams(temperature=(0.8, 0.0, 1.1)[b % 3], top_k=(50, 192, 400, 0)[b % 4], top_p=0.9,
+                                    repetition_penalty=(1.1, 0.95)[b % 7 == 0], presence_penalty=0.3, frequency_penalty=0.1)
+                     for b in range(B)]).to(DEV)
+    u = torch.rand(B, generator=g, device=DEV)
+    want, _ = s.sample_batch(x, p, u, hist.clone(), off)
+    step = s.prepare_batch(x, p, u, grown := hist.clone(), off, append_history=True)
+    step.launch()
+    torch.cuda.synchronize()
+    ws = step._keep[-1]
+    at = step._args.workspace - ws.data_ptr()
+    decided = ws[at:at + 4 * B].view(torch.int32) == -1
+    assert 20 < int(decided.sum()) < B - 20
+    assert torch.equal(step.ids, want)
+    hist[(start + length).long()] = want
+    assert torch.equal(grown, hist)

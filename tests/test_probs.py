@@ -110,3 +110,29 @@ def test_a_call_makes_one_workspace():
     after = s._local.__dict__.get("workspaces", {}).get(DEV)
     assert after is kept
     assert torch.equal(got, one_launch(s, logits, params, ids, off))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=str)
+@pytest.mark.parametrize("V,pad", [(2049, 1), (4096, 7), (10007, 64)])
+def test_two_launches_write_strided_rows_and_nothing_between(V, pad, dtype):
+    s = SAMPLER.resolve("hip", BackendContext(DEV, dtype))
+    B = 6
+    g = torch.Generator(device=DEV).manual_seed(V)
+    logits = (torch.randn(B, V, generator=g, device=DEV) * 3.0).to(dtype)
+    f = lambda v: torch.full((B,), v, device=DEV)  # noqa: E731
+    params = PackedParams(temperature=f(0.8), top_k=torch.zeros(B, dtype=torch.int32, device=DEV), top_p=f(0.9), min_p=f(0.0),
+                          repetition_penalty=f(1.1), presence_penalty=f(0.5), frequency_penalty=f(0.2))
+    off = torch.arange(0, 40 * B + 1, 40, dtype=torch.int32, device=DEV)
+    ids = torch.randint(0, V, (40 * B,), generator=g, device=DEV).to(torch.int32)
+    want = one_launch(s, logits, params, ids, off)
+    a, keep = s._args(logits, params, ids, off, own_workspace=True)
+    need = int(s._lib.vsamp_probs_workspace_bytes(B, V, a.hist_total))
+    ws = torch.empty(need + 256, dtype=torch.uint8, device=DEV)
+    a.workspace, a.workspace_bytes = (ws.data_ptr() + 255) & ~255, need
+    a.flags |= _lib.VSAMP_PROBS_STATES
+    out = torch.full((B, V + pad), -7.0, device=DEV)
+    print(f"probs stride V={V} pad={pad} {dtype}", flush=True)
+    _lib.check(s._lib.vsamp_probs(ctypes.byref(a), out.data_ptr(), V + pad, s._stream(DEV)))
+    torch.cuda.synchronize()
+    assert torch.equal(out[:, :V], want)
+    assert bool((out[:, V:] == -7.0).all())
