@@ -2,6 +2,8 @@
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import torch
 
@@ -46,3 +48,14 @@ def compare_ids(ids: torch.Tensor, res, dprob: torch.Tensor | None = None, rtol:
             if abs(dp[b] - want) > rtol * abs(want) + 1e-30:
                 bad.append((b, "draft_prob", dp[b], want))
     return ties, bad
+
+
+def launches(fn) -> int:
+    """Kernels of one call, from a captured graph (which is not run)."""
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g):
+        fn()
+    n = ctypes.c_size_t()
+    hip = ctypes.CDLL("libamdhip64.so")
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    return n.value

@@ -4,7 +4,6 @@ oracle, at the sizes and parameters where the route changes."""
 
 from __future__ import annotations
 
-import ctypes
 import math
 from dataclasses import fields
 
@@ -12,7 +11,7 @@ import numpy as np
 import pytest
 import torch
 
-from tests.parity import compare_ids, oracle
+from tests.parity import compare_ids, launches, oracle
 from vinfer_amd.registry import BackendContext
 from vinfer_amd.sampler import SAMPLER
 from vinfer_amd.sampling import PackedParams, SamplingParams, pack_history, pack_params
@@ -109,17 +108,6 @@ def test_more_fp32_rows_than_cus_equal_smaller_batches(V):
         torch.cuda.synchronize()
         assert torch.equal(got[0], torch.cat([p[0] for p in parts]))
         assert torch.equal(got[1], torch.cat([p[1] for p in parts]))
-
-
-def launches(fn) -> int:
-    """Kernels of one call, from a captured graph (which is not run)."""
-    g = torch.cuda.CUDAGraph(keep_graph=True)
-    with torch.cuda.graph(g):
-        fn()
-    n = ctypes.c_size_t()
-    hip = ctypes.CDLL("libamdhip64.so")
-    assert hip.hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n)) == 0
-    return n.value
 
 
 def penalised_step(s, B, V, mean=0.0, std=2.0, K=50, history=300, best=0, seed=0, **kw):

@@ -8,6 +8,7 @@ import ctypes
 import pytest
 import torch
 
+from tests.parity import launches
 from vinfer_amd import _lib
 from vinfer_amd.registry import BackendContext
 from vinfer_amd.sampler import SAMPLER
@@ -30,10 +31,12 @@ def one_launch(s, logits, params, hist_ids, hist_offsets):
 
 
 # (2048 ids a workgroup of the second launch: one short of a tile, one tile, one past it, a large and an odd
-# vocabulary; `offset` moves the rows off 16-byte alignment)
+# vocabulary, rows on both sides of the 8192 ids from which there are two launches; `offset` moves the rows off
+# 16-byte alignment)
 @pytest.mark.parametrize("pen", [False, True], ids=["plain", "penalties"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=str)
-@pytest.mark.parametrize("V,offset", [(1, 0), (2047, 0), (2048, 0), (2049, 1), (50257, 0), (151936, 0), (151936, 3)])
+@pytest.mark.parametrize("V,offset", [(1, 0), (2047, 0), (2048, 0), (2049, 1), (50257, 0), (151936, 0), (151936, 3),
+                                      (8192, 0), (8193, 0), (10239, 0), (10240, 0), (10241, 1)])
 def test_two_launches_equal_one(V, offset, dtype, pen):
     s = SAMPLER.resolve("hip", BackendContext(DEV, dtype))
     g = torch.Generator(device=DEV).manual_seed(V + offset)
@@ -95,7 +98,7 @@ def test_a_workspace_is_used_past_the_penalties_only_when_given_for_it(pen):
 def test_a_call_makes_one_workspace():
     # (the thread's kept workspace, which the draws use, neither grows nor is made for the probabilities)
     s = SAMPLER.resolve("hip", BackendContext(DEV, torch.float32))
-    B, V = 3, 3000
+    B, V = 3, 9000
     g = torch.Generator(device=DEV).manual_seed(4)
     logits = torch.randn(B, V, generator=g, device=DEV)
     f = lambda v: torch.full((B,), v, device=DEV)  # noqa: E731
@@ -113,7 +116,7 @@ def test_a_call_makes_one_workspace():
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=str)
-@pytest.mark.parametrize("V,pad", [(2049, 1), (4096, 7), (10007, 64)])
+@pytest.mark.parametrize("V,pad", [(8193, 1), (10240, 7), (10007, 64)])
 def test_two_launches_write_strided_rows_and_nothing_between(V, pad, dtype):
     s = SAMPLER.resolve("hip", BackendContext(DEV, dtype))
     B = 6
@@ -136,3 +139,15 @@ def test_two_launches_write_strided_rows_and_nothing_between(V, pad, dtype):
     torch.cuda.synchronize()
     assert torch.equal(out[:, :V], want)
     assert bool((out[:, V:] == -7.0).all())
+
+
+@pytest.mark.parametrize("V,want", [(1, 1), (2000, 1), (8192, 1), (8193, 2)])
+def test_short_rows_take_one_launch(V, want):
+    s = SAMPLER.resolve("hip", BackendContext(DEV, torch.bfloat16))
+    logits = torch.randn(2, V, device=DEV).to(torch.bfloat16)
+    f = lambda v: torch.full((2,), v, device=DEV)  # noqa: E731
+    params = PackedParams(temperature=f(0.8), top_k=torch.zeros(2, dtype=torch.int32, device=DEV), top_p=f(0.9), min_p=f(0.0),
+                          repetition_penalty=f(1.0), presence_penalty=f(0.0), frequency_penalty=f(0.0))
+    s.probs(logits, params)
+    torch.cuda.synchronize()
+    assert launches(lambda: s.probs(logits, params)) == want

@@ -383,18 +383,23 @@ int run_tile_pass(const vsamp_args* a, float* tile_max, uint32_t* arrive, hipStr
 
 // The probabilities' two launches keep the rows' states after the penalty part of the workspace.
 size_t probs_states(int64_t B, int64_t V, int64_t H) { return align_up(layout(B, V, H).total); }
+// Rows of one stripe or less are written from their own workgroup as fast as a second launch starts: 1 row of
+// 2000 11.2 us a call in one launch and 15.5 in two, 32 rows of 4000 14.8 and 16.5, of 8000 17.5 and 16.9, one
+// of 16000 21.3 and 16.7.
+bool probs_two(int64_t B, int64_t V) { return V > vs::kThreads * vs::kBlk && B <= 65535; }
 size_t probs_total(int64_t B, int64_t V, int64_t H) {
-  return probs_states(B, V, H) + sizeof(vs::RowState) * static_cast<size_t>(B);
+  return probs_two(B, V) ? probs_states(B, V, H) + sizeof(vs::RowState) * static_cast<size_t>(B) : layout(B, V, H).total;
 }
 
-// Probabilities: where the caller gives a workspace for the row states (VSAMP_PROBS_STATES: a call
-// without histories may otherwise share its workspace with others), the states' launch and a launch
-// that writes the rows over the whole chip (32 bf16 rows of 151936: 104.8 -> 32.3 us); otherwise one
-// launch, each row written by its own workgroup.
+// Probabilities: rows past a stripe, where the caller gives a workspace for the row states
+// (VSAMP_PROBS_STATES: a call without histories may otherwise share its workspace with others), the
+// states' launch and a launch that writes the rows over the whole chip (32 bf16 rows of 151936: 104.8 ->
+// 32.3 us); otherwise one launch, each row written by its own workgroup.
 template <class Tin>
 int run_probs(const vsamp_args* a, float* out, int64_t out_stride, hipStream_t st) {
-  if (!(a->flags & VSAMP_PROBS_STATES) || !a->workspace || (reinterpret_cast<uintptr_t>(a->workspace) & 255u) ||
-      a->workspace_bytes < probs_total(a->batch, a->vocab, a->hist_total) || a->batch > 65535)
+  if (!(a->flags & VSAMP_PROBS_STATES) || !probs_two(a->batch, a->vocab) || !a->workspace ||
+      (reinterpret_cast<uintptr_t>(a->workspace) & 255u) ||
+      a->workspace_bytes < probs_total(a->batch, a->vocab, a->hist_total))
     return run_sample<Tin>(a, out, out_stride, st);
   char* w = static_cast<char*>(a->workspace);
   vs::RowState* states = reinterpret_cast<vs::RowState*>(w + probs_states(a->batch, a->vocab, a->hist_total));

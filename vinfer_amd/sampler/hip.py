@@ -210,14 +210,15 @@ class HipSampler:
                 and B * ((_n_tiles(V) + 63) // 64) <= _TILE_FUSED_WORKGROUPS)
 
     def probs(self, logits, params, hist_ids=None, hist_offsets=None):
-        a, keep = self._args(logits, params, hist_ids, hist_offsets, own_workspace=True)
+        two = logits.dim() == 2 and logits.shape[1] > _PROBS_ONE_LAUNCH
+        a, keep = self._args(logits, params, hist_ids, hist_offsets, own_workspace=two)
         B, V = logits.shape
         out = torch.empty(B, V, dtype=torch.float32, device=logits.device)
-        # (the call's own workspace: the rows' states live in it between its two launches)
-        a.flags |= _lib.VSAMP_PROBS_STATES
-        a.workspace_bytes = int(self._lib.vsamp_probs_workspace_bytes(B, V, a.hist_total))
-        ws = torch.empty(a.workspace_bytes + 256, dtype=torch.uint8, device=logits.device)
-        a.workspace = (ws.data_ptr() + 255) & ~255
+        if two:  # (the call's own workspace: the rows' states live in it between its two launches)
+            a.flags |= _lib.VSAMP_PROBS_STATES
+            a.workspace_bytes = int(self._lib.vsamp_probs_workspace_bytes(B, V, a.hist_total))
+            ws = torch.empty(a.workspace_bytes + 256, dtype=torch.uint8, device=logits.device)
+            a.workspace = (ws.data_ptr() + 255) & ~255
         _lib.check(self._lib.vsamp_probs(ctypes.byref(a), out.data_ptr(), V, self._stream(logits.device)))
         del keep
         return out
@@ -634,6 +635,7 @@ def _n_tiles(V: int) -> int:
 # batches up to this many workgroups (rows times workgroups per row) take the tile pass in one
 # launch (the library's rule)
 _TILE_FUSED_WORKGROUPS = 256
+_PROBS_ONE_LAUNCH = 8192  # (probs: one launch up to this vocabulary, the library's rule)
 _LM_OWN_ROWS = 64  # (lm_head: the library GEMM and vsamp_tile_stats above this many rows)
 
 # the per-token call's parameter words: temperature, top_p, min_p, the three penalties (fp32),
