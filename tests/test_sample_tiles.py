@@ -431,3 +431,28 @@ def test_gpu_tile_pass_top_k_up_to_the_list(dtype):
         b, bp = row_passes(s, logits, pp, u, None, None, draft)
         torch.cuda.synchronize()
         assert torch.equal(a, b) and torch.equal(ap, bp), label
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=str)
+def test_gpu_tile_pass_min_p_around_what_the_list_holds(dtype):
+    # rows with c tokens above min-p, in tiles of their own or all in one run: as many tiles as are read at a time
+    # (64), as tell that the list's 256 tokens would not do, as the list holds and one more, and past 256 tiles
+    s = hip()
+    V = 151936
+    counts = [1, 63, 64, 65, 128, 200, 229, 230, 240, 255, 256, 257, 300, 1000]
+    g = torch.Generator(device=DEV).manual_seed(6)
+    for label in ("apart", "one run"):
+        x = torch.randn(len(counts), V, generator=g, device=DEV) - 20.0
+        for r, c in enumerate(counts):
+            at = torch.randperm(V // 128, generator=g, device=DEV)[:c] * 128 + r if label == "apart" else torch.arange(c, device=DEV)
+            x[r, at] = 5.0 + torch.rand(c, generator=g, device=DEV)
+        logits = x.to(dtype)
+        pp = pack_params([SamplingParams(temperature=1.0, min_p=0.2, top_p=0.97)] * len(counts)).to(DEV)
+        u = torch.rand(len(counts), generator=g, device=DEV)
+        draft = logits.float().argmax(dim=1).to(torch.int32)
+        print(f"tile pass min-p {label} {dtype}", flush=True)
+        a, ap = s.sample_tile_pass(logits, pp, u, None, None, draft)
+        b, bp = row_passes(s, logits, pp, u, None, None, draft)
+        torch.cuda.synchronize()
+        assert torch.equal(a, b) and torch.equal(ap, bp), label
