@@ -711,10 +711,15 @@ int vsamp_logprobs(const vsamp_args* a, const int32_t* tokens, int32_t n_top, fl
   l.out_top_ids = out_top_ids;
   l.out_top = out_top_logprobs;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (a->dtype == VSAMP_BF16)
-    hipLaunchKernelGGL(vs::k_logprobs<uint16_t>, dim3(a->batch), dim3(vs::kThreads), 0, st, l);
+  const bool streamed = l.V >= vs::kLpVocab;
+  if (a->dtype == VSAMP_BF16 && streamed)
+    hipLaunchKernelGGL((vs::k_logprobs<uint16_t, false, true>), dim3(a->batch), dim3(vs::kThreads), 0, st, l);
+  else if (a->dtype == VSAMP_BF16)
+    hipLaunchKernelGGL((vs::k_logprobs<uint16_t, false>), dim3(a->batch), dim3(vs::kThreads), 0, st, l);
+  else if (streamed)
+    hipLaunchKernelGGL((vs::k_logprobs<float, false, true>), dim3(a->batch), dim3(vs::kThreads), 0, st, l);
   else
-    hipLaunchKernelGGL(vs::k_logprobs<float>, dim3(a->batch), dim3(vs::kThreads), 0, st, l);
+    hipLaunchKernelGGL((vs::k_logprobs<float, false>), dim3(a->batch), dim3(vs::kThreads), 0, st, l);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? VSAMP_OK : hip_fail(e, "launch k_logprobs");
 }

@@ -206,6 +206,7 @@ __device__ __forceinline__ bool lp_one_pass(const LogprobArgs& a, const Row<uint
 // time).
 constexpr int kLpCap = 1023;
 constexpr int kLpDepth = 2;
+constexpr int kLpVocab = kLpDepth * kThreads * kBlk;  // the shortest row served: the sample
 constexpr int kLpBins = 8192;
 constexpr int kLpWords = kLpBins + 2 * (kLpCap + 1);  // LDS words: bins (then sort keys and list), staged elements
 template <class Tin>
@@ -214,7 +215,6 @@ __device__ __forceinline__ bool lp_stream(const LogprobArgs& a, const Row<Tin>& 
   const int tid = threadIdx.x;
   const int V = row.V;
   const int n = a.n_top;
-  if (V / kBlk / kThreads < kLpDepth) return false;  // (uniform)
   Cand* const stage = reinterpret_cast<Cand*>(area + kLpBins);
   WholeBlock<Tin> q[kLpDepth];
 #pragma unroll
@@ -300,11 +300,13 @@ __device__ __forceinline__ bool lp_stream(const LogprobArgs& a, const Row<Tin>& 
   return true;
 }
 
-template <class Tin, bool TILES = false>
+// STREAM: rows of at least kLpVocab, lp_stream first. (A launch of its own for the others: with lp_stream's
+// code in it too, jumped over, 64 fp32 rows of 7000 took 18.6 us, 17.5 without.)
+template <class Tin, bool TILES, bool STREAM = false>
 __global__ __launch_bounds__(kThreads) void k_logprobs(LogprobArgs a) {
   constexpr int kBins = 8192;  // by the top 13 bits of the ordered key
   constexpr bool kOnePass = sizeof(Tin) == 2 && !TILES;  // (bf16 rows: one pass over a 16-bit histogram)
-  __shared__ __align__(16) uint32_t h13[kOnePass ? 32768 : TILES ? kBins : kLpWords];  // (then the candidate list: kCandCap 8-byte entries)
+  __shared__ __align__(16) uint32_t h13[kOnePass ? 32768 : STREAM ? kLpWords : kBins];  // (then the candidate list: kCandCap 8-byte entries)
   __shared__ Radix rdx;
   __shared__ Search srch;
   __shared__ Cand top[kMaxTop];
@@ -322,8 +324,8 @@ __global__ __launch_bounds__(kThreads) void k_logprobs(LogprobArgs a) {
   row.eval = nullptr;
   row.nexc = 0;
   const int n = a.n_top;
-  exp_table_init();  // (published by the first barrier below)
-  if constexpr (!TILES) {
+  if constexpr (TILES || STREAM) exp_table_init();  // (published by the first barrier below)
+  if constexpr (STREAM) {
     if (lp_stream<Tin>(a, row, r, h13, sh, rdx.bk, srch.red64)) return;  // (uniform)
     __syncthreads();  // (every thread is done with its LDS)
   }
