@@ -144,6 +144,9 @@ def test_two_launches_only_past_one_row_a_cu_and_from_the_sample_on():
     # they give; pushed so far down that it would hold a third of the row, none does)
     ({"history": 800, "best": 400, "presence_penalty": 1.0}, True),
     ({"history": 800, "best": 400, "frequency_penalty": 3.0}, False),
+    # (greedy rows: the largest penalised value, the best tokens penalised or not)
+    ({"temperature": 0.0, "K": 0}, True), ({"temperature": 0.0, "history": 800, "best": 400}, True),
+    ({"temperature": 0.0, "repetition_penalty": 0.95}, False), ({"K": 0}, False),
     ({"repetition_penalty": 0.95}, False), ({"std": 0.0}, False),
 ], ids=str)
 def test_the_rows_that_the_candidates_decide(kw, decided):

@@ -1412,10 +1412,11 @@ __device__ __forceinline__ float sample_bound(uint32_t* h, float mx, uint32_t n,
   return elements_a_thread(t.reach) <= fits ? val_of(max(t.key, key_of(-INFINITY))) : -INFINITY;
 }
 
-// ---- top-k rows whose penalties only lower values ----------------------------------------------
+// ---- top-k and greedy rows whose penalties only lower values ------------------------------------
 // With rep >= 1, pres >= 0 and freq >= 0 no penalised value is above its original (each step of
 // apply_penalty rounds a value no larger). So every token whose penalised value reaches a bound
-// tau has an original value that does, and a top-k row needs the counts of those few tokens alone:
+// tau has an original value that does, and a top-k row (a greedy one as of K = 1) needs the counts of
+// those few tokens alone:
 // one pass over the row stages the elements >= tau, their ids go into an LDS hash table, one pass
 // over the history counts the ids it holds, and the candidates' penalised values >= tau, when at
 // least K of them, hold the top K (and the row's max). In place of the penalty pass -- the whole
@@ -1468,7 +1469,8 @@ __device__ __forceinline__ bool lowered_pass(const SampleArgs& a, Row<Tin> row, 
   const int tid = threadIdx.x;
   const int V = row.V;
   const int L = p.h1 - p.h0;
-  const uint32_t K = static_cast<uint32_t>(p.K);
+  const bool greedy = !(p.T > 0.0f);  // (the largest penalised value's first id)
+  const uint32_t K = greedy ? 1u : static_cast<uint32_t>(p.K);
   uint32_t* const bins = reinterpret_cast<uint32_t*>(&g) + kBitmapOffset;  // the sample's bins, then:
   uint32_t* const hkey = bins;                       // the hash table's ids
   uint32_t* const hcnt = hkey + kLowSlots;           // and counts, then:
@@ -1599,7 +1601,7 @@ __device__ __forceinline__ bool lowered_pass(const SampleArgs& a, Row<Tin> row, 
   }
   lds_barrier();
   const int n = static_cast<int>(sh[1]);
-  if (n < p.K) {  // (uniform)
+  if (n < static_cast<int>(K)) {  // (uniform)
     if constexpr (FIRST) {
       // the K-th largest of the candidates' penalised values: K tokens reach it
       for (int i = tid; i < kBoundWords / 4; i += kThreads) reinterpret_cast<uint4*>(bins)[i] = make_uint4(0, 0, 0, 0);
@@ -1613,6 +1615,12 @@ __device__ __forceinline__ bool lowered_pass(const SampleArgs& a, Row<Tin> row, 
     return false;
   }
   sort_top(cand, n, kk, srt);
+  Kept k;
+  if (greedy) {  // (uniform)
+    k.point = srt[0].id;
+    finish<false>(a, row, p, 0.0f, k, 0, &g.srch.vslot, r);
+    return true;
+  }
   const float T = p.T;
   const float mz = srt[0].x / T;
   if (!(mz > -INFINITY && mz < INFINITY)) return false;  // (uniform) point rows
@@ -1631,7 +1639,6 @@ __device__ __forceinline__ bool lowered_pass(const SampleArgs& a, Row<Tin> row, 
     if (tid == 0) reinterpret_cast<float*>(sh)[3] = x0;
   }
   lds_barrier();
-  Kept k;
   k.x0 = reinterpret_cast<const float*>(sh)[3];
   // every element >= x0 must be in the sorted list
   if (!(k.x0 >= tau) || (n > kSortCap && srt[kSortCap - 1].x >= k.x0)) return false;  // (uniform)
@@ -1647,7 +1654,7 @@ __device__ __forceinline__ bool lowered_topk_row(const SampleArgs& a, const Row<
   const int V = row.V;
   const int L = p.h1 - p.h0;
   // (uniform)
-  if (!(p.T > 0.0f) || p.K < 1 || p.K >= V || p.K > kLowK || L < 1 || a.out_probs) return false;
+  if (L < 1 || a.out_probs || (p.T > 0.0f && (p.K < 1 || p.K >= V || p.K > kLowK))) return false;
   if (!(p.rep >= 1.0f && p.rep < INFINITY && p.pres >= 0.0f && p.freq >= 0.0f)) return false;
   if (p.rep == 1.0f && p.pres == 0.0f && p.freq == 0.0f) return false;  // (no penalties: the generic path's own stream)
   if (V < kLowVocab) return false;
