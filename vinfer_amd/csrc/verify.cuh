@@ -136,16 +136,17 @@ struct ResidualSide {
 template <class Tin>
 __device__ __forceinline__ bool accepts(const VerifyArgs& a, int b, int j) {
   const int K = a.K;
+  // (no branch on the token, so that the states' loads do not wait for it; the logits' do)
   const int d = a.drafts[b * K + j];
-  if (d < 0 || d >= a.V) return false;  // a token outside the vocabulary is never accepted
   const RowState st = a.ts[b * (K + 1) + j];
   const RowState sd = a.ds[b * K + j];
-  const float xt = load_one<Tin>(static_cast<const Tin*>(a.tgt) + static_cast<int64_t>(b * (K + 1) + j) * a.tstride, d);
-  const float xd = load_one<Tin>(static_cast<const Tin*>(a.drf) + static_cast<int64_t>(b * K + j) * a.dstride, d);
+  const int at = d < 0 ? 0 : (d < a.V ? d : a.V - 1);
+  const float xt = load_one<Tin>(static_cast<const Tin*>(a.tgt) + static_cast<int64_t>(b * (K + 1) + j) * a.tstride, at);
+  const float xd = load_one<Tin>(static_cast<const Tin*>(a.drf) + static_cast<int64_t>(b * K + j) * a.dstride, at);
   const u64 P = token_mass(xt, d, st), Q = token_mass(xd, d, sd);
   const u128 lhs = static_cast<u128>(u24(a.u_acc[b * K + j])) * Q * kept_mass(st);  // < 2^127
   const u128 rhs = (static_cast<u128>(P) * kept_mass(sd)) << 24;
-  return lhs < rhs;
+  return (d == at) & (lhs < rhs);  // (a token outside the vocabulary is never accepted)
 }
 
 // One workgroup, a thread per sequence: the acceptance chain. Writes the accepted drafts and, when
