@@ -265,8 +265,8 @@ int vsamp_logprobs_tiles(const vsamp_args* args, const float* tile_max, const fl
  * decided from a few tiles instead of a pass over the row: greedy rows (the first max lies in
  * the first tile whose max is the row max) and rows sampled with top-k <= 256 or min-p (every
  * kept token lies in a tile whose max reaches a bound taken from the maxima), without
- * penalties. Every other row (penalties, top-p alone, NaN or infinite rows, more than 64
- * candidate tiles or 256 candidate tokens) takes vsamp_sample's row passes in the same launch.
+ * penalties. Every other row (penalties, top-p alone, NaN or infinite rows, more than 256
+ * candidate tiles or candidate tokens) takes vsamp_sample's row passes in the same launch.
  * Replaces the sampler call after the engine's LM head (models/qwen/model.py:230-233 ->
  * runtime/sampler.py:68-77) when the LM head is vsamp_lm_head. */
 int vsamp_sample_tiles(const vsamp_args* args, const float* tile_max, void* stream);

@@ -202,8 +202,7 @@ __device__ __forceinline__ bool lp_one_pass(const LogprobArgs& a, const Row<uint
 // A histogram's LDS atomic an element (about 9 clocks a wave) and a thread's three largest kept
 // an element bound the pass below it; this one is bound by the reads and the exponentials.
 // Measured (256 bf16 rows of 151936, top 20, half certain and half flat): 27-52 us a call with
-// lp_one_pass, by how many rows' lists were complete, 25.3-28.5 for all of them now (12.5 of it SIMD
-// time).
+// lp_one_pass, by how many rows' lists were complete, 24.1 for all of them now (12.5 of it SIMD time).
 constexpr int kLpCap = 1023;
 constexpr int kLpDepth = 2;
 constexpr int kLpVocab = kLpDepth * kThreads * kBlk;  // the shortest row served: the sample

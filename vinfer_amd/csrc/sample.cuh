@@ -1430,8 +1430,8 @@ __device__ __forceinline__ float sample_bound(uint32_t* h, float mx, uint32_t n,
 // with the penalty pass alone), 205 now; 256 rows 82, 56 and 62; one bf16 row 90, 81 and 30.
 // Returns false, with nothing written, for a row it does not decide (too many candidates, a NaN or
 // +inf, a threshold below tau): the caller runs the penalty pass.
-// Measured (1024 fp32 rows of 151936, top-k 50, histories up to 32768): 255.0 -> 160.7 us in one
-// launch, 136.6 with two workgroups a CU (k_lowered).
+// Measured (1024 fp32 rows of 151936, top-k 50, histories up to 32768): 248.2 us through the penalty
+// pass, 133.8 in k_lowered's launches.
 constexpr int kLowK = 192;       // top-k served
 constexpr int kLowDepth = 2;     // stripes sampled
 constexpr int kLowVocab = kLowDepth * kThreads * kBlk;  // the shortest row served: the sample
@@ -3288,9 +3288,9 @@ __device__ __forceinline__ bool fast_row(const SampleArgs& a, Row<uint16_t> row,
 //     row max (as values: -0 equals +0), and only that tile is read;
 //   * rows sampled at T > 0 with top-k (K <= kSortCap) or min-p: every kept token has
 //     x >= xlo, where for top-k xlo is the least x with fl(x / T) >= fl(theta / T), theta the
-//     K-th largest tile max to 20 bits of its key, exactly it for bf16 (the K largest tile maxima
-//     are K logits, so theta is at most the K-th largest logit, whose z every kept token
-//     reaches), and for min-p the least x whose p~ = exp(fl(x / T) - max z) reaches min_p; a
+//     K-th largest tile max to 20 bits of its key (the lowest value with those bits; the K largest
+//     tile maxima are K logits, so theta is at most the K-th largest logit, whose z every kept
+//     token reaches), and for min-p the least x whose p~ = exp(fl(x / T) - max z) reaches min_p; a
 //     kept token then lies in a tile whose max is >= xlo. The elements >= xlo of those tiles (at
 //     most kTileRowTiles tiles, at most kSortCap elements) are sorted as the generic path sorts its short lists, the exact top-k
 //     and min-p thresholds taken from them, and sorted_tail finishes the row: the same
@@ -3554,9 +3554,8 @@ __device__ __forceinline__ bool tile_row(const SampleArgs& a, const Row<Tin>& ro
   // those of the K-th largest's bin by the next 8 (of a bf16 value's 16-bit key all the rest): the
   // lowest value of that bin is at most the K-th largest tile max, so at most the K-th largest
   // logit. (The 12 bits alone leave a bin as wide as [8, 9) or [10, 11): at K = 20 of 151936 N(0, 3)
-  // logits half of the rows had more tiles at its floor than could be read and were handed on: 36.5 us
-  // a per-token call against 22.7 now, whichever the row; 36.5 against 25.5 at K = 100.) The row max rides the first barrier (one LDS
-  // atomicMax per wave).
+  // logits half of the rows had more tiles at its floor than could be read and were handed on, as at K =
+  // 100.) The row max rides the first barrier (one LDS atomicMax per wave).
   uint32_t* h12 = reinterpret_cast<uint32_t*>(&g) + kBitmapOffset;
   uint32_t* h8 = h12 + 4096;  // 256 bins
   uint32_t* smax = &g.rdx.ncand;
@@ -3816,8 +3815,9 @@ __global__ __launch_bounds__(kThreads) void k_sample(SampleArgs a_, PICK pick) {
 // lowered_topk_row alone, two workgroups a CU (60 KB of LDS, at most 64 VGPRs), so that one row's
 // decisions run while the other's row streams; k_sample holds one (160 KB). A row it decides is
 // marked in the workspace's n_exc, and k_sample with UndecidedRow takes the others in a launch after
-// it. Measured (1024 rows of 151936, top-k 50, histories up to 32768): 161.0 us in the one launch,
-// 136.6 in the two (131-135 and 4); 512 rows none of which it decides (top-k 1000): 261.0 and 262.2.
+// it. Measured (histories up to 2000, top-k 50): 512 rows of 151936 73.3 us in one launch of k_sample, 65.5
+// in the two; 1024 of 50257 77.5 and 57.9; 512 rows none of which it decides (top-k 1000, histories of
+// 4096) 224.5 and 228.5.
 constexpr uint32_t kRowDecided = 0xFFFFFFFFu;
 template <class Tin>
 __global__ __launch_bounds__(kThreads, 8) void k_lowered(SampleArgs a_) {
