@@ -52,11 +52,11 @@ extern "C" {
  * Needs penalties on (a history and a penalty column). */
 #define VSAMP_HIST_APPEND 4u
 /* Row states in the workspace (vsamp_probs only; ABI version 12): the call may keep its rows' states
- * there between two launches, so that it writes the rows over the whole chip, when V > 8192 (shorter rows
- * take one launch) and the workspace holds vsamp_probs_workspace_bytes(). The workspace is then in use until the call's work is done, with or
- * without histories: calls that overlap each need their own. Without it a call that applies no
- * penalties leaves the workspace alone, and one workgroup writes each row. The results are identical
- * either way. No reference counterpart. */
+ * there between two launches, so that it writes the rows over the whole chip, when V > 8192 (shorter
+ * rows take one launch) and the workspace holds vsamp_probs_workspace_bytes(). The workspace is then
+ * in use until the call's work is done, with or without histories: calls that overlap each need their
+ * own. Without it a call that applies no penalties leaves the workspace alone, and one workgroup
+ * writes each row. The results are identical either way. No reference counterpart. */
 #define VSAMP_PROBS_STATES 8u
 
 enum vsamp_dtype { VSAMP_BF16 = 0, VSAMP_F32 = 1 };
